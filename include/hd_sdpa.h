@@ -72,11 +72,12 @@ int hd_flash_attention(const void *q, const void *k, const void *vt,
 
 /* Causal prefix length of a plan (0 for a non-split plan or NULL). */
 /* Extension: hd_flash_attention with a workspace for the tail split. When the
- * (batch x heads x 128-query tiles) units leave a last, partly filled round
- * of resident blocks, those units run as 2-8 key-range chunks writing fp32
- * partials (running max, sum, unnormalised O) into ws, and a merge kernel
- * combines them; full attention only (no mask, ar_len == 0), otherwise and
- * when ws_bytes < hd_flash_ws_bytes() it behaves as hd_flash_attention.
+ * (batch x heads x query tiles) units that see every key leave a last, partly
+ * filled round of resident blocks, those units run as 2-16 key-range chunks
+ * writing fp32 partials (running max, sum, unnormalised O) into ws, and a
+ * merge kernel combines them (not for a mask together with ar_len > 0). With
+ * a dense mask, ws also holds one bit per mask tile: tiles of zeros are not
+ * read again for every head. A smaller ws leaves these out.
  * Results agree with the unsplit kernel to fp32 rounding of the merge. */
 int hd_flash_attention_ws(const void *q, const void *k, const void *vt, const void *mask,
                           void *out, int batch, int q_heads, int kv_heads, int seq, int head_dim,

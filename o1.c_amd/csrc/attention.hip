@@ -36,6 +36,9 @@
 #define FA_BQ 128      // queries per block (4 waves x 32)
 #define FA_BK 64       // keys per tile
 #define FA_TAU 8.0f    // lazy-rescale threshold (log2 units)
+#define FA_MAX_SPLIT 16 // most key chunks of a tail unit
+#define FA_PP_MIN 1024 // shortest sequence that the 8-wave blocks take
+#define FA_PP_MIN_DENSE 256   // with a dense mask
 #ifndef FA_PF
 #define FA_PF 8        // LDS fragment reads in flight ahead of the MFMAs (ping-pong kernel)
 #endif
@@ -45,13 +48,58 @@ __host__ __device__ __forceinline__ int perm16(int s) {
 }
 static inline int64_t fa_spad(int64_t s) { return (s + FA_BK - 1) / FA_BK * FA_BK; }
 
+// One bit per 32-row x 64-key tile of a dense mask: 0 where every value is
+// zero (adding it changes nothing). bits [ceil(S/32)][ceil(S/2048)], bit t % 32
+// of word t / 32 for key tile t. The mask is the same for every head, so one
+// pass over it here saves the 32 passes that the heads' blocks would make
+// over its zero part (a mask is usually causal text rows above zero rows).
+// One wave per (strip, 8 key tiles: one byte); a lane reads 8 consecutive keys
+// of 4 rows per tile, all 32 loads in flight.
+__global__ __launch_bounds__(64) void fa_mask_bits_kernel(const uint16_t *mask, uint8_t *bits, int S) {
+    const int lane = threadIdx.x;
+    uint32_t any[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int kv = (blockIdx.x * 8 + k) * 64 + (lane & 7) * 8;
+        any[k] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = blockIdx.y * 32 + i * 8 + (lane >> 3);
+            const uint16_t *p = mask + (size_t)row * S + kv;
+            if (row < S && kv + 8 <= S) {
+                u32x4_t v;
+                __builtin_memcpy(&v, p, 16);   // rows of an odd S start at any even address
+                any[k] |= v[0] | v[1] | v[2] | v[3];
+            } else if (row < S) {
+                for (int e = 0; kv + e < S; e++) any[k] |= (uint32_t)p[e];
+            }
+        }
+    }
+    uint32_t byte = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+        if (__builtin_amdgcn_ballot_w64((any[k] & 0x7fff7fffu) != 0)) byte |= 1u << k;
+    if (lane == 0) bits[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (uint8_t)byte;
+}
+
+// Row tiling of the ping-pong kernel's units: per (batch, kv head) the rows
+// [row0, row0 + 256 * ntile + left) are `ntile` whole 256-row tiles of every
+// query head of the group, then the `left` rows after them. The left-over
+// rows of up to `hp` = 256 / left heads share one unit (they read the same
+// keys), so 1024 + 1 rows cost 4 + 1/4 tiles per head and not 5. Units are
+// numbered whole tiles first.
+struct FaRows {
+    int row0, ntile, left, hp;
+};
+
 struct FaArgs {
     const uint16_t *q;     // [B,Hq,S,D]
     const uint16_t *k;     // [B,Hkv,S,D]
     const uint16_t *vt;    // [B,Hkv,D,S_pad] (perm16 columns)
     const uint16_t *mask;  // optional [S,S] additive bf16
+    const uint32_t *mask_bits;   // FA_DENSE, may be null: see fa_mask_bits_kernel
     uint16_t *out;         // seq-major [B,S,Hq*D] or head-major [B,Hq,S,D]
-    int S, S_pad, Hq, Hkv;
+    int batch, S, S_pad, Hq, Hkv;
     int ar_len;            // rows < ar_len: causal
     int q_row_begin;       // first query row of the launch (its q tiles start here)
     int q_row_end;         // only rows < q_row_end are computed/written
@@ -61,9 +109,13 @@ struct FaArgs {
     int out_rows;          // rows per sequence in `out` (S, or fewer for a staging buffer)
     // tail split: blocks [0, n_whole) each run one (b, head, q tile) unit over
     // all keys; the units from n_whole on run as `split` chunks of the key
-    // tiles each, writing unnormalised partials to `part` (merged afterwards)
-    int n_whole, split;
-    float *part;           // [n_tail * split][FA_BQ][FA_D] O, then [..][FA_BQ] (m, l)
+    // tiles each (n_chunks blocks), writing unnormalised partials to `part`
+    // (merged afterwards). flash_pp16_kernel<FA_CAUSAL>: the blocks after the
+    // chunks are the units of the causal rows [0, ar_len), the units before
+    // them cover rows [q_row_begin, q_row_end), which see every key
+    int n_whole, split, n_chunks;
+    FaRows full, causal;   // flash_pp16_kernel: row tiling of the two kinds of units
+    float *part;           // [n_chunks][FA_BQ][FA_D] O, then [..][FA_BQ] (m, l)
 };
 
 // 16-byte buffer load straight to LDS against a wave-uniform descriptor
@@ -307,7 +359,7 @@ __global__ __launch_bounds__(NWV * 64, 8 / NWV) void flash_fwd_kernel(FaArgs a) 
                                         o[dt][gq * 4 + 3]};
             }
         if (h == 0) {
-            float2 *pml = (float2 *)(a.part + (size_t)(gridDim.x - a.n_whole) * BQ * FA_D);
+            float2 *pml = (float2 *)(a.part + (size_t)a.n_chunks * BQ * FA_D);
             pml[(size_t)item * BQ + wave * 32 + l32] = make_float2(m_run, l_tot);
         }
         return;
@@ -394,7 +446,47 @@ __device__ __forceinline__ float xor16_32_sum(float v) {
     return xor32_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
-template <bool MASKED>
+// Unit `lin` of a row tiling: batch, kv head, first row and first query head
+// of the group; left: rows per head of a left-over unit, 0 for a whole tile.
+struct FaUnit {
+    int b, hk, qbase, g0, left;
+};
+__device__ __forceinline__ FaUnit fa_unit(const FaArgs &a, const FaRows &r, int batch, int lin) {
+    const int group = a.Hq / a.Hkv, n_whole_tiles = batch * a.Hkv * r.ntile * group;
+    FaUnit u;
+    int bh;
+    if (lin < n_whole_tiles) {   // heads of a group are neighbours: they share K / V^T in L2
+        u.g0 = lin % group;
+        lin /= group;
+        u.qbase = r.row0 + (lin % r.ntile) * 256;
+        bh = lin / r.ntile;
+        u.left = 0;
+    } else {
+        lin -= n_whole_tiles;
+        const int per = (group + r.hp - 1) / r.hp;
+        u.g0 = (lin % per) * r.hp;
+        u.qbase = r.row0 + r.ntile * 256;
+        bh = lin / per;
+        u.left = r.left;
+    }
+    u.hk = bh % a.Hkv;
+    u.b = bh / a.Hkv;
+    return u;
+}
+// Query row and head of row i (0..255) of a unit; row = INT_MAX where it has none.
+__device__ __forceinline__ int2 fa_unit_row(const FaArgs &a, const FaUnit &u, int i) {
+    const int group = a.Hq / a.Hkv;
+    if (u.left == 0) return make_int2(u.qbase + i, u.hk * group + u.g0);
+    const int k = i / u.left, hp = 256 / u.left;
+    if (k >= hp || u.g0 + k >= group) return make_int2(0x7fffffff, u.hk * group + u.g0);
+    return make_int2(u.qbase + i % u.left, u.hk * group + u.g0 + k);
+}
+
+// MODE FA_PLAIN: S % 64 == 0, every row sees every key. FA_CAUSAL: any S, and
+// the units past the chunks are causal rows. FA_DENSE: any S, an additive mask
+// (and the causal test per element when ar_len > 0 comes with it).
+enum { FA_PLAIN = 0, FA_CAUSAL = 1, FA_DENSE = 2 };
+template <int MODE>
 __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     constexpr int PF16 = FA_PF;   // 4 and 12 measured equal or slower
     constexpr int BQ = 256, LPW = 2, NB = 4;
@@ -404,31 +496,39 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     const int grp = wave >> 2;
     const int l16 = lane & 15, g = lane >> 4;
 
-    const int nqt = (a.q_row_end - a.q_row_begin + BQ - 1) / BQ;
-    const int group = a.Hq / a.Hkv;
     int lin = blockIdx.x, chunk = -1, item = 0;
-    if (lin >= a.n_whole) {
+    bool causal_unit = false;
+    if (MODE == FA_CAUSAL && lin >= a.n_whole + a.n_chunks) {
+        lin -= a.n_whole + a.n_chunks;
+        causal_unit = true;
+    } else if (lin >= a.n_whole) {
         item = lin - a.n_whole;
         chunk = item % a.split;
         lin = a.n_whole + item / a.split;
     } else {
         lin = fa_xcd_remap(lin, a.n_whole);
     }
-    const int gq = lin % group; lin /= group;
-    const int qt = lin % nqt; lin /= nqt;
-    const int hk = lin % a.Hkv;
-    const int b = lin / a.Hkv;
-    const int hq = hk * group + gq;
+    // (by value: a selected pointer into the arguments would be read with
+    // vector loads and make everything below per-lane)
+    FaRows rows = a.full;
+    if (MODE == FA_CAUSAL && causal_unit) rows = a.causal;
+    FaUnit un = fa_unit(a, rows, a.batch, lin);
+    un.b = __builtin_amdgcn_readfirstlane(un.b);
+    un.hk = __builtin_amdgcn_readfirstlane(un.hk);
+    un.qbase = __builtin_amdgcn_readfirstlane(un.qbase);
+    un.g0 = __builtin_amdgcn_readfirstlane(un.g0);
+    un.left = __builtin_amdgcn_readfirstlane(un.left);
+    const int b = un.b, hk = un.hk;
 
-    const int qbase = a.q_row_begin + qt * BQ;
-    const int q0 = qbase + wave * 32;
-    int my_q[2];
-    my_q[0] = q0 + l16;
-    my_q[1] = q0 + 16 + l16;
-    const bool causal_block = qbase < a.ar_len;
+    const int qbase = un.qbase;
+    const int q0 = qbase + (un.left ? 0 : wave * 32);   // lowest row of this wave
+    int2 rh[2];   // this lane's two query rows and their heads
+    rh[0] = fa_unit_row(a, un, wave * 32 + l16);
+    rh[1] = fa_unit_row(a, un, wave * 32 + 16 + l16);
+    const int my_q[2] = {rh[0].x, rh[1].x};
     int kv_end = a.S;
-    if (causal_block) {
-        int last_row = min(qbase + BQ, a.q_row_end) - 1;
+    if (MODE != FA_PLAIN && qbase < a.ar_len) {
+        const int last_row = qbase + (un.left ? un.left : BQ) - 1;
         if (last_row < a.ar_len) kv_end = last_row + 1;
     }
     int t_begin = 0, t_end = (kv_end + FA_BK - 1) / FA_BK;
@@ -442,7 +542,7 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     bf16x8_t qf[2][4];
 #pragma unroll
     for (int qq = 0; qq < 2; qq++) {
-        const uint16_t *qrow = a.q + (((size_t)b * a.Hq + hq) * a.S + min(my_q[qq], a.S - 1)) * FA_D;
+        const uint16_t *qrow = a.q + (((size_t)b * a.Hq + rh[qq].y) * a.S + min(my_q[qq], a.S - 1)) * FA_D;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) qf[qq][ks] = *(const bf16x8_t *)(qrow + ks * 32 + g * 8);
     }
@@ -557,25 +657,92 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 2 * PF16, 0);
     };
+    // dense mask of tile t in the order of the scores: lanes of row groups 2r
+    // and 2r + 1 need keys {0-3, 8-11} and {4-7, 12-15} of a 16-key run, so
+    // each loads 8 consecutive keys and one 16-lane row swap exchanges the
+    // inner halves. Requested at the start of tile t's MFMA phase, before the
+    // K / V^T loads of a later tile, so the values land under the MFMAs and
+    // the phase's vmcnt wait covers them. Rows start at any even address (S
+    // may be odd): unaligned 16-byte loads; the tile that holds key S - 1
+    // reads element by element, clamped to the row.
+    // Tiles that fa_mask_bits_kernel found to be all zero are not read: bit t
+    // of this wave's 32-row strip, 32 tiles per lane of `mbits`.
+    u32x4_t mk[2][2];
+    uint32_t mbits = ~0u;
+    if constexpr (MODE == FA_DENSE) {
+        const int strip = (qbase >> 5) + wave, nw = (a.S + FA_BK * 32 - 1) / (FA_BK * 32);
+        if (a.mask_bits) mbits = lane < nw && strip * 32 < a.S ? a.mask_bits[(size_t)strip * nw + lane] : 0u;
+    }
+    auto has_mask = [&](int t) {
+        return MODE == FA_DENSE && (__builtin_amdgcn_readlane(mbits, t >> 5) >> (t & 31) & 1);
+    };
+    auto load_mask = [&](int t) {
+        if (has_mask(t)) {
+            const int kv0 = t * FA_BK + (g >> 1) * 16 + (g & 1) * 8;
+#pragma unroll
+            for (int qq = 0; qq < 2; qq++) {
+                const uint16_t *row = a.mask + (size_t)min(my_q[qq], a.S - 1) * a.S;
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    const int k0 = kv0 + w * 32;
+                    if ((t + 1) * FA_BK <= a.S) {
+                        __builtin_memcpy(&mk[qq][w], row + k0, 16);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            mk[qq][w][e] = (uint32_t)row[min(k0 + 2 * e, a.S - 1)] |
+                                           ((uint32_t)row[min(k0 + 2 * e + 1, a.S - 1)] << 16);
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto swap_mask = [&]() {
+        if constexpr (MODE == FA_DENSE) {
+#pragma unroll
+            for (int qq = 0; qq < 2; qq++)
+#pragma unroll
+                for (int w = 0; w < 2; w++)
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const auto r = __builtin_amdgcn_permlane16_swap(mk[qq][w][e], mk[qq][w][e + 2], false, false);
+                        mk[qq][w][e] = r[0];
+                        mk[qq][w][e + 2] = r[1];
+                    }
+        }
+    };
     // softmax of S(t) into P(t), with the lazy O rescale
     auto softmax = [&](int t) {
         const int kv0 = t * FA_BK;
-        const bool need_mask = MASKED && (a.mask != nullptr || kv0 + FA_BK > a.S ||
-                                          (q0 < a.ar_len && kv0 + FA_BK - 1 > q0));
+        // the wave-uniform test is taken once per tile: tiles without dead
+        // keys run exactly the plain kernel's max loop
+        const bool dead_keys = MODE != FA_PLAIN &&
+                               (kv0 + FA_BK > a.S || (q0 < a.ar_len && kv0 + FA_BK - 1 > q0));
+        if (has_mask(t)) swap_mask();
 #pragma unroll
         for (int qq = 0; qq < 2; qq++) {
             float mt = -INFINITY;
-            if (need_mask) {
+            if (has_mask(t)) {
+                asm volatile("");
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t m2 = mk[qq][u >> 1][(u & 1) * 2 + (e >> 1)];
+                        s[qq][u][e] = fmaf(e & 1 ? hi_bf(m2) : lo_bf(m2), a.inv_scale, s[qq][u][e]);
+                    }
+            }
+            if (dead_keys) {
+                asm volatile("");   // a branch, not 32 selects in every tile
                 const int mq = my_q[qq];
 #pragma unroll
                 for (int u = 0; u < 4; u++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        float v = s[qq][u][e];
                         const int kv = kv0 + fa16_key(u, g * 4 + e);
                         const bool dead = kv >= a.S || (mq < a.ar_len && kv > mq);
-                        if (a.mask && !dead && mq < a.S) v += bf2f(a.mask[(size_t)mq * a.S + kv]) * a.inv_scale;
-                        if (dead) v = -INFINITY;
+                        const float v = dead ? -INFINITY : s[qq][u][e];
                         s[qq][u][e] = v;
                         mt = fmaxf(mt, v);
                     }
@@ -635,6 +802,7 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     if (grp) fa_barrier();
     {
         const bool ld = t_begin + 2 < t_end;
+        load_mask(t_begin);
         if (ld) issue(t_begin + 2);
         qk(t_begin);
         wait_next(ld);
@@ -645,6 +813,7 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         pin_softmax();
         fa_barrier();
         const bool ld = t + 2 < t_end;
+        load_mask(t);
         if (ld) issue(t + 2);
         pv_qk(t);
         wait_next(ld);
@@ -669,16 +838,16 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
                 *(f32x4_t *)(po + w * 32 + g * 8 + 4) = o[qq][w * 2 + 1];
             }
             if (g == 0) {
-                float2 *pml = (float2 *)(a.part + (size_t)(gridDim.x - a.n_whole) * BQ * FA_D);
+                float2 *pml = (float2 *)(a.part + (size_t)a.n_chunks * BQ * FA_D);
                 pml[(size_t)item * BQ + row] = make_float2(m_run[qq], l_tot);
             }
         } else if (my_q[qq] < a.q_row_end) {
             const float inv = 1.0f / l_tot;
             uint16_t *dst;
             if (a.out_seq_major)
-                dst = a.out + (((size_t)b * a.out_rows + my_q[qq]) * a.Hq + hq) * FA_D;
+                dst = a.out + (((size_t)b * a.out_rows + my_q[qq]) * a.Hq + rh[qq].y) * FA_D;
             else
-                dst = a.out + (((size_t)b * a.Hq + hq) * a.out_rows + my_q[qq]) * FA_D;
+                dst = a.out + (((size_t)b * a.Hq + rh[qq].y) * a.out_rows + my_q[qq]) * FA_D;
 #pragma unroll
             for (int w = 0; w < 4; w++) {
                 const f32x4_t x0 = o[qq][w * 2], x1 = o[qq][w * 2 + 1];
@@ -691,22 +860,48 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     if (!grp) fa_barrier();
 }
 
-// V [BH, S, D] -> vt [BH, D, S_pad] with perm16 columns and zero padding.
+// One block per 64-key tile: rows in through LDS (16-byte loads when V is
+// 16-byte aligned), 16-byte stores of 8 storage columns per dimension. HBM
+// bound in principle (4 B per element); at S = 2371, 8 heads it is one short
+// launch: 8.4 us with 2-byte accesses, 4.0 us in this form (S = 16640: 26.9 ->
+// 11.5 us).
+template <bool V16>
 __global__ __launch_bounds__(256) void fa_vt_kernel(const uint16_t *v, uint16_t *vt, int S,
                                                     int S_pad) {
-    __shared__ uint16_t tile[64][FA_D + 2];
+    constexpr int LD = FA_D + 8;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64][LD];
     const int bh = blockIdx.y, s0 = blockIdx.x * 64;
     const uint16_t *src = v + (size_t)bh * S * FA_D;
-    for (int i = threadIdx.x; i < 64 * FA_D; i += 256) {
-        int t = i / FA_D, d = i % FA_D;
-        tile[t][d] = (s0 + t < S) ? src[(size_t)(s0 + t) * FA_D + d] : (uint16_t)0;
+    if constexpr (V16) {
+        for (int i = threadIdx.x; i < 64 * FA_D / 8; i += 256) {
+            const int t = i / (FA_D / 8), c = (i % (FA_D / 8)) * 8;
+            u32x4_t x = {0, 0, 0, 0};
+            if (s0 + t < S) x = *(const u32x4_t *)(src + (size_t)(s0 + t) * FA_D + c);
+            *(u32x4_t *)&tile[t][c] = x;
+        }
+    } else {
+        for (int i = threadIdx.x; i < 64 * FA_D; i += 256) {
+            int t = i / FA_D, d = i % FA_D;
+            tile[t][d] = (s0 + t < S) ? src[(size_t)(s0 + t) * FA_D + d] : (uint16_t)0;
+        }
     }
     __syncthreads();
-    uint16_t *dst = vt + (size_t)bh * FA_D * S_pad;
-    for (int i = threadIdx.x; i < 64 * FA_D; i += 256) {
-        int d = i / 64, p = i % 64;   // p: storage column within the tile
-        dst[(size_t)d * S_pad + s0 + p] = tile[perm16(p)][d];
+    uint16_t *dst = vt + (size_t)bh * FA_D * S_pad + s0;
+    for (int i = threadIdx.x; i < FA_D * 8; i += 256) {
+        const int d = i / 8, p0 = (i % 8) * 8;   // 8 storage columns p0 .. p0+7 of the tile
+        u32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            o[e] = (uint32_t)tile[perm16(p0 + 2 * e)][d] | ((uint32_t)tile[perm16(p0 + 2 * e + 1)][d] << 16);
+        *(u32x4_t *)(dst + (size_t)d * S_pad + p0) = o;
     }
+}
+static void fa_vt_launch(const void *v, void *vt, int bh, int S, hipStream_t st) {
+    const dim3 g(hd_cdiv(fa_spad(S), 64), bh);
+    if ((uintptr_t)v % 16 == 0)
+        fa_vt_kernel<true><<<g, 256, 0, st>>>((const uint16_t *)v, (uint16_t *)vt, S, (int)fa_spad(S));
+    else
+        fa_vt_kernel<false><<<g, 256, 0, st>>>((const uint16_t *)v, (uint16_t *)vt, S, (int)fa_spad(S));
 }
 
 // Merges the tail units' key-chunk partials: O = sum_i w_i O_i / sum_i w_i l_i
@@ -732,12 +927,22 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaArgs a, int n_tail) {
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[e] = fmaf(w, pv[e], acc[e]);
     }
-    const int nqt = (a.q_row_end - a.q_row_begin + BQ - 1) / BQ, group = a.Hq / a.Hkv;
-    int lin = a.n_whole + tu;
-    const int g = lin % group; lin /= group;
-    const int qt = lin % nqt; lin /= nqt;
-    const int hk = lin % a.Hkv, b = lin / a.Hkv, hq = hk * group + g;
-    const int my_q = a.q_row_begin + qt * BQ + row;
+    int b, hq, my_q;
+    if constexpr (BQ == 256) {
+        const FaUnit un = fa_unit(a, a.full, a.batch, a.n_whole + tu);
+        const int2 rh = fa_unit_row(a, un, row);
+        b = un.b;
+        hq = rh.y;
+        my_q = rh.x;
+    } else {
+        const int nqt = (a.q_row_end - a.q_row_begin + BQ - 1) / BQ, group = a.Hq / a.Hkv;
+        int lin = a.n_whole + tu;
+        const int g = lin % group; lin /= group;
+        const int qt = lin % nqt; lin /= nqt;
+        b = lin / a.Hkv;
+        hq = (lin % a.Hkv) * group + g;
+        my_q = a.q_row_begin + qt * BQ + row;
+    }
     if (my_q >= a.q_row_end) return;
     const size_t o = a.out_seq_major ? (((size_t)b * a.out_rows + my_q) * a.Hq + hq) * FA_D + d0
                                      : (((size_t)b * a.Hq + hq) * a.out_rows + my_q) * FA_D + d0;
@@ -757,7 +962,7 @@ static int fa_slots(int nwv = 4) {
         int per4 = 0, per8 = 0, cus = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per4, flash_fwd_kernel<false, 4>, 256, 0) !=
                 hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per8, flash_pp16_kernel<false>, 512, 0) !=
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per8, flash_pp16_kernel<FA_PLAIN>, 512, 0) !=
                 hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             return 0;
@@ -787,23 +992,27 @@ extern "C" void hd_flash_make_vt(const void *v, void *vt, int bh, int seq) {
         snprintf(hd_cuda_errbuf(), 512, "flash_make_vt: bad args");
         return;
     }
-    dim3 g(hd_cdiv(fa_spad(seq), 64), bh);
-    fa_vt_kernel<<<g, 256, 0, hd_stream()>>>((const uint16_t *)v, (uint16_t *)vt, seq,
-                                             (int)fa_spad(seq));
+    fa_vt_launch(v, vt, bh, seq, hd_stream());
     hd_check_launch("flash_make_vt");
+}
+
+// Bytes of the zero-tile bits of a dense mask (0: too long for one lane per word).
+static int64_t fa_mask_bits_bytes(int seq) {
+    const int64_t words = (seq + FA_BK * 32 - 1) / (FA_BK * 32);
+    return words <= 64 ? (seq + 31) / 32 * words * 4 : 0;
 }
 
 static int fa_launch(const void *q, const void *k, const void *vt, const void *mask, void *out,
                      int batch, int hq, int hkv, int seq, int ar_len, int q_row_end, float scale,
                      int out_seq_major, hipStream_t st, void *ws = nullptr, int64_t ws_bytes = 0,
                      int out_rows = 0, int q_row_begin = 0) {
-    // A causal text prefix (rows < ar_len see keys <= row) over full
-    // attention below it: the prefix rows run as a masked launch of their
-    // own, whose blocks all end at their diagonal, and rows ar_len.. are plain
-    // full attention in the unmasked kernel with the tail split. One masked
-    // launch over all rows costs 7-12 % more: its block holding row ar_len
-    // runs every key with most of its waves masked, and it has no split.
-    if (ar_len > 0 && !mask && ws && q_row_begin == 0 && (seq % FA_BK) == 0 && ar_len < q_row_end) {
+    const bool prefix = ar_len > 0 && !mask && q_row_begin == 0 && ar_len < q_row_end;
+    // Short sequences (4-wave blocks) with a causal text prefix (rows < ar_len
+    // see keys <= row): the prefix rows run as a masked launch of their own,
+    // whose blocks all end at their diagonal, and rows ar_len.. are plain full
+    // attention. One masked launch over all rows costs 7-12 % more: its block
+    // holding row ar_len runs every key with most of its waves masked.
+    if (prefix && ws && seq < FA_PP_MIN && (seq % FA_BK) == 0) {
         const int rc = fa_launch(q, k, vt, nullptr, out, batch, hq, hkv, seq, ar_len, ar_len, scale,
                                  out_seq_major, st, nullptr, 0, out_rows, 0);
         if (rc) return rc;
@@ -816,6 +1025,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     a.vt = (const uint16_t *)vt;
     a.mask = (const uint16_t *)mask;
     a.out = (uint16_t *)out;
+    a.batch = batch;
     a.S = seq;
     a.S_pad = (int)fa_spad(seq);
     a.Hq = hq;
@@ -828,47 +1038,91 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     a.out_seq_major = out_seq_major;
     a.out_rows = out_rows > 0 ? out_rows : seq;
     // 8-wave blocks (one copy of each K / V^T tile for 256 queries) when the
-    // tail split can fill the last round and the sequence is long enough to
-    // amortise the larger block: +3 % at S = 16640 / 16896, equal at 4352;
-    // 4-wave blocks otherwise (without the split their finer grain wins)
-    const bool split_ok = ws && !mask && ar_len == 0;
-    const int nwv = split_ok && seq >= 1024 ? 8 : 4;
+    // sequence is long enough to amortise the larger block and
+    //  * the tail split can fill the last round (+3 % at S = 16640 / 16896,
+    //    equal at 4352; without the split the finer grain of 4 waves wins), or
+    //  * there is a causal prefix: its rows are units of their own behind the
+    //    full ones in the same grid, so that no block mixes both kinds
+    //    (S = 4239, 142 causal rows, one masked 4-wave launch: 314 -> 270 us;
+    //    S = 16499: 4080 -> 3630; 2 x 1101 rows: equal), or
+    //  * there is a dense mask: its values are prefetched as 8-byte pieces
+    //    under the MFMA phase and skipped where they are zero (4-wave blocks
+    //    with 2-byte loads: S = 300 26.8 -> 21.8 us, 1209 201 -> 53; equal
+    //    at 200, where one 256-row block per head is as long as two of 128).
+    const bool pp = mask ? seq >= FA_PP_MIN_DENSE : seq >= FA_PP_MIN && (prefix || (ws && ar_len == 0));
+    const int nwv = pp ? 8 : 4;
     const int BQ = nwv * 32;
-    const int nqt = (q_row_end - q_row_begin + BQ - 1) / BQ;
-    const int units = batch * hq * nqt;
-    bool masked = mask || ar_len > 0 || (seq % FA_BK) != 0;
-    // Tail split (full attention only): the units of the last partial round
-    // of resident blocks run as P key chunks each, launched last, so that
-    // round is filled instead of running a few blocks for a whole round.
+    const int group = hq / hkv;
+    int units, n_causal = 0;
+    a.full = a.causal = {};
+    if (pp) {
+        if (prefix) a.q_row_begin = ar_len;   // the causal rows are units of their own
+        auto rows_of = [&](int row0, int rows, bool share) {
+            FaRows r = {row0, rows / BQ, rows % BQ, 1};
+            if (r.left && share) r.hp = BQ / r.left < group ? BQ / r.left : group;
+            return r;
+        };
+        auto count = [&](const FaRows &r) {
+            return batch * hkv * (r.ntile * group + (r.left ? (group + r.hp - 1) / r.hp : 0));
+        };
+        a.full = rows_of(a.q_row_begin, q_row_end - a.q_row_begin, !mask);
+        units = count(a.full);
+        if (prefix) {
+            a.causal = rows_of(0, ar_len, false);
+            n_causal = count(a.causal);
+        }
+    } else {
+        units = batch * hq * ((q_row_end - a.q_row_begin + BQ - 1) / BQ);
+    }
+    // Tail split (units that see every key only): the units of the last
+    // partial round of resident blocks run as P key chunks each, launched
+    // last, so that round is filled (together with the causal units) instead
+    // of running a few blocks for a whole round.
     a.n_whole = units;
     a.split = 1;
     a.part = (float *)ws;
     int n_tail = 0;
+    // dense mask: the zero-tile bits lie behind the partials in the workspace
+    const int64_t bits_bytes = pp && mask && q_row_begin == 0 ? fa_mask_bits_bytes(seq) : 0;
+    const bool bits = bits_bytes > 0 && ws && bits_bytes <= ws_bytes;
+    if (bits) ws_bytes -= bits_bytes;
     const int slots = ws ? fa_slots(nwv) : 0;
-    if (slots > 0 && !mask && ar_len == 0 && units >= slots) {
+    if (slots > 0 && (ar_len == 0 || prefix) && units >= slots) {
         const int rem = units % slots, ntile = (seq + FA_BK - 1) / FA_BK;
-        int P = rem ? slots / rem : 1;
-        if (P > 8) P = 8;
+        int P = rem ? (slots - n_causal) / rem : 1;
+        if (P < 2 && rem) P = slots / rem;
+        if (P > FA_MAX_SPLIT) P = FA_MAX_SPLIT;
         if (P > ntile) P = ntile;
-        if (rem && P >= 2 && (int64_t)rem * P * BQ * (FA_D + 2) * 4 <= ws_bytes) {
+        const int64_t chunk_bytes = (int64_t)BQ * (FA_D + 2) * 4;
+        if (bits && rem * P * chunk_bytes > ws_bytes) P = (int)(ws_bytes / (rem * chunk_bytes));
+        if (rem && P >= 2 && rem * P * chunk_bytes <= ws_bytes) {
             n_tail = rem;
             a.n_whole = units - rem;
             a.split = P;
         }
     }
-    dim3 grid((unsigned)(a.n_whole + n_tail * a.split));
-    if (nwv == 8) {
+    a.n_chunks = n_tail * a.split;
+    a.mask_bits = nullptr;
+    if (bits) {
+        uint8_t *at = (uint8_t *)ws + (int64_t)a.n_chunks * BQ * (FA_D + 2) * 4;
+        fa_mask_bits_kernel<<<dim3((seq + FA_BK * 32 - 1) / (FA_BK * 32) * 4, (seq + 31) / 32), 64, 0, st>>>(
+            (const uint16_t *)mask, at, seq);
+        a.mask_bits = (const uint32_t *)at;
+    }
+    dim3 grid((unsigned)(a.n_whole + a.n_chunks + n_causal));
+    if (pp) {
         // the ping-pong form: +2.5-4.7 % at S = 4352-16640 over 8-wave
         // blocks in lockstep
-        if (masked) flash_pp16_kernel<true><<<grid, 512, 0, st>>>(a);
-        else flash_pp16_kernel<false><<<grid, 512, 0, st>>>(a);
+        if (mask) flash_pp16_kernel<FA_DENSE><<<grid, 512, 0, st>>>(a);
+        else if (ar_len > 0 || seq % FA_BK) flash_pp16_kernel<FA_CAUSAL><<<grid, 512, 0, st>>>(a);
+        else flash_pp16_kernel<FA_PLAIN><<<grid, 512, 0, st>>>(a);
     } else {
-        if (masked) flash_fwd_kernel<true, 4><<<grid, 256, 0, st>>>(a);
+        if (mask || ar_len > 0 || seq % FA_BK) flash_fwd_kernel<true, 4><<<grid, 256, 0, st>>>(a);
         else flash_fwd_kernel<false, 4><<<grid, 256, 0, st>>>(a);
     }
     if (n_tail) {
         dim3 gm((unsigned)hd_cdiv((int64_t)n_tail * BQ * (FA_D / 8), 256));
-        if (nwv == 8) fa_merge_kernel<256><<<gm, 256, 0, st>>>(a, n_tail);
+        if (pp) fa_merge_kernel<256><<<gm, 256, 0, st>>>(a, n_tail);
         else fa_merge_kernel<128><<<gm, 256, 0, st>>>(a, n_tail);
     }
     hipError_t e = hipGetLastError();
@@ -943,7 +1197,7 @@ static int plan_new(hd_sdpa_plan **out, int batch, int hq, int hkv, int sq, int 
         delete p;
         return sdpa_err("hipMalloc V^T staging failed");
     }
-    p->ws_bytes = hd_flash_ws_bytes();
+    p->ws_bytes = hd_flash_ws_bytes() + fa_mask_bits_bytes(sq);
     if (hipMalloc(&p->ws, (size_t)p->ws_bytes) != hipSuccess) {
         (void)hipFree(p->vt);
         delete p;
@@ -992,9 +1246,7 @@ extern "C" void hd_sdpa_destroy(hd_sdpa_plan *p) {
 static int plan_run(hd_sdpa_plan *p, const void *q, const void *k, const void *v, const void *mask,
                     void *out, void *stream, int ar_len, int q_row_end, bool to_stage = false) {
     hipStream_t st = stream ? (hipStream_t)stream : hd_stream();
-    dim3 g(hd_cdiv(fa_spad(p->Skv), 64), p->B * p->Hkv);
-    fa_vt_kernel<<<g, 256, 0, st>>>((const uint16_t *)v, (uint16_t *)p->vt, p->Skv,
-                                    (int)fa_spad(p->Skv));
+    fa_vt_launch(v, p->vt, p->B * p->Hkv, p->Skv, st);
     if (hipGetLastError() != hipSuccess) return sdpa_err("V^T staging launch failed");
     if (to_stage)   // pass 0: the causal rows into the plan's staging, seq-major
         return fa_launch(q, k, p->vt, mask, p->o_stage, p->B, p->Hq, p->Hkv, p->Sq, ar_len, q_row_end,
