@@ -22,6 +22,7 @@
 #include "../../include/hd_gemm.h"
 #include "../../include/hd_sdpa.h"
 #include "../../include/hd_block.h"
+#include "hd_common.hpp"
 
 static hd_block_config g_cfg = {1e-6f, 5000000.0f, 1.0f, {24, 20, 20}, 1};  // block.c:233-236
 
@@ -151,9 +152,9 @@ static hd_status block_core(const void *in, const float *cs, const void *mask, i
     }
     // QKV GEMM with q/k norm + rotary + V^T layout in its epilogue; shapes
     // outside that path take the GEMM then the standalone epilogue kernels
-    if (D != 128 || hd_linear_qkv_rope_ws(s.ln, bw->q_proj, bw->k_proj, bw->v_proj, bw->q_norm,
-                                          bw->k_norm, cs, s.q, s.k, s.vt, batch, (int)seq, H, KV,
-                                          HID, eps, s.fa_ws, s.fa_ws_bytes) != 0) {
+    if (D != 128 || hd_qkv_rope_gemm(s.ln, bw->q_proj, bw->k_proj, bw->v_proj, bw->q_norm, bw->k_norm,
+                                     cs, s.q, s.k, s.vt, batch, (int)seq, H, KV, HID, eps, s.fa_ws,
+                                     s.fa_ws_bytes) != 0) {
         hd_linear_concat3(s.ln, bw->q_proj, H * D, bw->k_proj, KV * D, bw->v_proj, KV * D, s.qkv,
                           M, HID);
         hd_qkv_epilogue(s.qkv, bw->q_norm, bw->k_norm, cs, s.q, s.k, nullptr, s.vt, batch,

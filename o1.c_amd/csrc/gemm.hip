@@ -149,8 +149,8 @@ template <int CPR> __device__ __forceinline__ int ms_swz(int r) {
 // x_{l+64}^2 then pairs 4, 2, 1 and 32, 16, 8 apart, so results are
 // bit-identical) and rotate-half rotary with bf16 rounding of every
 // product, stored straight to [B,H,S,128].
-// v heads: transposed stores into [B,KV,128,S] with key bits 2 and 3
-// exchanged (the flash kernel's V^T layout; S % 64 == 0 so no padding).
+// v heads: transposed stores into [B,KV,128,S_pad] with key bits 2 and 3
+// exchanged and zero columns past S (the flash kernel's V^T layout).
 template <int WTM, int LDW>
 __device__ __forceinline__ void qkv_epilogue(const GemmArgs &g, uint16_t *stg, int gm0, int hslot,
                                              int lane) {
@@ -234,12 +234,38 @@ __device__ __forceinline__ void qkv_epilogue(const GemmArgs &g, uint16_t *stg, i
             }
         }
     } else {
-        const int hk = hslot - H - KV;
+        const int hk = hslot - H - KV, SP = (S + 63) & ~63;
+        const bool one = g.M == S;   // one sequence: row m is key m
+        if (!one && S % 64) {
+            // zero columns behind each sequence that ends in these rows
+            for (int b = gm0 / S; (b + 1) * S <= gm0 + WTM && (b + 1) * S <= g.M; b++)
+                for (int i = lane; i < (SP - S) * 128; i += 64) {
+                    const int s = S + i % (SP - S), c = (s & ~12) | ((s & 4) << 1) | ((s & 8) >> 1);
+                    g.vt_out[(((size_t)b * KV + hk) * 128 + i / (SP - S)) * SP + c] = 0;
+                }
+        }
+        if (!one && S % 16) {
+            // sequences that start off the 16-key groups: a lane stores its
+            // key's 8 dimensions element by element (64 lanes fill 128 bytes
+            // of a column run)
+            for (int i = lane; i < WTM * 16; i += 64) {
+                const int r = i % WTM, d0 = (i / WTM) * 8, m = gm0 + r;
+                const u32x4_t x = *(const u32x4_t *)(stg + r * LDW + d0);
+                if (m >= g.M) continue;
+                const int b = m / S, s = m % S, c = (s & ~12) | ((s & 4) << 1) | ((s & 8) >> 1);
+                uint16_t *dst = g.vt_out + (((size_t)b * KV + hk) * 128 + d0) * SP + c;
+#pragma unroll
+                for (int e = 0; e < 8; e++) dst[(size_t)e * SP] = (uint16_t)(x[e >> 1] >> (16 * (e & 1)));
+            }
+            return;
+        }
         // 8 keys x 8 dimensions per lane and item: 8 16-byte row reads (the
         // item's keys, dimensions 8*lane%16 .. +7), a register transpose, 8
         // 16-byte stores (one per dimension: the 8 storage columns of one
         // half of a 16-key group). Items: (16-key group, half), 4 per pass.
-        const int dblk = lane & 15;
+        // Rows past M hold zeros (their A rows read as zero), so the groups
+        // up to S_pad of a single sequence write its padding too.
+        const int dblk = lane & 15, m_end = one ? SP : g.M;
         constexpr int NITEM = WTM / 8;
         for (int it = lane >> 4; it < NITEM; it += 4) {
             const int grp = it >> 1, half = it & 1;
@@ -251,9 +277,9 @@ __device__ __forceinline__ void qkv_epilogue(const GemmArgs &g, uint16_t *stg, i
                 const int src = (p & ~12) | ((p & 4) << 1) | ((p & 8) >> 1);  // key at that column
                 rw[e] = *(const u32x4_t *)(stg + (grp * 16 + src) * LDW + dblk * 8);
             }
-            if (m >= g.M) continue;
-            const int b = m / S, s = m % S;
-            uint16_t *dst = g.vt_out + (((size_t)b * KV + hk) * 128 + dblk * 8) * S + s + half * 8;
+            if (m >= m_end) continue;
+            const int b = one ? 0 : m / S, s = one ? m : m % S;
+            uint16_t *dst = g.vt_out + (((size_t)b * KV + hk) * 128 + dblk * 8) * SP + s + half * 8;
 #pragma unroll
             for (int dd = 0; dd < 8; dd++) {
                 const uint32_t sel = dd & 1 ? 0x07060302u : 0x05040100u;
@@ -261,7 +287,7 @@ __device__ __forceinline__ void qkv_epilogue(const GemmArgs &g, uint16_t *stg, i
 #pragma unroll
                 for (int w = 0; w < 4; w++)
                     pk[w] = __builtin_amdgcn_perm(rw[2 * w + 1][dd >> 1], rw[2 * w][dd >> 1], sel);
-                *(u32x4_t *)(dst + (size_t)dd * S) = pk;
+                *(u32x4_t *)(dst + (size_t)dd * SP) = pk;
             }
         }
     }
@@ -880,11 +906,6 @@ static void launch_ms(GemmArgs &g, void *ws = nullptr, int64_t ws_bytes = 0) {
 // path; a 192-row tile is taken when it quantises the grid onto the 256 CUs
 // better (M = 8704 without a workspace: 34 -> 46 row tiles), and 128x128
 // tiles for grids too small to fill the chip with 256x256 tiles.
-static double quant_eff(long tiles) {
-    long rounds = (tiles + 255) / 256;
-    return (double)tiles / (double)(rounds * 256);
-}
-
 // Estimated time (s) of a tile family: rounds of resident blocks, each the
 // time of `occ` tiles on a CU (2*BM*BNA*K flops at ~half the per-CU peak x
 // the family's relative per-flop efficiency: 192-row tiles 8-18 % slower
@@ -981,18 +1002,18 @@ static void gemm_launch(int epi, GemmArgs &g, void *ws = nullptr, int64_t ws_byt
 }
 
 // QKV projection with the q/k RMSNorm + rotary and the V^T layout fused into
-// the GEMM epilogue (EPI_QKV). Returns 1 without launching when the shape is
-// outside the fused path (the caller then runs hd_linear_concat3 +
-// hd_qkv_epilogue, which compute the same values).
-extern "C" int hd_linear_qkv_rope_ws(const void *x, const void *wq, const void *wk, const void *wv,
-                                     const void *qn_w, const void *kn_w, const float *cs, void *q,
-                                     void *k, void *vt, int batch, int seq, int heads, int kv_heads,
-                                     int hidden, float eps, void *ws, int64_t ws_bytes) {
+// the GEMM epilogue (EPI_QKV), any sequence length: vt is
+// [B, KV, 128, round_up(S, 64)] with zero padding. Returns 1 without launching
+// when the shape is outside the fused path (the caller then runs
+// hd_linear_concat3 + hd_qkv_epilogue, which compute the same values).
+int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *wv, const void *qn_w,
+                     const void *kn_w, const float *cs, void *q, void *k, void *vt, int batch, int seq,
+                     int heads, int kv_heads, int hidden, float eps, void *ws, int64_t ws_bytes) {
     if (!x || !wq || !wk || !wv || !qn_w || !kn_w || !cs || !q || !k || !vt || batch <= 0 ||
         seq <= 0 || heads <= 0 || kv_heads <= 0 || hidden <= 0)
         return 1;
     const int M = batch * seq, N = (heads + 2 * kv_heads) * 128;
-    const bool ok = seq % 64 == 0 && (heads * 128) % 256 == 0 &&
+    const bool ok = (heads * 128) % 256 == 0 &&
                     (kv_heads * 128) % 256 == 0 && hidden % 64 == 0 && hidden <= 8192 &&
                     (size_t)(M + 256) * hidden * 2 < ((size_t)1 << 31) &&
                     (size_t)heads * 128 * hidden * 2 < ((size_t)1 << 31) &&
@@ -1015,17 +1036,36 @@ extern "C" int hd_linear_qkv_rope_ws(const void *x, const void *wq, const void *
     g.k_out = (uint16_t *)k;
     g.vt_out = (uint16_t *)vt;
     g.seq = seq; g.heads = heads; g.kv_heads = kv_heads; g.eps = eps;
+    // the cheapest tile family, as in pick_and_launch (8 waves: two 64-wide
+    // wave tiles per head, 16x16x32 MFMA tiles)
     const long tn = N / 256;
     const long t256 = (long)((M + 255) / 256) * tn, t192 = (long)((M + 191) / 192) * tn;
+    const long t128 = (long)((M + 127) / 128) * tn * 2;
     if (ws && (uintptr_t)ws % 16) ws = nullptr;
-    const bool split256 =
-        ws && tail_split_of(t256, hidden / 64, (size_t)256 * 256 * 4, ws_bytes, (size_t)256 * 256 * 2) > 1;
-    const bool use192 = !split256 && quant_eff(t192) > quant_eff(t256) * 1.12;
-    // 8 waves: two 64-wide wave tiles per head, 16x16x32 MFMA tiles
-    if (use192) launch_ms<192, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws ? ws_bytes : 0);
-    else launch_ms<256, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws ? ws_bytes : 0);
+    if (!ws) ws_bytes = 0;
+    const int nk = hidden / 64;
+    auto split = [&](long t, int bm, int bn, int occ) {
+        return tail_split_of(t, nk, (size_t)bm * bn * 4, ws_bytes, (size_t)bm * bn * 2, occ);
+    };
+    const double c256 = tile_cost(t256, 1, 256, 256, hidden, 1.0, split(t256, 256, 256, 1));
+    const double c192 = tile_cost(t192, 1, 192, 256, hidden, 0.9, split(t192, 192, 256, 1));
+    const double c128 = tile_cost(t128, 2, 128, 128, hidden, 0.8, split(t128, 128, 128, 2));
+    if (c128 < c256 && c128 < c192) launch_ms<128, 128, 64, 2, 2, 2, EPI_QKV, 8, 2, 5, 16>(g, ws, ws_bytes);
+    else if (c192 < c256) launch_ms<192, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws_bytes);
+    else launch_ms<256, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws_bytes);
     hd_check_launch("linear_qkv_rope");
     return 0;
+}
+
+// Public form: whole 64-key groups only, so that a caller's vt of seq columns
+// is never written past them.
+extern "C" int hd_linear_qkv_rope_ws(const void *x, const void *wq, const void *wk, const void *wv,
+                                     const void *qn_w, const void *kn_w, const float *cs, void *q,
+                                     void *k, void *vt, int batch, int seq, int heads, int kv_heads,
+                                     int hidden, float eps, void *ws, int64_t ws_bytes) {
+    if (seq % 64) return 1;
+    return hd_qkv_rope_gemm(x, wq, wk, wv, qn_w, kn_w, cs, q, k, vt, batch, seq, heads, kv_heads, hidden,
+                            eps, ws, ws_bytes);
 }
 
 extern "C" int hd_linear_qkv_rope(const void *x, const void *wq, const void *wk, const void *wv,

@@ -11,6 +11,11 @@ hipStream_t hd_stream(void);
 // Records a launch failure (if any) of the previous kernel under `what`.
 void hd_check_launch(const char *what);
 
+// hd_linear_qkv_rope_ws for any sequence length (gemm.hip).
+int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *wv, const void *qn_w,
+                     const void *kn_w, const float *cs, void *q, void *k, void *vt, int batch, int seq,
+                     int heads, int kv_heads, int hidden, float eps, void *ws, int64_t ws_bytes);
+
 // ---- bf16 <-> fp32 ------------------------------------------------------
 // bf16 payloads are uint16_t. fp32 -> bf16 uses gfx950's v_cvt_pk_bf16_f32,
 // IEEE round-to-nearest-even: for finite values the same bits as the
