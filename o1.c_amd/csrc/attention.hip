@@ -48,38 +48,51 @@ __host__ __device__ __forceinline__ int perm16(int s) {
 }
 static inline int64_t fa_spad(int64_t s) { return (s + FA_BK - 1) / FA_BK * FA_BK; }
 
-// One bit per 32-row x 64-key tile of a dense mask: 0 where every value is
-// zero (adding it changes nothing). bits [ceil(S/32)][ceil(S/2048)], bit t % 32
-// of word t / 32 for key tile t. The mask is the same for every head, so one
-// pass over it here saves the 32 passes that the heads' blocks would make
-// over its zero part (a mask is usually causal text rows above zero rows).
-// One wave per (strip, 8 key tiles: one byte); a lane reads 8 consecutive keys
-// of 4 rows per tile, all 32 loads in flight.
-__global__ __launch_bounds__(64) void fa_mask_bits_kernel(const uint16_t *mask, uint8_t *bits, int S) {
+// Two bits per 32-row x 64-key tile of a dense mask: "mixed" 0 where every
+// value is zero (adding it changes nothing) or every value is "dead": so low
+// that mask / scale + score is -inf for any finite score. Two arrays [ceil(S/32)]
+// [ceil(S/2048)], mixed then dead, bit t % 32 of word t / 32 for key tile t. The
+// mask is the same for every head, so one pass over it here saves the heads'
+// blocks reading the tiles that need no values (a mask is usually causal text
+// rows, dead right of the diagonal, above zero rows). One wave per (strip, 8
+// key tiles: one byte); a lane reads 8 consecutive keys of 4 rows per tile, all
+// 32 loads in flight. Reads past S are moved back into the row: a tile may
+// then count as mixed that is not, never the reverse. S >= 8.
+__global__ __launch_bounds__(64) void fa_mask_bits_kernel(const uint16_t *mask, uint8_t *mixed, uint8_t *dead,
+                                                          int S, float inv_scale) {
     const int lane = threadIdx.x;
-    uint32_t any[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int kv = (blockIdx.x * 8 + k) * 64 + (lane & 7) * 8;
-        any[k] = 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = blockIdx.y * 32 + i * 8 + (lane >> 3);
-            const uint16_t *p = mask + (size_t)row * S + kv;
-            if (row < S && kv + 8 <= S) {
-                u32x4_t v;
-                __builtin_memcpy(&v, p, 16);   // rows of an odd S start at any even address
-                any[k] |= v[0] | v[1] | v[2] | v[3];
-            } else if (row < S) {
-                for (int e = 0; kv + e < S; e++) any[k] |= (uint32_t)p[e];
-            }
-        }
-    }
-    uint32_t byte = 0;
+    u32x4_t v[8][4];
 #pragma unroll
     for (int k = 0; k < 8; k++)
-        if (__builtin_amdgcn_ballot_w64((any[k] & 0x7fff7fffu) != 0)) byte |= 1u << k;
-    if (lane == 0) bits[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = (uint8_t)byte;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int kv = min((int)(blockIdx.x * 8 + k) * 64 + (lane & 7) * 8, S - 8);
+            const int row = min((int)blockIdx.y * 32 + i * 8 + (lane >> 3), S - 1);
+            __builtin_memcpy(&v[k][i], mask + (size_t)row * S + kv, 16);   // an odd S: any even address
+        }
+    uint32_t m = 0, d = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        uint32_t any = 0;
+        bool low = true;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                any |= v[k][i][e];
+                // a quarter of the product still overflows: finite scores cannot bring it back
+                low = low && lo_bf(v[k][i][e]) * (0.25f * inv_scale) < -3.4028235e38f &&
+                      hi_bf(v[k][i][e]) * (0.25f * inv_scale) < -3.4028235e38f;
+            }
+        const bool all_low = __builtin_amdgcn_ballot_w64(!low) == 0;
+        if (all_low) d |= 1u << k;
+        else if (__builtin_amdgcn_ballot_w64((any & 0x7fff7fffu) != 0)) m |= 1u << k;
+    }
+    if (lane == 0) {
+        const size_t at = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+        mixed[at] = (uint8_t)m;
+        dead[at] = (uint8_t)d;
+    }
 }
 
 // Row tiling of the ping-pong kernel's units: per (batch, kv head) the rows
@@ -665,14 +678,23 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     // the phase's vmcnt wait covers them. Rows start at any even address (S
     // may be odd): unaligned 16-byte loads; the tile that holds key S - 1
     // reads element by element, clamped to the row.
-    // Tiles that fa_mask_bits_kernel found to be all zero are not read: bit t
-    // of this wave's 32-row strip, 32 tiles per lane of `mbits`.
+    // Tiles that fa_mask_bits_kernel found to be all zero or all dead are not
+    // read: bit t of this wave's 32-row strip, 32 tiles per lane.
     u32x4_t mk[2][2];
-    uint32_t mbits = ~0u;
+    uint32_t mbits = ~0u, dbits = 0u;
     if constexpr (MODE == FA_DENSE) {
-        const int strip = (qbase >> 5) + wave, nw = (a.S + FA_BK * 32 - 1) / (FA_BK * 32);
-        if (a.mask_bits) mbits = lane < nw && strip * 32 < a.S ? a.mask_bits[(size_t)strip * nw + lane] : 0u;
+        const int strip = (qbase >> 5) + wave, strips = (a.S + 31) / 32, nw = (a.S + FA_BK * 32 - 1) / (FA_BK * 32);
+        if (a.mask_bits) {
+            mbits = 0u;
+            if (lane < nw && strip < strips) {
+                mbits = a.mask_bits[(size_t)strip * nw + lane];
+                dbits = a.mask_bits[(size_t)(strips + strip) * nw + lane];
+            }
+        }
     }
+    auto is_dead = [&](int t) {
+        return MODE == FA_DENSE && (__builtin_amdgcn_readlane(dbits, t >> 5) >> (t & 31) & 1);
+    };
     auto has_mask = [&](int t) {
         return MODE == FA_DENSE && (__builtin_amdgcn_readlane(mbits, t >> 5) >> (t & 31) & 1);
     };
@@ -732,6 +754,13 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
                         const uint32_t m2 = mk[qq][u >> 1][(u & 1) * 2 + (e >> 1)];
                         s[qq][u][e] = fmaf(e & 1 ? hi_bf(m2) : lo_bf(m2), a.inv_scale, s[qq][u][e]);
                     }
+            }
+            if (is_dead(t)) {
+                asm volatile("");
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s[qq][u][e] -= INFINITY;
             }
             if (dead_keys) {
                 asm volatile("");   // a branch, not 32 selects in every tile
@@ -996,10 +1025,10 @@ extern "C" void hd_flash_make_vt(const void *v, void *vt, int bh, int seq) {
     hd_check_launch("flash_make_vt");
 }
 
-// Bytes of the zero-tile bits of a dense mask (0: too long for one lane per word).
+// Bytes of the tile bits of a dense mask (0: too long for one lane per word).
 static int64_t fa_mask_bits_bytes(int seq) {
     const int64_t words = (seq + FA_BK * 32 - 1) / (FA_BK * 32);
-    return words <= 64 ? (seq + 31) / 32 * words * 4 : 0;
+    return words <= 64 ? (seq + 31) / 32 * words * 8 : 0;
 }
 
 static int fa_launch(const void *q, const void *k, const void *vt, const void *mask, void *out,
@@ -1046,8 +1075,9 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     //    (S = 4239, 142 causal rows, one masked 4-wave launch: 314 -> 270 us;
     //    S = 16499: 4080 -> 3630; 2 x 1101 rows: equal), or
     //  * there is a dense mask: its values are prefetched as 8-byte pieces
-    //    under the MFMA phase and skipped where they are zero (4-wave blocks
-    //    with 2-byte loads: S = 300 26.8 -> 21.8 us, 1209 201 -> 53; equal
+    //    under the MFMA phase, where a tile needs them (4-wave blocks
+    //    with 2-byte loads, causal text rows above zeros: S = 300 26.6 ->
+    //    25.6 us, 1209 199 -> 57, 4239 1937 -> 318; equal
     //    at 200, where one 256-row block per head is as long as two of 128).
     const bool pp = mask ? seq >= FA_PP_MIN_DENSE : seq >= FA_PP_MIN && (prefix || (ws && ar_len == 0));
     const int nwv = pp ? 8 : 4;
@@ -1082,7 +1112,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     a.split = 1;
     a.part = (float *)ws;
     int n_tail = 0;
-    // dense mask: the zero-tile bits lie behind the partials in the workspace
+    // dense mask: the tile bits lie behind the partials in the workspace
     const int64_t bits_bytes = pp && mask && q_row_begin == 0 ? fa_mask_bits_bytes(seq) : 0;
     const bool bits = bits_bytes > 0 && ws && bits_bytes <= ws_bytes;
     if (bits) ws_bytes -= bits_bytes;
@@ -1106,7 +1136,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     if (bits) {
         uint8_t *at = (uint8_t *)ws + (int64_t)a.n_chunks * BQ * (FA_D + 2) * 4;
         fa_mask_bits_kernel<<<dim3((seq + FA_BK * 32 - 1) / (FA_BK * 32) * 4, (seq + 31) / 32), 64, 0, st>>>(
-            (const uint16_t *)mask, at, seq);
+            (const uint16_t *)mask, at, at + bits_bytes / 2, seq, a.inv_scale);
         a.mask_bits = (const uint32_t *)at;
     }
     dim3 grid((unsigned)(a.n_whole + a.n_chunks + n_causal));

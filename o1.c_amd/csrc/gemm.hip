@@ -940,7 +940,7 @@ static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr,
     const int p192 = ws ? tail_split_of(t192, nk, (size_t)192 * 256 * 4, ws_bytes) : 1;
     const int p128 = ws ? tail_split_of(t128, nk, (size_t)128 * 128 * 4, ws_bytes, 0, 2) : 1;
     const double c256 = tile_cost(t256, 1, 256, 256, g.K, 1.0, p256);
-    const double c192 = tile_cost(t192, 1, 192, 256, g.K, 0.9, p192);
+    const double c192 = tile_cost(t192, 1, 192, 256, g.K, 0.85, p192);
     const double c128 = tile_cost(t128, 2, 128, 128, g.K, 0.8, p128);
     // buffer loads address with 32-bit byte offsets: both operands under 2 GiB
     const bool fits = (size_t)(g.M + 256) * g.K * 2 < ((size_t)1 << 31) &&
@@ -1048,7 +1048,7 @@ int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *
         return tail_split_of(t, nk, (size_t)bm * bn * 4, ws_bytes, (size_t)bm * bn * 2, occ);
     };
     const double c256 = tile_cost(t256, 1, 256, 256, hidden, 1.0, split(t256, 256, 256, 1));
-    const double c192 = tile_cost(t192, 1, 192, 256, hidden, 0.9, split(t192, 192, 256, 1));
+    const double c192 = tile_cost(t192, 1, 192, 256, hidden, 0.85, split(t192, 192, 256, 1));
     const double c128 = tile_cost(t128, 2, 128, 128, hidden, 0.8, split(t128, 128, 128, 2));
     if (c128 < c256 && c128 < c192) launch_ms<128, 128, 64, 2, 2, 2, EPI_QKV, 8, 2, 5, 16>(g, ws, ws_bytes);
     else if (c192 < c256) launch_ms<192, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws_bytes);
