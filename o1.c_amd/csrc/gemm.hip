@@ -27,7 +27,8 @@
 #include "../../include/hd_hip.h"
 #include "../../include/hd_gemm.h"
 
-enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_RES = 2, EPI_SWIGLU = 3, EPI_QKV = 4 };
+// GELU / GELU_ERF: bias, then the tanh / erf form on the bf16 sum
+enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_RES = 2, EPI_SWIGLU = 3, EPI_QKV = 4, EPI_GELU = 5, EPI_GELU_ERF = 6 };
 
 struct GemmArgs {
     const uint16_t *A;       // [M, K]
@@ -682,6 +683,357 @@ __global__ __launch_bounds__(WGM * WGN * 64, OCC) void gemm_ms_kernel(GemmArgs g
 }
 
 // ---------------------------------------------------------------------------
+// Middle-sized grids: one block of 8 waves per tile in two K groups of 4 waves
+// (WGM x WGN). Where the 256 x 256 tiles of a GEMM fill the chip badly, tiles
+// have to be smaller, and a small tile on 4 waves leaves one wave per SIMD with
+// nothing to hide its barrier and fragment reads behind; two blocks per CU give
+// a second wave only where the grid has 512 blocks. Here the second wave of
+// each SIMD works on the same tile: group 0 takes the first 32 of every 64-deep
+// K tile, group 1 the second, and the groups' accumulators meet in LDS at the
+// end (each wave adds its partner's half and finishes half of the rows).
+//  * LDS ring of NS stages filled by buffer loads straight to LDS; at tile kt
+//    the wait covers tile kt + 1, and kt + NS goes into the stage that tile kt's
+//    fragments have left. Loads past the chunk's or the matrix's K read as
+//    zero (per-lane offset past the records), so K % 8 == 0 is enough, the loop
+//    has no tail forms, and an odd tile count runs one tile of zeros;
+//  * the fragments of tile kt + 1 are read under the MFMAs of tile kt.
+// Per 64-deep K tile and CU the 8 waves read 8 (TM + TN) KB of fragments at
+// 128 B per cycle and issue 2 TM TN MFMAs of 16 cycles per SIMD: 640 against
+// 768 cycles for 192 x 128, 512 / 512 for 128 x 128, 384 / 256 for 128 x 64 and
+// 256 / 128 for 64 x 64, so the largest tile that still fills the CUs wins.
+// Measured (us, against the tiled kernels): o_proj of 94 rows 32.3 -> 17, of
+// 1152 rows 51.8 -> 45; SwiGLU of 94 rows 56 -> 46; 576 x 1152 x 1152 12.3 ->
+// 7.4; 576 x 1152 x 4352 25.3 -> 17.0; 432 x 4608 x 4608 40.9 -> 28.0.
+// ---------------------------------------------------------------------------
+template <int BM, int BN, int NS, int EPI, int OCC>
+__global__ __launch_bounds__(512, OCC) void gemm_kg_kernel(GemmArgs g) {
+    constexpr int WGM = 2, WGN = 2, WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 16, TN = WTN / 16, HM = TM / 2;
+    constexpr int BK = 64, AI = BM / 64, BI = BN / 64, LPT = AI + BI, STAGE = (BM + BN) * BK, GROUP_M = 8;
+    constexpr int WO = EPI == EPI_SWIGLU ? WTN / 2 : WTN, BN_OUT = WGN * WO;
+    static_assert(BM % 64 == 0 && BN % 64 == 0 && TM % 2 == 0 && (NS - 2) * LPT < 64, "tile");
+    static_assert(EPI != EPI_QKV || BN == 128, "one head per tile column");
+    constexpr int EXCH = 8 * HM * TN * 1024, STG = 8 * HM * 16 * (WO + 8) * 2;
+    constexpr int LDS0 = NS * STAGE * 2 > EXCH ? NS * STAGE * 2 : EXCH, LDS = LDS0 > STG ? LDS0 : STG;
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[LDS / 2];
+
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    int lin, chunk = -1, item = 0;
+    const int n_chunks = (int)gridDim.x - g.n_whole;
+    if ((int)blockIdx.x >= n_chunks) {
+        lin = xcd_remap(blockIdx.x - n_chunks, g.n_whole);
+    } else {
+        item = blockIdx.x;
+        chunk = item % g.split;
+        lin = g.n_whole + item / g.split;
+    }
+    const int in_group = GROUP_M * g.ntn, first_m = (lin / in_group) * GROUP_M;
+    const int gm = min(g.ntm - first_m, GROUP_M);
+    const int tm = first_m + (lin % in_group) % gm, tn = (lin % in_group) / gm;
+    const int m0 = tm * BM;
+    int kbase = 0, nk = (g.K + BK - 1) / BK;
+    if (chunk >= 0) {
+        const int k0 = chunk * nk / g.split, k1 = (chunk + 1) * nk / g.split;
+        kbase = k0;
+        nk = k1 - k0;
+    }
+    const int klim = min(g.K, (kbase + nk) * BK);   // first k that reads as zero
+
+    // loader: one instruction fills 8 tile rows of 128 bytes, chunks swizzled by row
+    const int sub = lane >> 3, cl = lane & 7;
+    const int bt0 = tn * BN;
+    const int bsg = EPI == EPI_SWIGLU ? 0 : (bt0 < g.seg_end[0] ? 0 : (bt0 < g.seg_end[1] ? 1 : 2));
+    const int bbase = bsg == 0 ? 0 : (bsg == 1 ? g.seg_end[0] : g.seg_end[1]);
+    const int brows = EPI == EPI_SWIGLU ? g.N
+                                        : (bsg == 0 ? g.seg_end[0] : (bsg == 1 ? g.seg_end[1] : g.seg_end[2])) - bbase;
+    const void *bp0 = bsg == 0 ? g.B[0] : (bsg == 1 ? g.B[1] : g.B[2]), *bp1 = g.B[1];
+    const int nb_a = (int)((size_t)g.M * g.K * 2), nb_b = (int)((size_t)brows * g.K * 2);
+    uint32_t a_vo[AI], b_vo[BI];
+    int b_up[BI], a_kc[AI], b_kc[BI];
+#pragma unroll
+    for (int i = 0; i < AI; i++) {
+        const int r = (wave * AI + i) * 8 + sub;
+        a_kc[i] = (cl ^ ms_swz<8>(r)) * 8;
+        a_vo[i] = m0 + r < g.M ? ((uint32_t)(m0 + r) * (uint32_t)g.K + a_kc[i]) * 2 : 0x80000000u;
+    }
+#pragma unroll
+    for (int i = 0; i < BI; i++) {
+        const int r = (wave * BI + i) * 8 + sub;
+        int n = bt0 + r - bbase;
+        b_up[i] = 0;
+        if (EPI == EPI_SWIGLU) {   // each wave column: WO gate rows, then the up rows of the same outputs
+            const int grp = r / WTN, j = r % WTN;
+            n = tn * BN_OUT + grp * WO + j % WO;
+            b_up[i] = __builtin_amdgcn_readfirstlane(((wave * BI + i) * 8) % WTN >= WO);
+        }
+        b_kc[i] = (cl ^ ms_swz<8>(r)) * 8;
+        b_vo[i] = n < brows ? ((uint32_t)n * (uint32_t)g.K + b_kc[i]) * 2 : 0x80000000u;
+    }
+    auto issue = [&](int kt) {
+        uint16_t *As = smem + (kt % NS) * STAGE, *Bs = As + BM * BK;
+        // a tile past the last one: the scalar offset stays inside the records
+        // (the range check subtracts it from their size)
+        const int k = (kbase + kt) * BK;
+        const uint32_t so = k < klim ? (uint32_t)k * 2 : 0u;
+#pragma unroll
+        for (int i = 0; i < AI; i++)
+            buf_load_lds16(g.A, nb_a, k + a_kc[i] < klim ? a_vo[i] : 0x80000000u, so,
+                           (HD_LDS void *)(As + (wave * AI + i) * 512));
+#pragma unroll
+        for (int i = 0; i < BI; i++)
+            buf_load_lds16(b_up[i] ? bp1 : bp0, nb_b, k + b_kc[i] < klim ? b_vo[i] : 0x80000000u, so,
+                           (HD_LDS void *)(Bs + (wave * BI + i) * 512));
+    };
+
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    bf16x8_t af[2][TM], bw[2][TN];
+    const int c = ((kg * 4 + lg) ^ ms_swz<8>(l16)) * 8;
+    auto ld = [&](int kt, int sl) {
+        const uint16_t *As = smem + (kt % NS) * STAGE, *Bs = As + BM * BK;
+#pragma unroll
+        for (int i = 0; i < TM; i++) af[sl][i] = *(const bf16x8_t *)(As + (wm * WTM + i * 16 + l16) * BK + c);
+#pragma unroll
+        for (int j = 0; j < TN; j++) bw[sl][j] = *(const bf16x8_t *)(Bs + (wn * WTN + j * 16 + l16) * BK + c);
+    };
+#pragma unroll
+    for (int t = 0; t < NS; t++) issue(t);
+    wait_vm_barrier<(NS - 1) * LPT>();
+    ld(0, 0);
+    auto tile = [&](int kt, auto par) {
+        constexpr int SL = decltype(par)::value;
+        wait_lgk_vm_barrier<(NS - 2) * LPT>();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(kt + NS);
+        ld(kt + 1, SL ^ 1);
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[SL][j], af[SL][i], acc[i][j], 0, 0, 0);
+        // fragment reads and refill loads between the MFMAs
+#pragma unroll
+        for (int q = 0; q < TM * TN; q++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (q < TM + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (q < LPT) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+    };
+    for (int kt = 0; kt < nk; kt += 2) {
+        tile(kt, std::integral_constant<int, 0>{});
+        tile(kt + 1, std::integral_constant<int, 1>{});
+    }
+    // the ring's loads have landed and every wave has left it
+    wait_lgk_vm_barrier<0>();
+    // the two groups' sums: wave w and w ^ 4 hold the same tile; group 0 keeps
+    // the first half of the row tiles, group 1 the second
+    f32x4_t *xch = (f32x4_t *)smem;
+#pragma unroll
+    for (int i = 0; i < HM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            xch[(wave * HM * TN + i * TN + j) * 64 + lane] = kg ? acc[i][j] : acc[HM + i][j];
+    __syncthreads();
+    f32x4_t sum[HM][TN];
+#pragma unroll
+    for (int i = 0; i < HM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            sum[i][j] = (kg ? acc[HM + i][j] : acc[i][j]) + xch[((wave ^ 4) * HM * TN + i * TN + j) * 64 + lane];
+    const int r0 = wm * WTM + kg * HM * 16;   // this wave's first row of the tile
+    if (chunk >= 0) {
+        float *pt = g.part + (size_t)item * BM * BN;
+#pragma unroll
+        for (int i = 0; i < HM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                *(f32x4_t *)(pt + (size_t)(r0 + i * 16 + l16) * BN + wn * WTN + j * 16 + lg * 4) = sum[i][j];
+        return;
+    }
+    constexpr int HR = HM * 16;
+    constexpr bool QKV = EPI == EPI_QKV;
+    constexpr int LDW = QKV ? 128 + 8 : WO + 8;
+    // QKV: the two waves of a row band stage one 128-wide head side by side
+    uint16_t *const band = smem + (kg * 2 + wm) * 2 * HR * (WO + 8);
+    uint16_t *stg = QKV ? band + wn * 64 : band + wn * HR * LDW;
+    static_assert(!QKV || HR * LDW <= 2 * HR * (WO + 8), "QKV staging");
+    __syncthreads();   // the exchange area has been read
+#pragma unroll
+    for (int i = 0; i < HM; i++)
+#pragma unroll
+        for (int j = 0; j < (EPI == EPI_SWIGLU ? TN / 2 : TN); j++) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = sum[i][j][e];
+                if (EPI == EPI_SWIGLU) v[e] = bfround(silu_rcp(bfround(v[e]))) * bfround(sum[i][j + TN / 2][e]);
+            }
+            *(u32x2_t *)(stg + (i * 16 + l16) * LDW + j * 16 + lg * 4) = (u32x2_t){pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        }
+    __syncthreads();
+    if constexpr (QKV) {
+        // the band's rows in multiples of 16 for the V^T groups
+        constexpr int H0 = (HR / 16 + 1) / 2 * 16, H1 = HR - H0;
+        if (wn == 0) qkv_epilogue<H0, LDW>(g, band, m0 + r0, tn, lane);
+        else if constexpr (H1 > 0) qkv_epilogue<H1, LDW>(g, band + H0 * LDW, m0 + r0 + H0, tn, lane);
+        return;
+    }
+    constexpr int CPRO = WO / 8, RPIO = 64 / CPRO;
+    const int gn0 = tn * BN_OUT + wn * WO;
+#pragma unroll
+    for (int q = 0; q < HR; q += RPIO) {
+        const int r = q + lane / CPRO, cc = (lane % CPRO) * 8;
+        const int m = m0 + r0 + r, n = gn0 + cc;
+        if (r < HR && m < g.M && n < g.N) {
+            u32x4_t v = *(const u32x4_t *)(stg + r * LDW + cc);
+            if (EPI != EPI_NONE && EPI != EPI_SWIGLU) {
+                const u32x4_t o = *(const u32x4_t *)(EPI == EPI_RES ? g.res + (size_t)m * g.ldc + n : g.bias + n);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = pack_bf2(lo_bf(v[e]) + lo_bf(o[e]), hi_bf(v[e]) + hi_bf(o[e]));
+                if (EPI == EPI_GELU || EPI == EPI_GELU_ERF)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        v[e] = EPI == EPI_GELU ? pack_bf2(gelu_tanh_f(lo_bf(v[e])), gelu_tanh_f(hi_bf(v[e])))
+                                               : pack_bf2(gelu_erf_f(lo_bf(v[e])), gelu_erf_f(hi_bf(v[e])));
+            }
+            *(u32x4_t *)(g.C + (size_t)m * g.ldc + n) = v;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows (M <= 16 * TM): the weight is read once from memory and sets the
+// time, so every CU has to stream its share of it. A block owns 16 * TN weight
+// rows and all of M; its 8 waves take the 64-deep K tiles round robin and read
+// both operands straight into registers (no wave shares an operand element
+// with another, so LDS would only add a copy), PD tiles ahead. A lane's 16
+// consecutive k of a tile feed two MFMAs: whole 128-byte lines per row, and
+// the same k order in both operands. The waves' sums meet in LDS, 8 tiles of
+// 16 x 16 at a time, and the thread that adds them applies the epilogue.
+// SwiGLU: the first TN / 2 tiles are gate rows, the others up rows of the same
+// columns.
+// 4096 x 4096, against one 128 x 128 tile per 128 weight rows (32 blocks on 256
+// CUs): 2 rows 30.3 -> 7.7 us (4.4 TB/s), 16 rows 30.6 -> 9.6. Past 16 rows the
+// activations, read again by every block in 64-byte row pieces, take over.
+// ---------------------------------------------------------------------------
+template <int TM, int TN, int PD, int EPI>
+__global__ __launch_bounds__(512, 1) void gemm_skinny_kernel(GemmArgs g) {
+    constexpr int NWV = 8, CH = 8, TNO = EPI == EPI_SWIGLU ? TN / 2 : TN;
+    __shared__ __attribute__((aligned(16))) f32x4_t red[NWV][CH][64];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * 16 * TNO, K = g.K, nkt = K / 64;
+    const uint16_t *bp[TN], *ap[TM];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int n = min(n0 + (j % TNO) * 16 + l16, g.N - 1);
+        bp[j] = (EPI == EPI_SWIGLU && j >= TNO ? g.B[1] : g.B[0]) + (size_t)n * K + wave * 64 + lg * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+        ap[i] = g.A + (size_t)min(i * 16 + l16, g.M - 1) * K + wave * 64 + lg * 16;
+    f32x4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    bf16x8_t bw[PD][TN][2], af[PD][TM][2];
+    auto load = [&](int t, int sl) {
+        const int o = t * NWV * 64;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            bw[sl][j][0] = *(const bf16x8_t *)(bp[j] + o);
+            bw[sl][j][1] = *(const bf16x8_t *)(bp[j] + o + 8);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            af[sl][i][0] = *(const bf16x8_t *)(ap[i] + o);
+            af[sl][i][1] = *(const bf16x8_t *)(ap[i] + o + 8);
+        }
+    };
+    auto mul = [&](int sl) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[sl][j][h], af[sl][i][h], acc[i][j], 0, 0, 0);
+    };
+    const int nt = (nkt - wave + NWV - 1) / NWV;   // this wave's K tiles
+#pragma unroll
+    for (int s = 0; s < PD; s++)
+        if (s < nt) load(s, s);
+    int t = 0;
+    for (; t + 2 * PD <= nt; t += PD)
+#pragma unroll
+        for (int s = 0; s < PD; s++) {
+            mul(s);
+            load(t + s + PD, s);
+        }
+    for (; t < nt; t += PD)
+#pragma unroll
+        for (int s = 0; s < PD; s++)
+            if (t + s < nt) {
+                mul(s);
+                if (t + s + PD < nt) load(t + s + PD, s);
+            }
+    // sums over the waves: items (row tile i, output tile j); SwiGLU items are
+    // gate / up pairs, half as many per pass
+    constexpr int IPP = EPI == EPI_SWIGLU ? CH / 2 : CH, ITEMS = TM * TNO;
+#pragma unroll
+    for (int p = 0; p < ITEMS; p += IPP) {
+        if (p) __syncthreads();
+#pragma unroll
+        for (int q = 0; q < IPP; q++) {
+            if (p + q < ITEMS) {
+                const int i = (p + q) / TNO, j = (p + q) % TNO;
+                red[wave][q][lane] = acc[i][j];
+                if (EPI == EPI_SWIGLU) red[wave][q + IPP][lane] = acc[i][j + TNO];
+            }
+        }
+        __syncthreads();
+        const int q = threadIdx.x >> 6;
+        if (q < IPP && p + q < ITEMS) {
+            const int i = (p + q) / TNO, j = (p + q) % TNO;
+            const int m = i * 16 + l16, n = n0 + j * 16 + lg * 4;
+            f32x4_t a = red[0][q][lane], u;
+#pragma unroll
+            for (int w = 1; w < NWV; w++) a += red[w][q][lane];
+            if (EPI == EPI_SWIGLU) {
+                u = red[0][q + IPP][lane];
+#pragma unroll
+                for (int w = 1; w < NWV; w++) u += red[w][q + IPP][lane];
+#pragma unroll
+                for (int e = 0; e < 4; e++) a[e] = bfround(silu_rcp(bfround(a[e]))) * bfround(u[e]);
+            }
+            if (m < g.M && n < g.N) {
+                u32x2_t pk = {pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
+                if (EPI == EPI_BIAS || EPI == EPI_RES) {
+                    const uint16_t *o = EPI == EPI_BIAS ? g.bias + n : g.res + (size_t)m * g.ldc + n;
+                    const u32x2_t ov = *(const u32x2_t *)o;
+#pragma unroll
+                    for (int e = 0; e < 2; e++)
+                        pk[e] = pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e]));
+                }
+                *(u32x2_t *)(g.C + (size_t)m * g.ldc + n) = pk;
+            }
+        }
+    }
+}
+
+template <int EPI> static void launch_skinny(GemmArgs &g) {
+    constexpr int TN = EPI == EPI_SWIGLU ? 2 : 1;
+    const unsigned nb = (unsigned)((g.N + 15) / 16);
+    if (g.M <= 16) gemm_skinny_kernel<1, TN, 8, EPI><<<nb, 512, 0, hd_stream()>>>(g);
+    else gemm_skinny_kernel<2, TN, 4, EPI><<<nb, 512, 0, hd_stream()>>>(g);
+}
+
+// ---------------------------------------------------------------------------
 // Reference kernel (gemm.cu:35-70 role): one fp32 dot product per output,
 // y = bf16(acc + bias). Correctness/debug backend and the fallback for
 // shapes the MFMA kernels do not take (K % 64, N % 8, misaligned).
@@ -782,11 +1134,15 @@ __global__ void gemm_tail_merge_kernel(GemmArgs g, int n_tail) {
         v[e] = x;
     }
     u32x2_t pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-    if (EPI == EPI_BIAS || EPI == EPI_RES) {
-        const uint16_t *o = EPI == EPI_BIAS ? g.bias + n : g.res + (size_t)m * g.ldc + n;
+    if (EPI != EPI_NONE && EPI != EPI_SWIGLU) {
+        const uint16_t *o = EPI == EPI_RES ? g.res + (size_t)m * g.ldc + n : g.bias + n;
         const u32x2_t ov = *(const u32x2_t *)o;
 #pragma unroll
-        for (int e = 0; e < 2; e++) pk[e] = pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e]));
+        for (int e = 0; e < 2; e++) {
+            pk[e] = pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e]));
+            if (EPI == EPI_GELU) pk[e] = pack_bf2(gelu_tanh_f(lo_bf(pk[e])), gelu_tanh_f(hi_bf(pk[e])));
+            if (EPI == EPI_GELU_ERF) pk[e] = pack_bf2(gelu_erf_f(lo_bf(pk[e])), gelu_erf_f(hi_bf(pk[e])));
+        }
     }
     *(u32x2_t *)(g.C + (size_t)m * g.ldc + n) = pk;
 }
@@ -927,8 +1283,130 @@ static double tile_cost(long units, int occ, int BM, int BNA, int K, double eff,
     return t;
 }
 
+template <int BM, int BN, int NS, int EPI, int OCC>
+static void launch_kg(GemmArgs &g, int P, void *ws) {
+    constexpr int BN_OUT = EPI == EPI_SWIGLU ? BN / 2 : BN;
+    g.ntm = (g.M + BM - 1) / BM;
+    g.ntn = (g.N + BN_OUT - 1) / BN_OUT;
+    const long units = (long)g.ntm * g.ntn;
+    const long n_tail = P > 1 ? units : 0;   // a split covers every tile
+    g.n_whole = (int)(units - n_tail);
+    g.split = P;
+    g.part = (float *)ws;
+    gemm_kg_kernel<BM, BN, NS, EPI, OCC><<<(unsigned)(g.n_whole + n_tail * P), 512, 0, hd_stream()>>>(g);
+    if (n_tail) {
+        if constexpr (EPI == EPI_QKV)
+            gemm_tail_qkv_fused_kernel<BM, BN, QKV_TAIL_RS>
+                <<<(unsigned)(n_tail * (BM / QKV_TAIL_RS) * (BN / 128)), 64, 0, hd_stream()>>>(g, (int)n_tail);
+        else
+            gemm_tail_merge_kernel<BM, BN, 2, EPI>
+                <<<hd_cdiv((size_t)n_tail * BM * (BN_OUT / 4), 256), 256, 0, hd_stream()>>>(g, (int)n_tail);
+    }
+}
+// Choice for grids of at most two rounds of 256 x 256 tiles. Measured us per
+// 64-deep K tile of one block per CU (warm and cold operands of the block's and
+// the vision tower's shapes), and per round what it costs beside its
+// K tiles:
+//   256x256 1.50, 192x256 1.32, old 128x128 0.45 alone and 0.90 for two per CU;
+//   K-group tiles 256x128 0.90, 192x128 0.66, 128x128 0.50, 64x128 0.345,
+//   64x64 0.21; the last two fit a CU twice, at 1.7-2 times the time.
+// The 128-wide families take 15 % longer on SwiGLU's two weights and, unsplit,
+// past K = 8192; the old 128 x 128 tiles 30 % longer when every tile is split.
+// A split adds the merge launch and its partials, written and read at 8 TB/s
+// (L2 and the cache behind it hold most). Tiles this small re-read the
+// operands: once these do not fit the L2s (32 MB in all) the re-reads are
+// served at 12-18 TB/s.
+struct SmallPick {
+    int fam, P;   // fam 0..4: kKg; 5 old 128x128, 6 192x256, 7 256x256
+    double us;
+};
+struct KgFam {
+    int bm, bn;
+    double us, fixed;
+    bool twice;
+};
+constexpr KgFam kKg[5] = {{64, 64, 0.21, 1.5, true}, {64, 128, 0.345, 1.5, true}, {128, 128, 0.50, 1.5, false},
+                          {192, 128, 0.66, 3.0, false}, {256, 128, 0.90, 3.0, false}};
+static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t ws_bytes) {
+    SmallPick best = {7, 1, 1e30};
+    const int nk = (K + 63) / 64;
+    const double foot = 2.0 * K * ((double)M + (swiglu ? 2.0 : 1.0) * N);
+    auto merge_us = [&](double tiles, int P, int bm, int bn) { return 5.0 + tiles * P * bm * bn * 8.0 / 8e6; };
+    auto offer = [&](int fam, int P, double us) {
+        if (fam < 6) us *= 1.03;   // near ties go to the large tiles
+        if (us < best.us) best = {fam, P, us};
+    };
+    for (int f = qkv ? 1 : 0; f < 5; f++) {
+        const KgFam &k = kKg[f];
+        const long tiles = (long)((M + k.bm - 1) / k.bm) * ((N + (swiglu ? k.bn / 2 : k.bn) - 1) / (swiglu ? k.bn / 2 : k.bn));
+        for (int P = 1; P <= 8; P++) {
+            if (P > 1 && (nk / P < 4 || tiles * P > (k.twice ? 512 : 256) ||
+                          (int64_t)tiles * P * k.bm * k.bn * 4 > ws_bytes))
+                break;
+            const double u = (double)tiles * P / 256;
+            const double rounds = u <= 1 ? 1.0 : !k.twice ? (double)((tiles * P + 255) / 256)
+                                                 : u <= 2 ? 1.4 + 0.3 * u : 1.1 * u;
+            double t = 3.0 + rounds * (k.fixed + ((nk + P - 1) / P) * k.us * (swiglu || K > 8192 ? 1.15 : 1.0));
+            const double reread = tiles * (double)(k.bm + k.bn) * K * 2;
+            if (foot > 32e6 && reread / 12e6 > t) t = reread / 12e6;
+            offer(f, P, t + (P > 1 ? merge_us(tiles, P, k.bm, k.bn) : 0.0));
+        }
+    }
+    auto big = [&](int fam, int bm, int bna, int occ, double us1, double us2, size_t stage) {
+        const int bn = swiglu ? bna / 2 : bna;
+        const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn), slots = 256L * occ;
+        const int P = tail_split_of(tiles, nk, (size_t)bm * bna * 4, ws_bytes, stage, occ);
+        const long full = tiles / slots, rem = tiles % slots;
+        if (occ == 2 && swiglu && tiles <= 256) return;   // one wave per SIMD: 0.83 on two cold weights
+        const double usf = occ == 2 ? us2 : us1;
+        auto round = [&](long n) { return n <= 256 ? us1 : us1 * 1.6 + (us2 - us1 * 1.6) * (n - 256) / 256; };
+        if (rem && P > 1)
+            offer(fam, P, 4.0 + full * nk * usf + (nk + P - 1) / P * (full || occ == 1 ? usf : 1.3 * usf) +
+                              merge_us(rem, P, bm, bna));
+        double t = 4.0 + nk * (full * usf + (rem ? (occ == 2 ? round(rem) : us1) : 0.0));
+        if (occ == 2) {
+            if (K > 8192) t *= 1.15;
+            const double reread = tiles * (double)(bm + bna) * K * 2;
+            if (foot > 32e6 && reread / 18e6 > t) t = reread / 18e6;
+        }
+        offer(fam, 1, t);
+    };
+    if (K % 64 == 0) {
+        const size_t s = qkv ? 2 : 0;
+        big(5, 128, 128, 2, swiglu ? 0.55 : 0.45, swiglu ? 1.10 : 0.90, s * 128 * 128);
+        big(6, 192, 256, 1, 1.32, 1.32, s * 192 * 256);
+        big(7, 256, 256, 1, 1.50, 1.50, s * 256 * 256);
+    }
+    return best;
+}
+template <int EPI> static const char *launch_small(GemmArgs &g, const SmallPick &b, bool launch, void *ws, int64_t ws_bytes) {
+    static const char *name[8] = {"bf16_64x64x64_kg2", "bf16_64x128x64_kg2", "bf16_128x128x64_kg2", "bf16_192x128x64_kg2",
+                                  "bf16_256x128x64_kg2", "bf16_128x128x64_w2x2_occ2_m16", "bf16_192x256x64_w2x4_m16_ring_buf",
+                                  "bf16_256x256x64_w2x4_m16_ring_buf"};
+    if (b.P == 1) ws = nullptr;   // the tiled families split by themselves when they are given a workspace
+    if (launch) switch (b.fam) {
+    case 0: if constexpr (EPI != EPI_QKV) launch_kg<64, 64, 5, EPI, 4>(g, b.P, ws); break;
+    case 1: launch_kg<64, 128, 3, EPI, 4>(g, b.P, ws); break;
+    case 2: launch_kg<128, 128, 5, EPI, 1>(g, b.P, ws); break;
+    case 3: launch_kg<192, 128, 4, EPI, 1>(g, b.P, ws); break;
+    case 4: launch_kg<256, 128, 3, EPI, 1>(g, b.P, ws); break;
+    case 5: launch_ms<128, 128, 64, 2, 2, 2, EPI, 8, 2, 5, 16>(g, ws, ws_bytes); break;
+    case 6: launch_ms<192, 256, 64, 2, 2, 4, EPI, 8, 1, 5, 16>(g, ws, ws_bytes); break;
+    case 7: launch_ms<256, 256, 64, 2, 2, 4, EPI, 8, 1, 5, 16>(g, ws, ws_bytes); break;
+    }
+    return name[b.fam];
+}
+
 template <int EPI>
 static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr, int64_t ws_bytes = 0) {
+    // few rows (one segment of weights only: concat3 keeps the tiled kernels);
+    // past 16 rows the activations' re-reads catch up with the weight: at 32
+    // rows 13.0 us against 16 (4096 x 4096), but 41 against 31 (K = 12288)
+    const bool one_seg = EPI == EPI_SWIGLU || g.seg_end[0] == g.N;
+    if (one_seg && g.K % 64 == 0 && (g.M <= 16 || (g.M <= 32 && g.K <= 4096 && EPI != EPI_SWIGLU))) {
+        if (launch) launch_skinny<EPI>(g);
+        return "bf16_skinny";
+    }
     const int bn_out = EPI == EPI_SWIGLU ? 128 : 256;
     const long tn = (g.N + bn_out - 1) / bn_out;
     const long t256 = (long)((g.M + 255) / 256) * tn;
@@ -957,17 +1435,9 @@ static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr,
         if (launch) launch_ms<256, 256, 64, 2, 2, 4, EPI, 3, 1, 0, 16>(g, ws, ws_bytes);
         return split256 ? "bf16_256x256x64_w2x4_m16_ring_tailsplit" : "bf16_256x256x64_w2x4_m16_ring";
     }
-    // Small grids (the 256 x 256 tiles fill at most one round, K <= 4096, no
-    // SwiGLU): 128 x 128 tiles, two blocks per CU, no K split. The vision
-    // tower's M = 1728 GEMMs (K = 1152): 11.5-20 us against 22-27 us with a
-    // 4-chunk K split; a 1152-token block's o_proj: equal at block level.
-    // Longer K (the 12288-deep down projection) and the SwiGLU epilogue stay
-    // on the 256-row tiles (120 vs 139-150 us; 192-212 vs 208-223 us).
-    const int slots1 = gemm_slots() > 0 ? gemm_slots() : 256;
-    if (EPI != EPI_SWIGLU && t256 <= slots1 && g.K <= 4096) {
-        if (launch) launch_ms<128, 128, 64, 2, 2, 2, EPI, 8, 2, 5, 16>(g);
-        return "bf16_128x128x64_w2x2_occ2_m16";
-    }
+    if (t256 <= 512)
+        return launch_small<EPI>(g, pick_small(g.M, g.N, g.K, EPI == EPI_SWIGLU, false, ws ? ws_bytes : 0), launch, ws,
+                                 ws ? ws_bytes : 0);
     if (c128 < c256 && c128 < c192) {
         if (launch) launch_ms<128, 128, 64, 2, 2, 2, EPI, 8, 2, 5, 16>(g, ws, ws_bytes);
         return p128 > 1 ? "bf16_128x128x64_w2x2_occ2_m16_split" : "bf16_128x128x64_w2x2_occ2_m16";
@@ -1043,6 +1513,11 @@ int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *
     const long t128 = (long)((M + 127) / 128) * tn * 2;
     if (ws && (uintptr_t)ws % 16) ws = nullptr;
     if (!ws) ws_bytes = 0;
+    if (t256 <= 512) {
+        launch_small<EPI_QKV>(g, pick_small(M, N, hidden, false, true, ws_bytes), true, ws, ws_bytes);
+        hd_check_launch("linear_qkv_rope");
+        return 0;
+    }
     const int nk = hidden / 64;
     auto split = [&](long t, int bm, int bn, int occ) {
         return tail_split_of(t, nk, (size_t)bm * bn * 4, ws_bytes, (size_t)bm * bn * 2, occ);

@@ -35,6 +35,14 @@ __device__ __forceinline__ float bfround(float f) { return bf2f(f2bf(f)); }
 __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
 
+// ---- GELU, tanh and erf forms (vision_kernels.cu) -----------------------
+__device__ __forceinline__ float gelu_tanh_f(float v) {
+    return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+}
+__device__ __forceinline__ float gelu_erf_f(float v) {
+    return 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
+}
+
 // ---- MFMA operand types -------------------------------------------------
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));

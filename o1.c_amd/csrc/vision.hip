@@ -89,13 +89,6 @@ __global__ void __launch_bounds__(256) v_layernorm_kernel(const uint16_t *__rest
     }
 }
 
-__device__ __forceinline__ float gelu_tanh_f(float v) {
-    return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
-}
-__device__ __forceinline__ float gelu_erf_f(float v) {
-    return 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
-}
-
 // In place over [rows, ld] with `cols` live columns; columns [cols, ld)
 // are set to zero (the padded K of the following GEMM). ld, cols % 8 == 0.
 template <bool TANH>
