@@ -110,9 +110,8 @@ struct FaArgs {
     const uint16_t *k;     // [B,Hkv,S,D]
     const uint16_t *vt;    // [B,Hkv,D,S_pad] (perm16 columns)
     const uint16_t *mask;  // optional [S,S] additive bf16
-    const uint32_t *mask_bits;   // FA_DENSE, may be null: see fa_mask_bits_kernel
     uint16_t *out;         // seq-major [B,S,Hq*D] or head-major [B,Hq,S,D]
-    int batch, S, S_pad, Hq, Hkv;
+    int S, S_pad, Hq, Hkv;
     int ar_len;            // rows < ar_len: causal
     int q_row_begin;       // first query row of the launch (its q tiles start here)
     int q_row_end;         // only rows < q_row_end are computed/written
@@ -127,8 +126,12 @@ struct FaArgs {
     // chunks are the units of the causal rows [0, ar_len), the units before
     // them cover rows [q_row_begin, q_row_end), which see every key
     int n_whole, split, n_chunks;
-    FaRows full, causal;   // flash_pp16_kernel: row tiling of the two kinds of units
     float *part;           // [n_chunks][FA_BQ][FA_D] O, then [..][FA_BQ] (m, l)
+    // from here on not read by the plain kernels: a further cache line of
+    // arguments costs a block ~0.5 us at its start
+    int batch;
+    FaRows full, causal;   // flash_pp16_kernel: row tiling of the two kinds of units
+    const uint32_t *mask_bits;   // FA_DENSE, may be null: see fa_mask_bits_kernel
 };
 
 // 16-byte buffer load straight to LDS against a wave-uniform descriptor
@@ -495,7 +498,9 @@ __device__ __forceinline__ int2 fa_unit_row(const FaArgs &a, const FaUnit &u, in
     return make_int2(u.qbase + i % u.left, u.hk * group + u.g0 + k);
 }
 
-// MODE FA_PLAIN: S % 64 == 0, every row sees every key. FA_CAUSAL: any S, and
+// MODE FA_PLAIN: S % 64 == 0, every row sees every key, tiles of every head by
+// themselves (the row bookkeeping of the other modes costs it 1-7 %, more than
+// sharing left-over rows gives). FA_CAUSAL: any S, and
 // the units past the chunks are causal rows. FA_DENSE: any S, an additive mask
 // (and the causal test per element when ar_len > 0 comes with it).
 enum { FA_PLAIN = 0, FA_CAUSAL = 1, FA_DENSE = 2 };
@@ -509,6 +514,14 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     const int grp = wave >> 2;
     const int l16 = lane & 15, g = lane >> 4;
 
+    // every kernel argument is in its register from here on: one wait for
+    // all of them, and no scalar load that may still be in flight in the loop,
+    // which would make the compiler drain all LDS reads (lgkmcnt(0)) at the
+    // first fragment of every tile (1.5 % of the kernel)
+    asm volatile("" ::"s"(a.part), "s"(a.out), "s"(a.n_chunks), "s"(a.q_row_end), "s"(a.out_rows),
+                 "s"(a.out_seq_major), "s"(a.Hq), "s"(a.Hkv), "s"(a.scale_log2), "s"(a.q), "s"(a.k), "s"(a.vt), "s"(a.S),
+                 "s"(a.S_pad), "s"(a.n_whole), "s"(a.split), "s"(a.q_row_begin));
+    if constexpr (MODE != FA_PLAIN) asm volatile("" ::"s"(a.ar_len), "s"(a.inv_scale), "s"(a.mask));
     int lin = blockIdx.x, chunk = -1, item = 0;
     bool causal_unit = false;
     if (MODE == FA_CAUSAL && lin >= a.n_whole + a.n_chunks) {
@@ -521,28 +534,44 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     } else {
         lin = fa_xcd_remap(lin, a.n_whole);
     }
-    // (by value: a selected pointer into the arguments would be read with
-    // vector loads and make everything below per-lane)
-    FaRows rows = a.full;
-    if (MODE == FA_CAUSAL && causal_unit) rows = a.causal;
-    FaUnit un = fa_unit(a, rows, a.batch, lin);
-    un.b = __builtin_amdgcn_readfirstlane(un.b);
-    un.hk = __builtin_amdgcn_readfirstlane(un.hk);
-    un.qbase = __builtin_amdgcn_readfirstlane(un.qbase);
-    un.g0 = __builtin_amdgcn_readfirstlane(un.g0);
-    un.left = __builtin_amdgcn_readfirstlane(un.left);
-    const int b = un.b, hk = un.hk;
-
-    const int qbase = un.qbase;
-    const int q0 = qbase + (un.left ? 0 : wave * 32);   // lowest row of this wave
-    int2 rh[2];   // this lane's two query rows and their heads
-    rh[0] = fa_unit_row(a, un, wave * 32 + l16);
-    rh[1] = fa_unit_row(a, un, wave * 32 + 16 + l16);
-    const int my_q[2] = {rh[0].x, rh[1].x};
-    int kv_end = a.S;
-    if (MODE != FA_PLAIN && qbase < a.ar_len) {
-        const int last_row = qbase + (un.left ? un.left : BQ) - 1;
-        if (last_row < a.ar_len) kv_end = last_row + 1;
+    int b, hk, qbase, q0, kv_end = a.S;
+    int my_q[2], my_h[2];   // this lane's two query rows and their heads
+    if constexpr (MODE == FA_PLAIN) {
+        const int nqt = (a.q_row_end - a.q_row_begin + BQ - 1) / BQ, group = a.Hq / a.Hkv;
+        const int gq = lin % group; lin /= group;
+        const int qt = lin % nqt; lin /= nqt;
+        hk = lin % a.Hkv;
+        b = lin / a.Hkv;
+        qbase = a.q_row_begin + qt * BQ;
+        q0 = qbase + wave * 32;
+        my_q[0] = q0 + l16;
+        my_q[1] = q0 + 16 + l16;
+        my_h[0] = my_h[1] = hk * group + gq;
+    } else {
+        // (by value: a selected pointer into the arguments would be read with
+        // vector loads and make everything below per-lane)
+        FaRows rows = a.full;
+        if (MODE == FA_CAUSAL && causal_unit) rows = a.causal;
+        FaUnit un = fa_unit(a, rows, a.batch, lin);
+        un.b = __builtin_amdgcn_readfirstlane(un.b);
+        un.hk = __builtin_amdgcn_readfirstlane(un.hk);
+        un.qbase = __builtin_amdgcn_readfirstlane(un.qbase);
+        un.g0 = __builtin_amdgcn_readfirstlane(un.g0);
+        un.left = __builtin_amdgcn_readfirstlane(un.left);
+        b = un.b;
+        hk = un.hk;
+        qbase = un.qbase;
+        q0 = qbase + (un.left ? 0 : wave * 32);   // lowest row of this wave
+#pragma unroll
+        for (int qq = 0; qq < 2; qq++) {
+            const int2 rh = fa_unit_row(a, un, wave * 32 + qq * 16 + l16);
+            my_q[qq] = rh.x;
+            my_h[qq] = rh.y;
+        }
+        if (qbase < a.ar_len) {
+            const int last_row = qbase + (un.left ? un.left : BQ) - 1;
+            if (last_row < a.ar_len) kv_end = last_row + 1;
+        }
     }
     int t_begin = 0, t_end = (kv_end + FA_BK - 1) / FA_BK;
     if (chunk >= 0) {
@@ -555,7 +584,7 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     bf16x8_t qf[2][4];
 #pragma unroll
     for (int qq = 0; qq < 2; qq++) {
-        const uint16_t *qrow = a.q + (((size_t)b * a.Hq + rh[qq].y) * a.S + min(my_q[qq], a.S - 1)) * FA_D;
+        const uint16_t *qrow = a.q + (((size_t)b * a.Hq + my_h[qq]) * a.S + min(my_q[qq], a.S - 1)) * FA_D;
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) qf[qq][ks] = *(const bf16x8_t *)(qrow + ks * 32 + g * 8);
     }
@@ -763,13 +792,16 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
                     for (int e = 0; e < 4; e++) s[qq][u][e] -= INFINITY;
             }
             if (dead_keys) {
-                asm volatile("");   // a branch, not 32 selects in every tile
+                // a branch, not 32 selects in every tile, and its key
+                // indexes are formed inside it
+                int kvb = kv0;
+                asm volatile("" : "+s"(kvb));
                 const int mq = my_q[qq];
 #pragma unroll
                 for (int u = 0; u < 4; u++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const int kv = kv0 + fa16_key(u, g * 4 + e);
+                        const int kv = kvb + fa16_key(u, g * 4 + e);
                         const bool dead = kv >= a.S || (mq < a.ar_len && kv > mq);
                         const float v = dead ? -INFINITY : s[qq][u][e];
                         s[qq][u][e] = v;
@@ -814,11 +846,6 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         if (issued) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         else fa_wait_vm0();
     };
-    {
-        float *part = a.part;
-        uint16_t *outp = a.out;
-        asm volatile("" ::"s"(part), "s"(outp));
-    }
     // the barrier sequence of the phases above (2T + 3 barriers per wave)
     issue(t_begin);
     if (t_begin + 1 < t_end) {
@@ -874,9 +901,9 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
             const float inv = 1.0f / l_tot;
             uint16_t *dst;
             if (a.out_seq_major)
-                dst = a.out + (((size_t)b * a.out_rows + my_q[qq]) * a.Hq + rh[qq].y) * FA_D;
+                dst = a.out + (((size_t)b * a.out_rows + my_q[qq]) * a.Hq + my_h[qq]) * FA_D;
             else
-                dst = a.out + (((size_t)b * a.Hq + rh[qq].y) * a.out_rows + my_q[qq]) * FA_D;
+                dst = a.out + (((size_t)b * a.Hq + my_h[qq]) * a.out_rows + my_q[qq]) * FA_D;
 #pragma unroll
             for (int w = 0; w < 4; w++) {
                 const f32x4_t x0 = o[qq][w * 2], x1 = o[qq][w * 2 + 1];
@@ -936,7 +963,8 @@ static void fa_vt_launch(const void *v, void *vt, int bh, int S, hipStream_t st)
 // Merges the tail units' key-chunk partials: O = sum_i w_i O_i / sum_i w_i l_i
 // with w_i = 2^((m_i - max_j m_j) * scale_log2). One thread per (row, 8
 // consecutive d): two 16-byte partial loads per chunk, one 16-byte store.
-template <int BQ>
+// SHARED: units of fa_unit's numbering (left-over rows share units).
+template <int BQ, bool SHARED>
 __global__ __launch_bounds__(256) void fa_merge_kernel(FaArgs a, int n_tail) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     const int d0 = (idx % (FA_D / 8)) * 8, row = (idx / (FA_D / 8)) % BQ, tu = idx / (FA_D / 8 * BQ);
@@ -957,7 +985,7 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaArgs a, int n_tail) {
         for (int e = 0; e < 8; e++) acc[e] = fmaf(w, pv[e], acc[e]);
     }
     int b, hq, my_q;
-    if constexpr (BQ == 256) {
+    if constexpr (SHARED) {
         const FaUnit un = fa_unit(a, a.full, a.batch, a.n_whole + tu);
         const int2 rh = fa_unit_row(a, un, row);
         b = un.b;
@@ -1084,8 +1112,9 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     const int BQ = nwv * 32;
     const int group = hq / hkv;
     int units, n_causal = 0;
+    const bool plain = !mask && ar_len == 0 && seq % FA_BK == 0;
     a.full = a.causal = {};
-    if (pp) {
+    if (pp && !plain) {
         if (prefix) a.q_row_begin = ar_len;   // the causal rows are units of their own
         auto rows_of = [&](int row0, int rows, bool share) {
             FaRows r = {row0, rows / BQ, rows % BQ, 1};
@@ -1144,7 +1173,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
         // the ping-pong form: +2.5-4.7 % at S = 4352-16640 over 8-wave
         // blocks in lockstep
         if (mask) flash_pp16_kernel<FA_DENSE><<<grid, 512, 0, st>>>(a);
-        else if (ar_len > 0 || seq % FA_BK) flash_pp16_kernel<FA_CAUSAL><<<grid, 512, 0, st>>>(a);
+        else if (!plain) flash_pp16_kernel<FA_CAUSAL><<<grid, 512, 0, st>>>(a);
         else flash_pp16_kernel<FA_PLAIN><<<grid, 512, 0, st>>>(a);
     } else {
         if (mask || ar_len > 0 || seq % FA_BK) flash_fwd_kernel<true, 4><<<grid, 256, 0, st>>>(a);
@@ -1152,8 +1181,9 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     }
     if (n_tail) {
         dim3 gm((unsigned)hd_cdiv((int64_t)n_tail * BQ * (FA_D / 8), 256));
-        if (pp) fa_merge_kernel<256><<<gm, 256, 0, st>>>(a, n_tail);
-        else fa_merge_kernel<128><<<gm, 256, 0, st>>>(a, n_tail);
+        if (!pp) fa_merge_kernel<128, false><<<gm, 256, 0, st>>>(a, n_tail);
+        else if (plain) fa_merge_kernel<256, false><<<gm, 256, 0, st>>>(a, n_tail);
+        else fa_merge_kernel<256, true><<<gm, 256, 0, st>>>(a, n_tail);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
