@@ -10,9 +10,8 @@
  *
  *   pixel_values [n, 1536] bf16 (patchified, processor layout)
  *     -> patch embed GEMM + interpolated position embedding  [n, 1152]
- *     -> 27 blocks: LayerNorm, qkv, 2-D rotary, full attention (the flash
- *        kernel at head_dim 128 over zero-padded heads), proj, LayerNorm,
- *        fc1, GELU(tanh), fc2                                  [n, 1152]
+ *     -> 27 blocks: LayerNorm, qkv, 2-D rotary, full attention, proj,
+ *        LayerNorm, fc1, GELU(tanh), fc2                                  [n, 1152]
  *     -> merger: LayerNorm(1152), 4-row view, fc1, GELU(erf), fc2 -> [m, 4096]
  *     -> deepstack mergers after blocks 8/16/24 (LayerNorm over 4608)
  *
@@ -47,8 +46,8 @@ extern "C" {
 /* vision.h:51-69: block-0 snapshot slots. This build captures HD_B0_INPUT,
  * HD_B0_NORM1, HD_B0_QKV, HD_B0_ATTN_MERGED, HD_B0_PROJ, HD_B0_ATTN_RESID,
  * HD_B0_NORM2, HD_B0_FC2 and HD_B0_OUTPUT; the head-major q/k/v slots hold
- * the zero-padded [16, n, 128] layout the flash kernel reads, and HD_B0_FC1
- * the GELU input at a 4352-column row stride. */
+ * [16, n, 128] rows zero past column 72, and HD_B0_FC1 the rows fc2 reads, at a
+ * 4352-column row stride with zeros past column 4304. */
 enum {
     HD_B0_INPUT = 0,
     HD_B0_NORM1,
@@ -117,11 +116,12 @@ typedef struct {
  *   h_a        [n,1152]  residual stream (block input / output)
  *   attn_resid [n,1152]  residual after attention
  *   ln1        [n,1152]  LayerNorm output, later the merged attention rows
- *   qkv        [n,3456]  qkv projection, later the flash output [n,16*128]
- *   q, k, v    [16,n+128,128] zero-padded head-major operands
- *   scores     [16,128,round_up(n,64)] V^T for the flash kernel
- *   fc1        [n,4352]  fc1 / GELU rows (zero columns 4304..4351)
- *   fc2        [1152,4352] the current block's fc2 weight, zero-padded
+ *   qkv        [n,3456]  qkv projection
+ *   q, k       [16,n,72] head-major operands after the rotary
+ *   scores     [16,72,round_up(n,64)] V^T for the attention kernel
+ *   fc1        [n,4352]  fc1 rows after the GELU, 4304 columns of each (mergers:
+ *                        [n/4,4608])
+ *   fc2        [1152,4352] the current block's fc2 weight, 4304 columns of each row
  *   cosf, sinf [n,72]    fp32 rotary tables */
 typedef struct {
     int64_t patch_out, pos_emb, rot, h_a, h_b, ln1, attn_resid, ln2, fc2, mlp_resid, q, k, v, qr,

@@ -916,6 +916,211 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
     if (!grp) fa_barrier();
 }
 
+// ---------------------------------------------------------------------------
+// Full attention at head_dim 72 (the vision tower), operands unpadded: q, k
+// [BH, S, 72], vt [BH, 72, S_pad] (perm16 columns, zero past S), out seq-major
+// [B, S, heads * 72]. The 4-wave kernel's scheme (32 queries per wave, 32x32x16
+// MFMAs, S^T then O^T) with 5 k-steps of 16 for 72 + 8 zero dimensions and 3
+// row tiles of 32 for 72 + 24 zero rows: 22 MFMAs per 64 keys, where heads
+// padded to 128 take 32, and half their memory. K rows stand 176 bytes apart in
+// LDS (11 16-byte chunks, the last two zero: 16 rows of one chunk hit 16 bank
+// groups); chunks and rows past 72 are loads past the records, which read zero.
+// KS waves share each 32 queries, every KS-th key tile each, and merge at the
+// end: the tower's 576 rows are 80 blocks of 128 queries, so with KS = 2 its
+// 144 blocks of 64 take half the key tiles each on otherwise idle CUs.
+// @V72@
+// ---------------------------------------------------------------------------
+struct FaV72Args {
+    const uint16_t *q, *k, *vt;
+    uint16_t *out;
+    int S, S_pad, heads;
+    float scale_log2;
+};
+template <int KS>
+__global__ __launch_bounds__(256, KS == 1 ? 3 : 2) void flash_v72_kernel(FaV72Args a) {
+    constexpr int D = 72, KP = 88, VR = 96, BK = 64, QG = 4 / KS, KT = BK * KP, VT = VR * BK;
+    constexpr int KI = BK * KP / 8 / 64, VI = VR * BK / 8 / 64;   // load instructions of a tile: 11 and 12
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[2 * KS * (KT + VT)];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave / QG, qw = wave % QG;
+    const int bh = blockIdx.y, q0 = blockIdx.x * QG * 32 + qw * 32, my_q = q0 + l32;
+    const int nt = (a.S + BK - 1) / BK, nit = (nt + KS - 1) / KS;
+
+    const uint16_t *qrow = a.q + ((size_t)bh * a.S + min(my_q, a.S - 1)) * D;
+    bf16x8_t qf[5];
+#pragma unroll
+    for (int ks = 0; ks < 5; ks++) {
+        const int d = ks * 16 + h * 8;
+        qf[ks] = __builtin_bit_cast(bf16x8_t, (u32x4_t){0, 0, 0, 0});
+        if (d < D) qf[ks] = *(const bf16x8_t *)(qrow + d);
+    }
+    const uint16_t *kbase = a.k + (size_t)bh * a.S * D, *vbase = a.vt + (size_t)bh * D * a.S_pad;
+    const int kbytes = a.S * D * 2, vbytes = D * a.S_pad * 2;
+    // a tile's loads are spread over the QG waves of its key group
+    constexpr int KPW = (KI + QG - 1) / QG, VPW = (VI + QG - 1) / QG;
+    uint32_t k_vo[KPW], v_vo[VPW];
+#pragma unroll
+    for (int i = 0; i < KPW; i++) {
+        const int c = (qw * KPW + i) * 64 + lane, row = c / (KP / 8), ch = c % (KP / 8);
+        k_vo[i] = ch < D / 8 ? (uint32_t)(row * D + ch * 8) * 2 : 0x80000000u;
+    }
+#pragma unroll
+    for (int i = 0; i < VPW; i++) {
+        const int row = (qw * VPW + i) * 8 + (lane >> 3);
+        v_vo[i] = row < D ? (uint32_t)(row * a.S_pad + ((lane & 7) ^ ((row >> 1) & 7)) * 8) * 2 : 0x80000000u;
+    }
+    auto issue = [&](int it, int buf) {
+        const int t = it * KS + kg;
+        // a key group without a tile in the last round reads zeros; the scalar
+        // offset stays inside the records
+        const bool live = t < nt;
+        uint16_t *Ks = smem + (buf * KS + kg) * (KT + VT), *Vs = Ks + KT;
+#pragma unroll
+        for (int i = 0; i < KPW; i++)
+            if (qw * KPW + i < KI)
+                fa_buf_load16(kbase, kbytes, live ? k_vo[i] : 0x80000000u, live ? (uint32_t)t * BK * D * 2 : 0u,
+                              (HD_LDS void *)(Ks + (qw * KPW + i) * 512));
+#pragma unroll
+        for (int i = 0; i < VPW; i++)
+            if (qw * VPW + i < VI)
+                fa_buf_load16(vbase, vbytes, live ? v_vo[i] : 0x80000000u, live ? (uint32_t)t * BK * 2 : 0u,
+                              (HD_LDS void *)(Vs + (qw * VPW + i) * 512));
+    };
+    f32x16_t o[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[i][r] = 0.f;
+    float m_run = -1e30f, l_run = 0.f;
+
+    issue(0, 0);
+    fa_wait_vm0();
+    __syncthreads();
+    for (int it = 0; it < nit; it++) {
+        const int buf = it & 1, t = it * KS + kg, kv0 = t * BK;
+        if (it + 1 < nit) issue(it + 1, buf ^ 1);
+        if (t < nt) {
+            const uint16_t *Ks = smem + (buf * KS + kg) * (KT + VT), *Vs = Ks + KT;
+            f32x16_t s[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) s[j][r] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < 5; ks++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const bf16x8_t kf = *(const bf16x8_t *)(Ks + (j * 32 + l32) * KP + (ks * 2 + h) * 8);
+                    s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[j], 0, 0, 0);
+                }
+            float mt = -INFINITY;
+            if (kv0 + BK > a.S) {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int kv = kv0 + j * 32 + (r >> 2) * 8 + h * 4 + (r & 3);
+                        s[j][r] = kv < a.S ? s[j][r] : -INFINITY;
+                        mt = fmaxf(mt, s[j][r]);
+                    }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[j][r]);
+            }
+            mt = xor32_max(mt);
+            if (__builtin_amdgcn_ballot_w64((mt - m_run) * a.scale_log2 > FA_TAU)) {
+                const float m_new = fmaxf(m_run, mt);
+                const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * a.scale_log2);
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[i][r] *= alpha;
+            }
+            const float mc = -m_run * a.scale_log2;
+            bf16x8_t pf[4];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    bf16x8_t pv;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const float p = __builtin_amdgcn_exp2f(fmaf(s[j][hh * 8 + e], a.scale_log2, mc));
+                        l_run += p;
+                        pv[e] = (__bf16)p;
+                    }
+                    pf[j * 2 + hh] = pv;
+                }
+#pragma unroll
+            for (int st = 0; st < 4; st++)
+#pragma unroll
+                for (int dt = 0; dt < 3; dt++) {
+                    const int row = dt * 32 + l32;
+                    const bf16x8_t vf = *(const bf16x8_t *)(Vs + row * BK + ((st * 2 + h) ^ ((row >> 1) & 7)) * 8);
+                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[st], o[dt], 0, 0, 0);
+                }
+        }
+        fa_wait_vm0();
+        __syncthreads();
+    }
+    float l_tot = xor32_sum(l_run);
+    if constexpr (KS == 2) {
+        // key group 1 hands its sums over (the tile buffers are free), group 0
+        // merges them relative to the larger of the two running maxima
+        float *x = (float *)smem + qw * 50 * 64 + lane;   // [50][64] per 32 queries
+        if (kg == 1) {
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) x[(i * 16 + r) * 64] = o[i][r];
+            x[48 * 64] = m_run;
+            x[49 * 64] = l_tot;
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        const float m1 = x[48 * 64], m = fmaxf(m_run, m1);
+        const float w0 = __builtin_amdgcn_exp2f((m_run - m) * a.scale_log2);
+        const float w1 = __builtin_amdgcn_exp2f((m1 - m) * a.scale_log2);
+        l_tot = l_tot * w0 + x[49 * 64] * w1;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[i][r] = o[i][r] * w0 + x[(i * 16 + r) * 64] * w1;
+    }
+    if (my_q >= a.S) return;
+    const float inv = 1.0f / l_tot;
+    // lane (query, h) holds dimensions dt*32 + g*8 + h*4 .. +3: 8-byte stores,
+    // two lanes fill 16 bytes; dimensions past 72 are dropped
+    uint16_t *dst = a.out + (((size_t)(bh / a.heads) * a.S + my_q) * a.heads + bh % a.heads) * D;
+#pragma unroll
+    for (int dt = 0; dt < 3; dt++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int d = dt * 32 + g * 8 + h * 4;
+            if (dt * 32 + g * 8 < D)
+                *(u32x2_t *)(dst + d) = (u32x2_t){pack_bf2(o[dt][g * 4] * inv, o[dt][g * 4 + 1] * inv),
+                                                  pack_bf2(o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv)};
+        }
+}
+
+int hd_flash_v72(const void *q, const void *k, const void *vt, void *out, int batch, int heads, int seq,
+                 float scale) {
+    FaV72Args a = {(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)vt, (uint16_t *)out, seq,
+                   (int)fa_spad(seq), heads, scale * 1.44269504088896341f};
+    if (batch * heads * ((seq + 63) / 64) <= 256)
+        flash_v72_kernel<2><<<dim3((seq + 63) / 64, batch * heads), 256, 0, hd_stream()>>>(a);
+    else
+        flash_v72_kernel<1><<<dim3((seq + 127) / 128, batch * heads), 256, 0, hd_stream()>>>(a);
+    hd_check_launch("flash_v72");
+    return 0;
+}
+
+// V [BH, S, D] -> vt [BH, D, S_pad] with perm16 columns and zero padding.
 // One block per 64-key tile: rows in through LDS (16-byte loads when V is
 // 16-byte aligned), 16-byte stores of 8 storage columns per dimension. HBM
 // bound in principle (4 B per element); at S = 2371, 8 heads it is one short

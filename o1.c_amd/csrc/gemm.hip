@@ -26,6 +26,7 @@
 #include "hd_common.hpp"
 #include "../../include/hd_hip.h"
 #include "../../include/hd_gemm.h"
+#include "../../include/hd_vision.h"
 
 // GELU / GELU_ERF: bias, then the tanh / erf form on the bf16 sum
 enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_RES = 2, EPI_SWIGLU = 3, EPI_QKV = 4, EPI_GELU = 5, EPI_GELU_ERF = 6 };
@@ -40,6 +41,7 @@ struct GemmArgs {
     int M, N, K;             // N = output columns
     int ldc;
     int ntm, ntn;            // tile grid
+    int lda, ldb;            // operand row strides, K-group kernels only (0: K)
     // EPI_QKV: per-head q/k RMSNorm + rotary into head-major q, k and the
     // flash V^T layout (columns: q heads, k heads, v heads of 128)
     const uint16_t *qn_w, *kn_w;   // [128] norm gains
@@ -63,6 +65,13 @@ struct GemmArgs {
 // ~10 VALU instructions per output and most of the per-tile epilogue time.
 __device__ __forceinline__ float silu_rcp(float g) {
     return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+}
+
+// GELU of two packed bf16 values where the epilogue has one.
+template <int EPI> __device__ __forceinline__ uint32_t epi_gelu(uint32_t v) {
+    if (EPI == EPI_GELU) return pack_bf2(gelu_tanh_f(lo_bf(v)), gelu_tanh_f(hi_bf(v)));
+    if (EPI == EPI_GELU_ERF) return pack_bf2(gelu_erf_f(lo_bf(v)), gelu_erf_f(hi_bf(v)));
+    return v;
 }
 
 __device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -671,11 +680,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, OCC) void gemm_ms_kernel(GemmArgs g
         const int m = gm0 + r, n = gn0 + cc;
         if (m < g.M && n < g.N) {
             u32x4_t v = *(const u32x4_t *)(stg + r * LDW + cc);
-            if (EPI == EPI_BIAS || EPI == EPI_RES) {
-                u32x4_t o = EPI == EPI_BIAS ? *(const u32x4_t *)(g.bias + n) : resv[EPI == EPI_RES ? r0 / RPIO : 0];
+            if (EPI != EPI_NONE && EPI != EPI_SWIGLU) {
+                u32x4_t o = EPI != EPI_RES ? *(const u32x4_t *)(g.bias + n) : resv[EPI == EPI_RES ? r0 / RPIO : 0];
 #pragma unroll
                 for (int e = 0; e < 4; e++)
-                    v[e] = pack_bf2(lo_bf(v[e]) + lo_bf(o[e]), hi_bf(v[e]) + hi_bf(o[e]));
+                    v[e] = epi_gelu<EPI>(pack_bf2(lo_bf(v[e]) + lo_bf(o[e]), hi_bf(v[e]) + hi_bf(o[e])));
             }
             *(u32x4_t *)(g.C + (size_t)m * g.ldc + n) = v;
         }
@@ -748,14 +757,15 @@ __global__ __launch_bounds__(512, OCC) void gemm_kg_kernel(GemmArgs g) {
     const int brows = EPI == EPI_SWIGLU ? g.N
                                         : (bsg == 0 ? g.seg_end[0] : (bsg == 1 ? g.seg_end[1] : g.seg_end[2])) - bbase;
     const void *bp0 = bsg == 0 ? g.B[0] : (bsg == 1 ? g.B[1] : g.B[2]), *bp1 = g.B[1];
-    const int nb_a = (int)((size_t)g.M * g.K * 2), nb_b = (int)((size_t)brows * g.K * 2);
+    const uint32_t lda = g.lda ? g.lda : g.K, ldb = g.ldb ? g.ldb : g.K;
+    const int nb_a = (int)(((size_t)(g.M - 1) * lda + g.K) * 2), nb_b = (int)(((size_t)(brows - 1) * ldb + g.K) * 2);
     uint32_t a_vo[AI], b_vo[BI];
     int b_up[BI], a_kc[AI], b_kc[BI];
 #pragma unroll
     for (int i = 0; i < AI; i++) {
         const int r = (wave * AI + i) * 8 + sub;
         a_kc[i] = (cl ^ ms_swz<8>(r)) * 8;
-        a_vo[i] = m0 + r < g.M ? ((uint32_t)(m0 + r) * (uint32_t)g.K + a_kc[i]) * 2 : 0x80000000u;
+        a_vo[i] = m0 + r < g.M ? ((uint32_t)(m0 + r) * lda + a_kc[i]) * 2 : 0x80000000u;
     }
 #pragma unroll
     for (int i = 0; i < BI; i++) {
@@ -768,7 +778,7 @@ __global__ __launch_bounds__(512, OCC) void gemm_kg_kernel(GemmArgs g) {
             b_up[i] = __builtin_amdgcn_readfirstlane(((wave * BI + i) * 8) % WTN >= WO);
         }
         b_kc[i] = (cl ^ ms_swz<8>(r)) * 8;
-        b_vo[i] = n < brows ? ((uint32_t)n * (uint32_t)g.K + b_kc[i]) * 2 : 0x80000000u;
+        b_vo[i] = n < brows ? ((uint32_t)n * ldb + b_kc[i]) * 2 : 0x80000000u;
     }
     auto issue = [&](int kt) {
         uint16_t *As = smem + (kt % NS) * STAGE, *Bs = As + BM * BK;
@@ -893,12 +903,8 @@ __global__ __launch_bounds__(512, OCC) void gemm_kg_kernel(GemmArgs g) {
             if (EPI != EPI_NONE && EPI != EPI_SWIGLU) {
                 const u32x4_t o = *(const u32x4_t *)(EPI == EPI_RES ? g.res + (size_t)m * g.ldc + n : g.bias + n);
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = pack_bf2(lo_bf(v[e]) + lo_bf(o[e]), hi_bf(v[e]) + hi_bf(o[e]));
-                if (EPI == EPI_GELU || EPI == EPI_GELU_ERF)
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        v[e] = EPI == EPI_GELU ? pack_bf2(gelu_tanh_f(lo_bf(v[e])), gelu_tanh_f(hi_bf(v[e])))
-                                               : pack_bf2(gelu_erf_f(lo_bf(v[e])), gelu_erf_f(hi_bf(v[e])));
+                for (int e = 0; e < 4; e++)
+                    v[e] = epi_gelu<EPI>(pack_bf2(lo_bf(v[e]) + lo_bf(o[e]), hi_bf(v[e]) + hi_bf(o[e])));
             }
             *(u32x4_t *)(g.C + (size_t)m * g.ldc + n) = v;
         }
@@ -1013,12 +1019,12 @@ __global__ __launch_bounds__(512, 1) void gemm_skinny_kernel(GemmArgs g) {
             }
             if (m < g.M && n < g.N) {
                 u32x2_t pk = {pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3])};
-                if (EPI == EPI_BIAS || EPI == EPI_RES) {
-                    const uint16_t *o = EPI == EPI_BIAS ? g.bias + n : g.res + (size_t)m * g.ldc + n;
+                if (EPI != EPI_NONE && EPI != EPI_SWIGLU) {
+                    const uint16_t *o = EPI != EPI_RES ? g.bias + n : g.res + (size_t)m * g.ldc + n;
                     const u32x2_t ov = *(const u32x2_t *)o;
 #pragma unroll
                     for (int e = 0; e < 2; e++)
-                        pk[e] = pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e]));
+                        pk[e] = epi_gelu<EPI>(pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e])));
                 }
                 *(u32x2_t *)(g.C + (size_t)m * g.ldc + n) = pk;
             }
@@ -1138,11 +1144,8 @@ __global__ void gemm_tail_merge_kernel(GemmArgs g, int n_tail) {
         const uint16_t *o = EPI == EPI_RES ? g.res + (size_t)m * g.ldc + n : g.bias + n;
         const u32x2_t ov = *(const u32x2_t *)o;
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            pk[e] = pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e]));
-            if (EPI == EPI_GELU) pk[e] = pack_bf2(gelu_tanh_f(lo_bf(pk[e])), gelu_tanh_f(hi_bf(pk[e])));
-            if (EPI == EPI_GELU_ERF) pk[e] = pack_bf2(gelu_erf_f(lo_bf(pk[e])), gelu_erf_f(hi_bf(pk[e])));
-        }
+        for (int e = 0; e < 2; e++)
+            pk[e] = epi_gelu<EPI>(pack_bf2(lo_bf(pk[e]) + lo_bf(ov[e]), hi_bf(pk[e]) + hi_bf(ov[e])));
     }
     *(u32x2_t *)(g.C + (size_t)m * g.ldc + n) = pk;
 }
@@ -1315,7 +1318,7 @@ static void launch_kg(GemmArgs &g, int P, void *ws) {
 // A split adds the merge launch and its partials, written and read at 8 TB/s
 // (L2 and the cache behind it hold most). Tiles this small re-read the
 // operands: once these do not fit the L2s (32 MB in all) the re-reads are
-// served at 12-18 TB/s.
+// served at 16-18 TB/s.
 struct SmallPick {
     int fam, P;   // fam 0..4: kKg; 5 old 128x128, 6 192x256, 7 256x256
     double us;
@@ -1348,7 +1351,7 @@ static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t 
                                                  : u <= 2 ? 1.4 + 0.3 * u : 1.1 * u;
             double t = 3.0 + rounds * (k.fixed + ((nk + P - 1) / P) * k.us * (swiglu || K > 8192 ? 1.15 : 1.0));
             const double reread = tiles * (double)(k.bm + k.bn) * K * 2;
-            if (foot > 32e6 && reread / 12e6 > t) t = reread / 12e6;
+            if (foot > 32e6 && reread / 16e6 > t) t = reread / 16e6;
             offer(f, P, t + (P > 1 ? merge_us(tiles, P, k.bm, k.bn) : 0.0));
         }
     }
@@ -1435,7 +1438,7 @@ static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr,
         if (launch) launch_ms<256, 256, 64, 2, 2, 4, EPI, 3, 1, 0, 16>(g, ws, ws_bytes);
         return split256 ? "bf16_256x256x64_w2x4_m16_ring_tailsplit" : "bf16_256x256x64_w2x4_m16_ring";
     }
-    if (t256 <= 512)
+    if (t256 <= 512 || g.K % 64)   // only the K-group kernels take K % 64 != 0
         return launch_small<EPI>(g, pick_small(g.M, g.N, g.K, EPI == EPI_SWIGLU, false, ws ? ws_bytes : 0), launch, ws,
                                  ws ? ws_bytes : 0);
     if (c128 < c256 && c128 < c192) {
@@ -1458,8 +1461,16 @@ static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr,
     return split256 ? "bf16_256x256x64_w2x4_m16_ring_buf_tailsplit" : "bf16_256x256x64_w2x4_m16_ring_buf";
 }
 
-static bool mfma_ok(const void *x, const void *y, int N, int K) {
-    return K % 64 == 0 && N % 8 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)y % 16 == 0);
+static bool mfma_ok(const void *x, const void *y, int N, int K, int kmod = 64) {
+    return K % kmod == 0 && N % 8 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)y % 16 == 0);
+}
+
+// hd_linear / hd_linear_ws: K in whole 16-byte chunks on the K-group kernels
+// (32-bit byte offsets, 16-byte rows); other shapes run the reference kernel.
+static bool linear_ok(const void *x, const void *w, const void *y, int M, int N, int K) {
+    if (K % 64 == 0) return mfma_ok(x, y, N, K);
+    return mfma_ok(x, y, N, K, 8) && (uintptr_t)w % 16 == 0 && (size_t)(M + 256) * K * 2 < ((size_t)1 << 31) &&
+           (size_t)(N + 256) * K * 2 < ((size_t)1 << 31);
 }
 
 static void gemm_launch(int epi, GemmArgs &g, void *ws = nullptr, int64_t ws_bytes = 0) {
@@ -1468,6 +1479,8 @@ static void gemm_launch(int epi, GemmArgs &g, void *ws = nullptr, int64_t ws_byt
     case EPI_BIAS: pick_and_launch<EPI_BIAS>(g, true, ws, ws_bytes); break;
     case EPI_RES: pick_and_launch<EPI_RES>(g, true, ws, ws_bytes); break;
     case EPI_SWIGLU: pick_and_launch<EPI_SWIGLU>(g, true, ws, ws_bytes); break;
+    case EPI_GELU: pick_and_launch<EPI_GELU>(g, true, ws, ws_bytes); break;
+    case EPI_GELU_ERF: pick_and_launch<EPI_GELU_ERF>(g, true, ws, ws_bytes); break;
     }
 }
 
@@ -1631,7 +1644,7 @@ extern "C" double hd_mfma_probe(const void *ops, int n_ops, int blocks, int iter
 extern "C" const char *hd_gemm_config_name(int M, int N, int K, int epi) {
     GemmArgs g = {};
     g.M = M; g.N = N; g.K = K;
-    if (K % 64 || N % 8) return "reference";
+    if (K % 8 || N % 8) return "reference";
     switch (epi) {
     case EPI_BIAS: return pick_and_launch<EPI_BIAS>(g, false);
     case EPI_RES: return pick_and_launch<EPI_RES>(g, false);
@@ -1666,7 +1679,7 @@ extern "C" void hd_linear(const void *x, const void *w, const void *bias, void *
         snprintf(hd_cuda_errbuf(), 512, "linear: transpose_w=0 unsupported");
         return;
     }
-    if (!g_use_production || !mfma_ok(x, y, N, K) || (bias && (uintptr_t)bias % 16)) {
+    if (!g_use_production || !linear_ok(x, w, y, M, N, K) || (bias && (uintptr_t)bias % 16)) {
         // reference backend: fp32 result + bias rounded once; production
         // rounding (two roundings) is kept by adding the bias separately.
         hd_linear_reference(x, w, nullptr, y, M, N, K, 1);
@@ -1688,9 +1701,53 @@ extern "C" void hd_linear(const void *x, const void *w, const void *bias, void *
     hd_check_launch("linear");
 }
 
+void hd_linear_gelu(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, bool erf,
+                    void *ws, int64_t ws_bytes, int ldc) {
+    if (!x || !w || !bias || !y || M <= 0 || N <= 0 || K <= 0 || !linear_ok(x, w, y, M, N, K) ||
+        ((uintptr_t)bias | (uintptr_t)ws) % 16 || (!g_use_production && ldc == N)) {
+        if (ldc != N) {
+            snprintf(hd_cuda_errbuf(), 512, "linear_gelu: bad args");
+            return;
+        }
+        hd_linear(x, w, bias, y, M, N, K, 1);
+        if (erf) hd_vision_gelu_exact(y, y, (size_t)M * N);
+        else hd_vision_gelu(y, y, (size_t)M * N);
+        return;
+    }
+    GemmArgs g = {};
+    g.A = (const uint16_t *)x;
+    g.B[0] = g.B[1] = g.B[2] = (const uint16_t *)w;
+    g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
+    g.C = (uint16_t *)y;
+    g.bias = (const uint16_t *)bias;
+    g.M = M; g.N = N; g.K = K; g.ldc = ldc;
+    gemm_launch(erf ? EPI_GELU_ERF : EPI_GELU, g, ws, ws ? ws_bytes : 0);
+    hd_check_launch("linear_gelu");
+}
+
+void hd_linear_strided(const void *x, int lda, const void *w, int ldb, const void *bias, void *y, int M, int N,
+                       int K, void *ws, int64_t ws_bytes) {
+    if (!x || !w || !bias || !y || M <= 0 || N <= 0 || K % 64 == 0 || lda < K || ldb < K || lda % 8 || ldb % 8 ||
+        !linear_ok(x, w, y, M, N, K) || ((uintptr_t)bias | (uintptr_t)ws) % 16 ||
+        ((size_t)M * lda | (size_t)N * ldb) >= ((size_t)1 << 30)) {
+        snprintf(hd_cuda_errbuf(), 512, "linear_strided: bad args");
+        return;
+    }
+    GemmArgs g = {};
+    g.A = (const uint16_t *)x;
+    g.B[0] = g.B[1] = g.B[2] = (const uint16_t *)w;
+    g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
+    g.C = (uint16_t *)y;
+    g.bias = (const uint16_t *)bias;
+    g.M = M; g.N = N; g.K = K; g.ldc = N;
+    g.lda = lda; g.ldb = ldb;
+    gemm_launch(EPI_BIAS, g, ws, ws ? ws_bytes : 0);
+    hd_check_launch("linear_strided");
+}
+
 extern "C" void hd_linear_ws(const void *x, const void *w, const void *bias, void *y, int M, int N,
                              int K, void *ws, int64_t ws_bytes) {
-    if (!x || !w || !y || M <= 0 || N <= 0 || K <= 0 || !mfma_ok(x, y, N, K) ||
+    if (!x || !w || !y || M <= 0 || N <= 0 || K <= 0 || !linear_ok(x, w, y, M, N, K) ||
         (bias && (uintptr_t)bias % 16) || (ws && (uintptr_t)ws % 16) || !g_use_production) {
         hd_linear(x, w, bias, y, M, N, K, 1);
         return;

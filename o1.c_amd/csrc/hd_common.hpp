@@ -16,6 +16,17 @@ int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *
                      const void *kn_w, const float *cs, void *q, void *k, void *vt, int batch, int seq,
                      int heads, int kv_heads, int hidden, float eps, void *ws, int64_t ws_bytes);
 
+// y = bf16(gelu(bf16(bf16(x . w^T) + bias))), tanh or erf form, rows of ldc (gemm.hip).
+void hd_linear_gelu(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, bool erf,
+                    void *ws, int64_t ws_bytes, int ldc);
+// hd_linear_ws over operand rows of lda and ldb elements, K % 8 == 0 but not K % 64 (gemm.hip).
+void hd_linear_strided(const void *x, int lda, const void *w, int ldb, const void *bias, void *y, int M, int N,
+                       int K, void *ws, int64_t ws_bytes);
+// Attention of the vision tower: q, k [batch * heads, seq, 72], vt [batch * heads, 72, round_up(seq, 64)]
+// in the flash key order, out [batch, seq, heads * 72] (attention.hip).
+int hd_flash_v72(const void *q, const void *k, const void *vt, void *out, int batch, int heads, int seq,
+                 float scale);
+
 // ---- bf16 <-> fp32 ------------------------------------------------------
 // bf16 payloads are uint16_t. fp32 -> bf16 uses gfx950's v_cvt_pk_bf16_f32,
 // IEEE round-to-nearest-even: for finite values the same bits as the
@@ -36,8 +47,12 @@ __device__ __forceinline__ float lo_bf(uint32_t w) { return __uint_as_float(w <<
 __device__ __forceinline__ float hi_bf(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
 
 // ---- GELU, tanh and erf forms (vision_kernels.cu) -----------------------
+// 0.5 (1 + tanh(u)) = 1 / (1 + e^-2u): no cancellation where tanh nears -1, and
+// the hardware exp and reciprocal (about 1 ulp each) instead of tanhf's ~50
+// instructions, which were half of a small fc1 GEMM's time as its epilogue.
 __device__ __forceinline__ float gelu_tanh_f(float v) {
-    return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+    const float u2 = 1.5957691216057308f * (v + 0.044715f * v * v * v);
+    return v * __builtin_amdgcn_rcpf(1.0f + __expf(-u2));
 }
 __device__ __forceinline__ float gelu_erf_f(float v) {
     return 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));

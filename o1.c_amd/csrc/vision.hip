@@ -19,9 +19,10 @@
 namespace {
 
 constexpr int kH = HD_VISION_HIDDEN, kNH = HD_VISION_HEADS, kD = HD_VISION_HEAD_DIM;
-constexpr int kI = HD_VISION_INTERMEDIATE, kIP = 4352;   // fc1 width padded to 64
+constexpr int kI = HD_VISION_INTERMEDIATE, kIP = 4352;   // fc1 width, and the row stride it is kept at (whole
+                                                         // 128-byte lines)
 constexpr int kO = HD_VISION_OUT_HIDDEN, kU = HD_VISION_MERGE_SIZE * HD_VISION_MERGE_SIZE;
-constexpr int kDP = 128;                                  // head_dim of the flash kernel
+constexpr int kDP = 128;                                  // head_dim of the q / k / v snapshots
 constexpr int kQKV = 3 * kH;
 constexpr int kNSide = 48;                                // sqrt(HD_VISION_NUM_POS)
 constexpr int kDsLayers[HD_VISION_NUM_DS] = HD_VISION_DS_LAYERS;
@@ -32,6 +33,34 @@ __device__ __forceinline__ float wsum(float v) {
     return v;
 }
 
+// A weight copied to rows of `ld` elements by spare blocks of another launch
+// (cols, ld % 8 == 0; nothing when src is null). fc2's rows of 4304 elements
+// start off the 128-byte lines, so every 64-deep K tile of a row touches two
+// lines (17.0 -> 29 us at 576 rows); on rows of 4352 each touches one. As a
+// launch of its own the copy took 5.4 us; behind the LayerNorm that runs before
+// fc1 it costs @RP@ us and leaves the weight in the caches for fc2.
+struct Repitch {
+    const uint16_t *src;
+    uint16_t *dst;
+    int rows, cols, ld;
+    __device__ __forceinline__ void copy(int block, int blocks) const {
+        const int cpr = cols >> 3, n = rows * cpr;
+        for (int i0 = block * 1024; i0 < n; i0 += blocks * 1024) {
+            u32x4_t v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = min(i0 + k * 256 + (int)threadIdx.x, n - 1);
+                v[k] = *(const u32x4_t *)(src + (size_t)i * 8);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = i0 + k * 256 + (int)threadIdx.x;
+                if (i < n) *(u32x4_t *)(dst + (size_t)(i / cpr) * ld + (i % cpr) * 8) = v[k];
+            }
+        }
+    }
+};
+
 // One wave per row. x = bf16(a + b) when b is given (written to sum_out if
 // non-null), then y = bf16((x - mean) * rsqrt(var + eps) * w + bias) with
 // mean and var = E[x^2] - mean^2 in fp32 (vision_kernels.cu:50-87).
@@ -41,74 +70,71 @@ __global__ void __launch_bounds__(256) v_layernorm_kernel(const uint16_t *__rest
                                                           const uint16_t *__restrict__ w,
                                                           const uint16_t *__restrict__ bias,
                                                           uint16_t *__restrict__ y, int rows,
-                                                          int cols, float eps) {
+                                                          int cols, float eps, Repitch rp) {
+    const int ln_blocks = (rows + 3) / 4;
+    if ((int)blockIdx.x >= ln_blocks) {
+        rp.copy((int)blockIdx.x - ln_blocks, (int)gridDim.x - ln_blocks);
+        return;
+    }
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= rows) return;
     const size_t base = (size_t)row * cols;
     const int nch = cols >> 3;
+    // the first NREG chunks of a lane (1152 columns: 3, the whole row) stay in
+    // registers between the two passes
+    constexpr int NREG = 3;
+    u32x4_t keep[NREG];
+    auto chunk = [&](int c) {
+        u32x4_t v = *(const u32x4_t *)(a + base + c * 8);
+        if (b) {
+            const u32x4_t vb = *(const u32x4_t *)(b + base + c * 8);
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = pack_bf2(lo_bf(v[j]) + lo_bf(vb[j]), hi_bf(v[j]) + hi_bf(vb[j]));
+        }
+        return v;
+    };
     float s = 0.f, s2 = 0.f;
-    for (int c = lane; c < nch; c += 64) {
-        u32x4_t va = *(const u32x4_t *)(a + base + c * 8), vb = {0, 0, 0, 0};
-        if (b) vb = *(const u32x4_t *)(b + base + c * 8);
-        u32x4_t vs;
+    auto add = [&](const u32x4_t &v, int c) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            float x0 = lo_bf(va[j]), x1 = hi_bf(va[j]);
-            if (b) {
-                x0 = bfround(x0 + lo_bf(vb[j]));
-                x1 = bfround(x1 + hi_bf(vb[j]));
-                vs[j] = pack_bf2(x0, x1);
-            }
+            const float x0 = lo_bf(v[j]), x1 = hi_bf(v[j]);
             s += x0 + x1;
             s2 += x0 * x0 + x1 * x1;
         }
-        if (b && sum_out) *(u32x4_t *)(sum_out + base + c * 8) = vs;
+        if (b && sum_out) *(u32x4_t *)(sum_out + base + c * 8) = v;
+    };
+#pragma unroll
+    for (int i = 0; i < NREG; i++) {
+        const int c = lane + i * 64;
+        if (c < nch) keep[i] = chunk(c);
     }
+#pragma unroll
+    for (int i = 0; i < NREG; i++) {
+        const int c = lane + i * 64;
+        if (c < nch) add(keep[i], c);
+    }
+    for (int c = lane + NREG * 64; c < nch; c += 64) add(chunk(c), c);
     s = wsum(s);
     s2 = wsum(s2);
     const float mean = s / (float)cols;
     const float var = s2 / (float)cols - mean * mean;
     const float inv = rsqrtf(var + eps);
-    for (int c = lane; c < nch; c += 64) {
-        u32x4_t va = *(const u32x4_t *)(a + base + c * 8), vb = {0, 0, 0, 0};
-        if (b) vb = *(const u32x4_t *)(b + base + c * 8);
-        u32x4_t gw = *(const u32x4_t *)(w + c * 8), gb = {0, 0, 0, 0};
+    auto put = [&](const u32x4_t &v, int c) {
+        const u32x4_t gw = *(const u32x4_t *)(w + c * 8);
+        u32x4_t gb = {0, 0, 0, 0}, o;
         if (bias) gb = *(const u32x4_t *)(bias + c * 8);
-        u32x4_t o;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float x0 = lo_bf(va[j]), x1 = hi_bf(va[j]);
-            if (b) {
-                x0 = bfround(x0 + lo_bf(vb[j]));
-                x1 = bfround(x1 + hi_bf(vb[j]));
-            }
-            o[j] = pack_bf2((x0 - mean) * inv * lo_bf(gw[j]) + lo_bf(gb[j]),
-                            (x1 - mean) * inv * hi_bf(gw[j]) + hi_bf(gb[j]));
-        }
+        for (int j = 0; j < 4; j++)
+            o[j] = pack_bf2((lo_bf(v[j]) - mean) * inv * lo_bf(gw[j]) + lo_bf(gb[j]),
+                            (hi_bf(v[j]) - mean) * inv * hi_bf(gw[j]) + hi_bf(gb[j]));
         *(u32x4_t *)(y + base + c * 8) = o;
-    }
-}
-
-// In place over [rows, ld] with `cols` live columns; columns [cols, ld)
-// are set to zero (the padded K of the following GEMM). ld, cols % 8 == 0.
-template <bool TANH>
-__global__ void v_gelu_kernel(uint16_t *__restrict__ x, int rows, int cols, int ld) {
-    const int cpr = ld >> 3;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * cpr) return;
-    const int c = (int)(i % cpr) * 8;
-    u32x4_t *p = (u32x4_t *)(x + (i / cpr) * ld + c);
-    if (c >= cols) {
-        *p = u32x4_t{0, 0, 0, 0};
-        return;
-    }
-    u32x4_t v = *p;
+    };
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const float a = lo_bf(v[j]), b = hi_bf(v[j]);
-        v[j] = TANH ? pack_bf2(gelu_tanh_f(a), gelu_tanh_f(b)) : pack_bf2(gelu_erf_f(a), gelu_erf_f(b));
+    for (int i = 0; i < NREG; i++) {
+        const int c = lane + i * 64;
+        if (c < nch) put(keep[i], c);
     }
-    *p = v;
+    for (int c = lane + NREG * 64; c < nch; c += 64) put(chunk(c), c);
 }
 
 template <bool TANH>
@@ -190,20 +216,21 @@ __global__ void v_cos_sin_kernel(const uint16_t *__restrict__ rot, float *__rest
 
 // qkv [R*n, 3, heads, D] (R images of n rows) -> q, k (rotary applied in
 // fp32, one rounding, rope.cu:157-180), head-major [R, heads, n, DP] with
-// columns [D, DP) zero (the flash kernel's head_dim-128 operands), and v
-// written straight into the flash kernel's V^T operand [R*heads, DP, S_pad]
-// (64-key tiles whose storage column p holds key p with bits 2 and 3
-// exchanged; rows d >= D and keys >= n zero). One block per (64-row tile,
-// image, head) stages the tile's q, k and v slices in LDS; 16-byte loads and
-// stores. v itself (head-major like q) is written only when v_out is not
-// null (the block-0 snapshots). D = 72, DP = 128 (D % 8 == 0, and the
-// 144-byte head slices keep 16-byte alignment).
-__global__ __launch_bounds__(256) void v_qkv_rope_vt_kernel(
+// columns [D, DP) zero, and v written straight into the flash kernels' V^T
+// operand [R*heads, D, S_pad] (64-key tiles whose storage column p holds key p
+// with bits 2 and 3 exchanged; keys >= n zero). DP = 72: the attention kernel's
+// operands; DP = 128: the head-major snapshots, with v (like q) instead of V^T.
+// One block per (64-row tile, image and head) stages the tile's q, k and v
+// slices in LDS; 16-byte loads and stores. D = 72: rotary partners lie 36
+// columns away, so a lane works on groups of 4.
+// One launch's latency bounds it (144 blocks at 576 rows): 8.1 -> @ROPE@ us with
+// the tables read 16 bytes at a time and rows of 72 instead of 128.
+template <int DP>
+__global__ __launch_bounds__(256) void v_qkv_rope_kernel(
     const uint16_t *__restrict__ qkv, const float *__restrict__ cosd, const float *__restrict__ sind,
-    uint16_t *__restrict__ q, uint16_t *__restrict__ k, uint16_t *__restrict__ vt,
-    uint16_t *__restrict__ v_out, int n, int s_pad) {
-    constexpr int D = kD, DP = kDP, CH = D / 8, LD = D + 8;
-    static_assert(D % 8 == 0 && D <= DP && DP % 8 == 0, "16-byte head slices");
+    uint16_t *__restrict__ q, uint16_t *__restrict__ k, uint16_t *__restrict__ v, int n, int s_pad) {
+    constexpr int D = kD, CH = D / 8, LD = D + 8, half = D / 2;
+    static_assert(D % 8 == 0 && half % 4 == 0 && D <= DP && DP % 8 == 0, "16-byte head slices, 4-column groups");
     __shared__ __attribute__((aligned(16))) uint16_t t[3][64][LD];
     const int s0 = blockIdx.x * 64, h = blockIdx.y % kNH, img = blockIdx.y / kNH;
     const int bh = blockIdx.y;
@@ -216,68 +243,59 @@ __global__ __launch_bounds__(256) void v_qkv_rope_vt_kernel(
         *(u32x4_t *)&t[part][r][c] = val;
     }
     __syncthreads();
-    const int half = D / 2;
-    // q, k: rows [s0, s0 + 64) x 16 chunks of 8 columns (chunks >= CH zero)
     for (int i = threadIdx.x; i < 64 * (DP / 8); i += 256) {
         const int r = i / (DP / 8), c = (i % (DP / 8)) * 8, srow = s0 + r;
         if (srow >= n) continue;
         const size_t o = ((size_t)bh * n + srow) * DP + c;
         u32x4_t oq = {0, 0, 0, 0}, ok = {0, 0, 0, 0};
         if (c < D) {
-            uint16_t rq[8], rk[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int d = c + e, dp = d < half ? d + half : d - half;
-                const float cc = cosd[(size_t)srow * D + d], sn = sind[(size_t)srow * D + d];
-                const float q0 = bf2f(t[0][r][d]), qh = bf2f(t[0][r][dp]);
-                const float k0 = bf2f(t[1][r][d]), kh = bf2f(t[1][r][dp]);
-                rq[e] = f2bf(d < half ? q0 * cc - qh * sn : q0 * cc + qh * sn);
-                rk[e] = f2bf(d < half ? k0 * cc - kh * sn : k0 * cc + kh * sn);
-            }
+            for (int w = 0; w < 2; w++) {
+                const int d = c + w * 4, dp = d < half ? d + half : d - half;
+                const float sg = d < half ? -1.f : 1.f;
+                const float4 cc = *(const float4 *)(cosd + (size_t)srow * D + d);
+                const float4 sn = *(const float4 *)(sind + (size_t)srow * D + d);
+                const float cv[4] = {cc.x, cc.y, cc.z, cc.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
+                float rq[4], rk[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                oq[e] = (uint32_t)rq[2 * e] | ((uint32_t)rq[2 * e + 1] << 16);
-                ok[e] = (uint32_t)rk[2 * e] | ((uint32_t)rk[2 * e + 1] << 16);
+                for (int e = 0; e < 4; e++) {
+                    const float q0 = bf2f(t[0][r][d + e]), qh = bf2f(t[0][r][dp + e]);
+                    const float k0 = bf2f(t[1][r][d + e]), kh = bf2f(t[1][r][dp + e]);
+                    rq[e] = q0 * cv[e] + sg * (qh * sv[e]);
+                    rk[e] = k0 * cv[e] + sg * (kh * sv[e]);
+                }
+                oq[w * 2] = pack_bf2(rq[0], rq[1]);
+                oq[w * 2 + 1] = pack_bf2(rq[2], rq[3]);
+                ok[w * 2] = pack_bf2(rk[0], rk[1]);
+                ok[w * 2 + 1] = pack_bf2(rk[2], rk[3]);
             }
         }
-        *(u32x4_t *)(q + o) = oq;
-        *(u32x4_t *)(k + o) = ok;
-        if (v_out) {
+        if (q) *(u32x4_t *)(q + o) = oq;
+        if (k) *(u32x4_t *)(k + o) = ok;
+        if (DP != D && v) {
             u32x4_t ov = {0, 0, 0, 0};
             if (c < D) ov = *(const u32x4_t *)&t[2][r][c];
-            *(u32x4_t *)(v_out + o) = ov;
+            *(u32x4_t *)(v + o) = ov;
         }
     }
-    // V^T: rows d < DP, 8 chunks of 8 storage columns of this 64-key tile
-    for (int i = threadIdx.x; i < DP * 8; i += 256) {
+    if (DP != D) return;
+    // V^T: rows d < D, 8 chunks of 8 storage columns of this 64-key tile
+    for (int i = threadIdx.x; i < D * 8; i += 256) {
         const int d = i / 8, p0 = (i % 8) * 8;
-        u32x4_t ov = {0, 0, 0, 0};
-        if (d < D) {
+        u32x4_t ov;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int pa = p0 + 2 * e, pb = pa + 1;
-                const int ka = (pa & ~12) | ((pa & 4) << 1) | ((pa & 8) >> 1);
-                const int kb = (pb & ~12) | ((pb & 4) << 1) | ((pb & 8) >> 1);
-                ov[e] = (uint32_t)t[2][ka][d] | ((uint32_t)t[2][kb][d] << 16);
-            }
+        for (int e = 0; e < 4; e++) {
+            const int pa = p0 + 2 * e, pb = pa + 1;
+            const int ka = (pa & ~12) | ((pa & 4) << 1) | ((pa & 8) >> 1);
+            const int kb = (pb & ~12) | ((pb & 4) << 1) | ((pb & 8) >> 1);
+            ov[e] = (uint32_t)t[2][ka][d] | ((uint32_t)t[2][kb][d] << 16);
         }
-        *(u32x4_t *)(vt + ((size_t)bh * DP + d) * s_pad + s0 + p0) = ov;
+        *(u32x4_t *)(v + ((size_t)bh * D + d) * s_pad + s0 + p0) = ov;
     }
 }
 
-// flash output [n, heads*DP] (seq-major) -> [n, heads*D]; one thread per
-// 8 consecutive columns (D % 8 == 0)
-__global__ void v_unpad_heads_kernel(const uint16_t *__restrict__ in, uint16_t *__restrict__ out,
-                                     int n, int heads, int D, int DP) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int cpr = D / 8;
-    if (i >= (size_t)n * heads * cpr) return;
-    const int c = (int)(i % cpr) * 8, h = (int)((i / cpr) % heads);
-    const size_t s = i / ((size_t)cpr * heads);
-    *(u32x4_t *)(out + (s * heads + h) * D + c) = *(const u32x4_t *)(in + (s * heads + h) * DP + c);
-}
-
-// rows x cols -> rows x ld, columns [cols, ld) zero (cols, ld % 8 == 0)
+// rows of ld elements, columns [cols, ld) as zeros (cols, ld % 8 == 0): the fc1
+// snapshot
 __global__ void v_pad_rows_kernel(const uint16_t *__restrict__ in, uint16_t *__restrict__ out,
                                   int rows, int cols, int ld) {
     const int cpr = ld >> 3;
@@ -286,7 +304,7 @@ __global__ void v_pad_rows_kernel(const uint16_t *__restrict__ in, uint16_t *__r
     const size_t r = i / cpr;
     const int c = (int)(i % cpr) * 8;
     u32x4_t v = {0, 0, 0, 0};
-    if (c < cols) v = *(const u32x4_t *)(in + r * cols + c);
+    if (c < cols) v = *(const u32x4_t *)(in + r * ld + c);
     *(u32x4_t *)(out + r * ld + c) = v;
 }
 
@@ -380,21 +398,16 @@ bool bad(const char *what) {
 }
 
 void layernorm(const void *a, const void *b, void *sum_out, const void *w, const void *bias, void *y,
-               int rows, int cols, float eps) {
-    v_layernorm_kernel<<<hd_cdiv(rows, 4), 256, 0, hd_stream()>>>(
+               int rows, int cols, float eps, const Repitch &rp = Repitch{}) {
+    const unsigned extra = rp.src ? 512 : 0;
+    v_layernorm_kernel<<<hd_cdiv(rows, 4) + extra, 256, 0, hd_stream()>>>(
         (const uint16_t *)a, (const uint16_t *)b, (uint16_t *)sum_out, (const uint16_t *)w,
-        (const uint16_t *)bias, (uint16_t *)y, rows, cols, eps);
-}
-
-template <bool TANH>
-void gelu_padded(void *x, int rows, int cols, int ld) {
-    v_gelu_kernel<TANH><<<hd_cdiv((size_t)rows * (ld / 8), 256), 256, 0, hd_stream()>>>(
-        (uint16_t *)x, rows, cols, ld);
+        (const uint16_t *)bias, (uint16_t *)y, rows, cols, eps, rp);
 }
 
 // ---- workspace layout ----
 struct Layout {
-    int64_t h, ar, ln, tmp, qkv, q, k, v, vt, f1, w2, cs, sn, gws, total;
+    int64_t h, ar, ln, tmp, qkv, q, k, vt, f1, w2, cs, sn, gws, total;
 };
 
 int64_t al(int64_t b) { return (b + 255) & ~(int64_t)255; }
@@ -404,18 +417,16 @@ Layout layout_of(int64_t R, int64_t n) {
     Layout L;
     int64_t b = 0;
     const int64_t N = R * n;
-    // head-major operands [R, 16, n, 128] plus one 128-row tile of slack:
-    // the flash kernel reads whole 128-row query / key tiles
-    const int64_t hm = (R * kNH * n + 128) * kDP * 2;
+    // head-major operands [R, 16, n, 72]
+    const int64_t hm = R * kNH * n * kD * 2;
     L.tmp = b; b += al(N * kH * 2);
     L.h = b; b += al(N * kH * 2);
     L.ar = b; b += al(N * kH * 2);
     L.ln = b; b += al(N * kH * 2);
-    L.qkv = b; b += al(N * (kQKV > kNH * kDP ? kQKV : kNH * kDP) * 2);
+    L.qkv = b; b += al(N * kQKV * 2);
     L.q = b; b += al(hm);
     L.k = b; b += al(hm);
-    L.v = b; b += al(hm);
-    L.vt = b; b += al(hd_flash_vt_bytes((int)R, kNH, (int)n));
+    L.vt = b; b += al(R * kNH * kD * ((n + 63) / 64 * 64) * 2);
     L.f1 = b; b += al(N * kIP * 2);
     L.w2 = b; b += al((int64_t)kH * kIP * 2);
     L.cs = b; b += al(n * kD * 4);
@@ -602,7 +613,6 @@ extern "C" void hd_vision_layout(int64_t n, int64_t m, hd_vision_offsets *o) {
     o->qkv = L.qkv;
     o->q = L.q;
     o->k = L.k;
-    o->v = L.v;
     o->scores = L.vt;
     o->fc1 = L.f1;
     o->fc2 = L.w2;
@@ -732,6 +742,20 @@ extern "C" hd_status hd_vision_prepare_tables(hd_vision_workspace *ws, int n, in
     return HD_OK;
 }
 
+// fc1 of a merger with its erf GELU; `pre` (may be null) receives the values
+// before the GELU.
+static void merger_fc1(const hd_vision_merger_binding *d, const void *x, void *f1, int m, void *pre, void *ws,
+                       int64_t ws_bytes) {
+    const int W = kU * kH;
+    if (!pre) {
+        hd_linear_gelu(x, d->fc1_w, d->fc1_b, f1, m, W, W, true, ws, ws_bytes, W);
+        return;
+    }
+    hd_linear_ws(x, d->fc1_w, d->fc1_b, f1, m, W, W, ws, ws_bytes);
+    snap(pre, f1, (size_t)m * W * 2);
+    hd_vision_gelu_exact(f1, f1, (size_t)m * W);
+}
+
 // R images of the same grid_h x grid_w: every GEMM, LayerNorm and
 // elementwise kernel runs over the R*n rows at once, attention per image
 // (the flash kernel's batch dimension).
@@ -759,9 +783,9 @@ static hd_status forward_impl(const hd_vision_binding *bw, hd_vision_workspace *
     uint16_t *tmp = (uint16_t *)(base + L.tmp), *h = (uint16_t *)(base + L.h);
     uint16_t *ar = (uint16_t *)(base + L.ar), *ln = (uint16_t *)(base + L.ln);
     uint16_t *qkv = (uint16_t *)(base + L.qkv), *q = (uint16_t *)(base + L.q);
-    uint16_t *k = (uint16_t *)(base + L.k), *v = (uint16_t *)(base + L.v);
-    uint16_t *vt = (uint16_t *)(base + L.vt), *f1 = (uint16_t *)(base + L.f1);
+    uint16_t *k = (uint16_t *)(base + L.k);
     uint16_t *w2 = (uint16_t *)(base + L.w2);
+    uint16_t *vt = (uint16_t *)(base + L.vt), *f1 = (uint16_t *)(base + L.f1);
     float *cs = (float *)(base + L.cs), *sn = (float *)(base + L.sn);
     void *gws = base + L.gws;
     const int64_t gwsb = hd_gemm_ws_bytes();
@@ -789,35 +813,32 @@ static hd_status forward_impl(const hd_vision_binding *bw, hd_vision_workspace *
         }
         hd_linear_ws(ln, b->qkv_w, b->qkv_b, qkv, N, kQKV, kH, gws, gwsb);
         if (s0) snap(s0[HD_B0_QKV], qkv, (size_t)N * kQKV * 2);
-        v_qkv_rope_vt_kernel<<<dim3((unsigned)((n + 63) / 64), (unsigned)(R * kNH)), 256, 0, st>>>(
-            qkv, cs, sn, q, k, vt, s0 ? v : nullptr, n, (int)((n + 63) / 64 * 64));
-        if (s0) {
-            snap(s0[HD_B0_Q], q, (size_t)R * kNH * n * kDP * 2);
-            snap(s0[HD_B0_K], k, (size_t)R * kNH * n * kDP * 2);
-            snap(s0[HD_B0_V], v, (size_t)R * kNH * n * kDP * 2);
-        }
-        // full attention per image over the zero-padded heads; output
-        // [R*n, 16*128] (seq-major) into qkv
-        if (hd_flash_attention(q, k, vt, nullptr, qkv, R, kNH, kNH, n, kDP, 0, scale, 1)) {
+        const dim3 rg((unsigned)((n + 63) / 64), (unsigned)(R * kNH));
+        v_qkv_rope_kernel<kD><<<rg, 256, 0, st>>>(qkv, cs, sn, q, k, vt, n, (int)((n + 63) / 64 * 64));
+        if (s0 && (s0[HD_B0_Q] || s0[HD_B0_K] || s0[HD_B0_V]))
+            v_qkv_rope_kernel<kDP><<<rg, 256, 0, st>>>(qkv, cs, sn, (uint16_t *)s0[HD_B0_Q], (uint16_t *)s0[HD_B0_K],
+                                                       (uint16_t *)s0[HD_B0_V], n, 0);
+        // full attention per image, output [R*n, 16*72] (seq-major)
+        if (hd_flash_v72(q, k, vt, ln, R, kNH, n, scale)) {
             hd_set_error("vision: attention failed: %s", hd_cuda_last_error());
             return HD_ERR_RUNTIME;
         }
-        v_unpad_heads_kernel<<<hd_cdiv((size_t)N * kH / 8, 256), 256, 0, st>>>(qkv, ln, N, kNH, kD, kDP);
         if (s0) snap(s0[HD_B0_ATTN_MERGED], ln, nH);
         hd_linear_ws(ln, b->proj_w, b->proj_b, tmp, N, kH, kH, gws, gwsb);
         if (s0) snap(s0[HD_B0_PROJ], tmp, nH);
         // attn_resid = bf16(h + proj); ln = LayerNorm2(attn_resid)
-        layernorm(h, tmp, ar, b->norm2_w, b->norm2_b, ln, N, kH, eps);
+        // (and the fc2 weight at its aligned row stride)
+        layernorm(h, tmp, ar, b->norm2_w, b->norm2_b, ln, N, kH, eps,
+                  Repitch{(const uint16_t *)b->fc2_w, w2, kH, kI, kIP});
         if (s0) {
             snap(s0[HD_B0_ATTN_RESID], ar, nH);
             snap(s0[HD_B0_NORM2], ln, nH);
         }
-        hd_linear_ld(ln, b->fc1_w, b->fc1_b, f1, N, kI, kH, kIP);
-        gelu_padded<true>(f1, N, kI, kIP);
-        if (s0) snap(s0[HD_B0_FC1], f1, (size_t)N * kIP * 2);
-        v_pad_rows_kernel<<<hd_cdiv((size_t)kH * (kIP / 8), 256), 256, 0, st>>>(
-            (const uint16_t *)b->fc2_w, w2, kH, kI, kIP);
-        hd_linear_ws(f1, w2, b->fc2_b, tmp, N, kH, kIP, gws, gwsb);
+        hd_linear_gelu(ln, b->fc1_w, b->fc1_b, f1, N, kI, kH, false, gws, gwsb, kIP);
+        if (s0 && s0[HD_B0_FC1])
+            v_pad_rows_kernel<<<hd_cdiv((size_t)N * (kIP / 8), 256), 256, 0, st>>>(
+                f1, (uint16_t *)s0[HD_B0_FC1], N, kI, kIP);
+        hd_linear_strided(f1, kIP, w2, kIP, b->fc2_b, tmp, N, kH, kI, gws, gwsb);
         if (s0) snap(s0[HD_B0_FC2], tmp, nH);
         // h = bf16(attn_resid + fc2), then the next LayerNorm (next block's
         // norm1, or the final merger's norm over 1152)
@@ -838,9 +859,7 @@ static hd_status forward_impl(const hd_vision_binding *bw, hd_vision_workspace *
             uint16_t *dn = ar;                 // [m, 4608] == [N, 1152]; attn_resid is dead here
             layernorm(h, nullptr, nullptr, d->norm_w, d->norm_b, dn, m, kU * kH, eps);
             snap(sd[0], dn, nH);
-            hd_linear_ws(dn, d->fc1_w, d->fc1_b, f1, m, kU * kH, kU * kH, gws, gwsb);
-            snap(sd[1], f1, (size_t)m * kU * kH * 2);
-            gelu_padded<false>(f1, m, kU * kH, kU * kH);
+            merger_fc1(d, dn, f1, m, sd[1], gws, gwsb);
             snap(sd[2], f1, (size_t)m * kU * kH * 2);
             if (deepstack_out[ds_j])
                 hd_linear_ws(f1, d->fc2_w, d->fc2_b, deepstack_out[ds_j], m, kO, kU * kH, gws, gwsb);
@@ -853,9 +872,7 @@ static hd_status forward_impl(const hd_vision_binding *bw, hd_vision_workspace *
     void **sm = ws->merger_snaps;
     snap(sm[0], ln, nH);
     snap(sm[1], ln, nH);
-    hd_linear_ws(ln, bw->merger.fc1_w, bw->merger.fc1_b, f1, m, kU * kH, kU * kH, gws, gwsb);
-    snap(sm[2], f1, (size_t)m * kU * kH * 2);
-    gelu_padded<false>(f1, m, kU * kH, kU * kH);
+    merger_fc1(&bw->merger, ln, f1, m, sm[2], gws, gwsb);
     snap(sm[3], f1, (size_t)m * kU * kH * 2);
     hd_linear_ws(f1, bw->merger.fc2_w, bw->merger.fc2_b, image_embeds_out, m, kO, kU * kH, gws, gwsb);
     snap(sm[4], image_embeds_out, (size_t)m * kO * 2);
