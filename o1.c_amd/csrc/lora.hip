@@ -1,13 +1,16 @@
 // GPU LoRA merge-on-load: W = bf16(float(W) + s * (up @ down)), fp32 delta.
-// Replaces hd_lora_merge_gpu (lora_merge.cu:35-104). One launch per target;
-// the delta never reaches HBM. Two kernels:
+// Replaces hd_lora_merge_gpu (lora_merge.cu:35-104). The delta never reaches
+// HBM. Two kernels:
 //  - lora_merge_stream_kernel (R <= 64, R % 4 == 0): persistent blocks
-//    stream W through an LDS ring, rank product on the bf16 matrix cores
-//    with fp32 operands split in three bf16 parts;
+//    stream W through registers, rank product on the bf16 matrix cores
+//    with fp32 operands split in three bf16 parts; one launch for up to
+//    LM_TG targets;
 //  - lora_merge_mfma_kernel (any other R): a block per 128 x 128 tile, rank
-//    product on the fp32 matrix cores (v_mfma_f32_32x32x2_f32).
+//    product on the fp32 matrix cores (v_mfma_f32_32x32x2_f32); one launch
+//    per target.
 #include <stdio.h>
 
+#include <algorithm>
 #include <map>
 #include <vector>
 
@@ -154,27 +157,28 @@ __device__ __forceinline__ void split3(float x, uint16_t &h0, uint16_t &h1, uint
     h2 = f2bf(r1 - bf2f(h1));
 }
 
-// Streaming merge for R <= 64 (R % 4 == 0, K % 8 == 0): a persistent block of
-// 8 waves per CU walks a contiguous run of 128 x 64 tiles of W (row strips
-// first), so the whole launch is one stream of W reads and writes:
-//  - W tiles go global -> LDS with buffer loads straight to LDS, two tiles
-//    ahead, into a ring of three 16 KB slots; the update reads W from LDS in
-//    the accumulator layout, writes the bf16 result back in place, and the
-//    tile leaves with coalesced 16-byte buffer stores;
-//  - the rank product uses the three-part split above (six bf16 part
-//    products per fp32 product, in three accumulators); the up strip's part
-//    planes are staged once per row strip and each wave keeps its B
-//    fragments of them in registers for the whole strip; the down slice's
-//    planes are staged once per tile, into one of two plane buffers, from
-//    registers loaded a tile ahead, while the tile's MFMAs run (all twelve A
-//    fragments of a tile are requested before its first MFMA);
-//  - MFMA A = down^T (rows: W columns k), B = up (columns: W rows n), so a
-//    lane holds four consecutive k of one W row per accumulator group.
-// Every vector memory instruction in the loop is issued unconditionally
-// (offsets past the data read as zero or are dropped), so the counts behind
-// the hand-placed vmcnt waits for the ring hold on every path; register
-// loads go through the compiler, which places their waits.
-#define LT_N 128
+// Streaming merge for R <= 64 (R % 4 == 0, K % 8 == 0). Persistent blocks of 8
+// waves, one per CU, walk contiguous runs of 256 x 64 tiles of W, so the launch
+// is one stream of W reads and writes, which bounds it:
+//  * wave w owns rows 32 w .. 32 w + 31 of a tile, MFMA A = down^T (rows:
+//    columns k of W), B = up (columns: rows of W). The A rows take k in an order
+//    that leaves a lane with 8 consecutive columns of one row: W goes from
+//    memory to registers and back in 16-byte pieces, two tiles ahead, with no
+//    pass through LDS, and a load covers 64 bytes of each of 16 rows (with
+//    32 x 32 products it would be 32 bytes of 32 rows: 219 us instead of 198);
+//  * the up rows of a wave are split into their three bf16 parts in registers,
+//    once per row strip; only the down slice, which all waves share, is staged
+//    in LDS: its part planes are written for the next tile while the current
+//    tile's MFMAs run, into the other of two buffers;
+//  * waves 4 .. 7 run half a tile behind waves 0 .. 3, so that on each SIMD one
+//    wave updates and stores while the other multiplies (in step: 217 us).
+// One layer's seven targets at R = 64, 386 MB of W read and written: 241 us ->
+// 197 us per call, 189 us in the kernel = 4.1 TB/s (a copy here reaches 4.8).
+// Before, 128 x 64 tiles with W, up and down all staged in LDS took one launch
+// per shape, and five LDS passes over W. Without the MFMAs it would take 178 us.
+// Every load and store is unconditional: offsets past the data read as zero
+// or are dropped.
+#define LT_N 256
 #define LT_K 64
 #define LT_LD 72   // plane row stride (bf16): 144-byte rows, conflict-free 16-byte reads
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t lt_rsrc(const void *base, uint32_t nbytes) {
@@ -184,103 +188,75 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t lt_rsrc(const void *base, uint
     return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0,
                                              __builtin_amdgcn_readfirstlane(nbytes), 0x00020000);
 }
-// One launch merges every target of a batch that shares (N, K, R): the
-// tiles of all of them form one index space (target-major, then row strip,
-// then column tile) that the persistent blocks split evenly, so small
-// targets (the 1024-row k / v projections) no longer pay a launch and a
-// pipeline fill each.
+// One launch merges up to LM_TG targets of any shapes, handed over by value:
+// their tiles form one index space (target-major, then row strip, then column
+// tile) that the blocks split evenly; first[g] is the first tile of target g.
+#define LM_TG 32
 struct LmTarget {
     uint16_t *w;
     const float *up;
     const float *down;
     float scale;
+    int N, K, R, ntk, nstrip;
 };
-__global__ __launch_bounds__(512, 1) void lora_merge_stream_kernel(const LmTarget *__restrict__ tg, int N,
-                                                                 int K, int R, int ntk, int nstrip,
-                                                                 int total) {
-    __shared__ __attribute__((aligned(1024))) uint16_t wring[3][LT_N * LT_K];
-    __shared__ __attribute__((aligned(16))) uint16_t upl[3][LT_N * LT_LD];
+struct LmBatch {
+    int n, total;
+    int first[LM_TG];
+    LmTarget t[LM_TG];
+};
+__global__ __launch_bounds__(512, 1) void lora_merge_stream_kernel(const LmBatch bt) {
     __shared__ __attribute__((aligned(16))) uint16_t dpl[2][3][LT_K * LT_LD];
 #if defined(__HIP_DEVICE_COMPILE__)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int l32 = lane & 31, lh = lane >> 5;
-    const int tb = (int)((int64_t)blockIdx.x * total / gridDim.x);
-    const int te = (int)((int64_t)(blockIdx.x + 1) * total / gridDim.x);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lg = lane >> 4;
+    const int tb = (int)((int64_t)blockIdx.x * bt.total / gridDim.x);
+    const int te = (int)((int64_t)(blockIdx.x + 1) * bt.total / gridDim.x);
     if (tb >= te) return;
     const uint32_t OOB = 0x80000000u;
-    const uint32_t w_bytes = (uint32_t)((size_t)N * K * 2), u_bytes = (uint32_t)((size_t)N * R * 4),
-                   d_bytes = (uint32_t)((size_t)R * K * 4);
-    const int tpt = nstrip * ntk;   // tiles per target
-    // Each wave owns the 32 x 32 sub-tile of W its accumulator covers (rows
-    // nblk*32.., columns kblk*32..) and alone loads, updates and stores it,
-    // so W needs no barrier. Its 2 KB in a ring slot: instruction i, lane L
-    // -> sub-tile row r = 16 i + L / 4, 16-byte position p = L % 4 of the
-    // 64-byte row, holding column chunk c = p ^ ((r >> 2) & 3) (the XOR
-    // spreads the update's 8-byte reads of 32 rows over the banks).
-    const int kblk = wave & 1, nblk = wave >> 1;
-    int wn[2], wc[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int r = i * 16 + (lane >> 2);
-        wn[i] = nblk * 32 + r;
-        wc[i] = kblk * 32 + ((lane & 3) ^ ((r >> 2) & 3)) * 8;
-    }
-    // tile coordinates (row strip, column tile) and ring slots advance
-    // incrementally: a division by the runtime ntk costs tens of scalar
-    // instructions, and every wave needs them for three tiles per step
     struct TC {
         int g, tn, tk;   // target, row strip, column tile
         bool ok;         // the tile exists (t < te)
-        uint16_t *w;     // the target's tensors and scale (wave-uniform)
-        const float *up, *down;
-        float scale;
-    };
-    auto tc_load = [&](TC &c) {
-        const int gg = c.g < total / tpt ? c.g : 0;   // past the last target: any valid entry
-        c.w = tg[gg].w;
-        c.up = tg[gg].up;
-        c.down = tg[gg].down;
-        c.scale = tg[gg].scale;
+        LmTarget d;      // the target (wave-uniform)
     };
     auto tc_next = [&](TC c, int t_next) {
         c.tk++;
-        if (c.tk == ntk) {
+        if (c.tk == c.d.ntk) {
             c.tk = 0;
             c.tn++;
-            if (c.tn == nstrip) {
+            if (c.tn == c.d.nstrip) {
                 c.tn = 0;
                 c.g++;
-                tc_load(c);
+                c.d = bt.t[c.g < bt.n ? c.g : 0];   // past the last target: any valid entry
             }
         }
         c.ok = t_next < te;
         return c;
     };
-    auto w_off = [&](const TC &c, int i) -> uint32_t {
-        const int gn = c.tn * LT_N + wn[i], gk = c.tk * LT_K + wc[i];
-        return c.ok && gn < N && gk < K ? (uint32_t)(gn * K + gk) * 2u : OOB;
+    // piece p of four: row (p / 2) * 16 + l16, columns (p % 2) * 32 + lg * 8 .. +7
+    auto w_off = [&](const TC &c, int p) -> uint32_t {
+        const int gn = c.tn * LT_N + wave * 32 + (p / 2) * 16 + l16, gk = c.tk * LT_K + (p % 2) * 32 + lg * 8;
+        return c.ok && gn < c.d.N && gk < c.d.K ? ((uint32_t)gn * (uint32_t)c.d.K + (uint32_t)gk) * 2u : OOB;
     };
-    auto issue_w = [&](const TC &c, int sl) {
-        uint16_t *sub = wring[sl] + wave * 1024;
-        const __amdgpu_buffer_rsrc_t rw = lt_rsrc(c.w, w_bytes);
+    auto load_w = [&](const TC &c, u32x4_t (&w)[4]) {
+        const __amdgpu_buffer_rsrc_t rw = lt_rsrc(c.d.w, (uint32_t)((size_t)c.d.N * c.d.K * 2));
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (HD_LDS void *)(sub + i * 512), 16, w_off(c, i), 0, 0,
-                                                     0);
+        for (int p = 0; p < 4; p++)
+            w[p] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, w_off(c, p), 0, 0));
     };
     // down slice of a tile: ranks rr, rr + 1, columns kc .. kc + 3
     const int kc = (tid % 16) * 4, rr = (tid / 16) * 2;
-    f32x4_t DA[2], DB[2];
     auto load_down = [&](const TC &c, f32x4_t (&d)[2]) {
-        const __amdgpu_buffer_rsrc_t rd = lt_rsrc(c.down, d_bytes);
+        const __amdgpu_buffer_rsrc_t rd = lt_rsrc(c.d.down, (uint32_t)((size_t)c.d.R * c.d.K * 4));
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int r = rr + j, gk = c.tk * LT_K + kc;
-            const uint32_t o = c.ok && r < R && gk < K ? (uint32_t)(r * K + gk) * 4u : OOB;
+            const uint32_t o = c.ok && r < c.d.R && gk < c.d.K ? ((uint32_t)r * (uint32_t)c.d.K + (uint32_t)gk) * 4u : OOB;
             d[j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rd, o, 0, 0));
         }
     };
-    // down registers -> part planes [k][r] of buffer b
+    // down registers -> part planes of buffer b: column k = 32 kp + 8 g + 4 h + e
+    // in plane row 32 kp + 16 h + 4 g + e
+    const int krow = (kc & 32) | ((kc & 4) << 2) | ((kc & 24) >> 1);
     auto put_down = [&](const f32x4_t (&d)[2], int b) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -289,180 +265,137 @@ __global__ __launch_bounds__(512, 1) void lora_merge_stream_kernel(const LmTarge
             split3(d[1][e], h1[0], h1[1], h1[2]);
 #pragma unroll
             for (int pl = 0; pl < 3; pl++)
-                *(uint32_t *)(dpl[b][pl] + (kc + e) * LT_LD + rr) = (uint32_t)h0[pl] | ((uint32_t)h1[pl] << 16);
+                *(uint32_t *)(dpl[b][pl] + (krow + e) * LT_LD + rr) = (uint32_t)h0[pl] | ((uint32_t)h1[pl] << 16);
         }
     };
-    auto stage_up = [&](const TC &c) {   // the up strip's part planes; drains the queue
-        const __amdgpu_buffer_rsrc_t ru = lt_rsrc(c.up, u_bytes);
-        const int row = tid / 4, r16 = (tid % 4) * 16, gn = c.tn * LT_N + row;
-        float uv[16];
+    // this lane's up rows in three parts: B operands, row nb*16 + l16, ranks
+    // ks*32 + lg*8 .. +7
+    bf16x8_t fb[2][2][3];
+    auto load_up = [&](const TC &c) {
+        const __amdgpu_buffer_rsrc_t ru = lt_rsrc(c.d.up, (uint32_t)((size_t)c.d.N * c.d.R * 4));
+        f32x4_t u[4][2];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = r16 + 4 * j;
-            const uint32_t o = gn < N && r < R ? (uint32_t)(gn * R + r) * 4u : OOB;
-            const f32x4_t v = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
-            uv[4 * j] = v[0]; uv[4 * j + 1] = v[1]; uv[4 * j + 2] = v[2]; uv[4 * j + 3] = v[3];
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        uint16_t h[3][16];
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) split3(uv[e], h[0][e], h[1][e], h[2][e]);
-#pragma unroll
-        for (int pl = 0; pl < 3; pl++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                u32x4_t v;
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    v[e] = (uint32_t)h[pl][q * 8 + 2 * e] | ((uint32_t)h[pl][q * 8 + 2 * e + 1] << 16);
-                *(u32x4_t *)(upl[pl] + row * LT_LD + r16 + q * 8) = v;
+            for (int j = 0; j < 2; j++) {
+                const int gn = c.tn * LT_N + wave * 32 + (i / 2) * 16 + l16, r = (i % 2) * 32 + lg * 8 + j * 4;
+                const uint32_t o = gn < c.d.N && r < c.d.R ? ((uint32_t)gn * (uint32_t)c.d.R + (uint32_t)r) * 4u : OOB;
+                u[i][j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ru, o, 0, 0));
             }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            u32x4_t v[3];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                uint16_t h0[3], h1[3];
+                split3(u[i][e >> 1][(e & 1) * 2], h0[0], h0[1], h0[2]);
+                split3(u[i][e >> 1][(e & 1) * 2 + 1], h1[0], h1[1], h1[2]);
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) v[pl][e] = (uint32_t)h0[pl] | ((uint32_t)h1[pl] << 16);
+            }
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) fb[i / 2][i % 2][pl] = __builtin_bit_cast(bf16x8_t, v[pl]);
+        }
     };
-    // prologue: W(tb), down(tb), W(tb+1), down(tb+1); the planes of tile tb
     TC c0;                                // tile t
-    c0.g = tb / tpt;
-    c0.tn = (tb % tpt) / ntk;
-    c0.tk = tb % ntk;
+    int tfirst = 0;
+    c0.g = 0;
+#pragma unroll
+    for (int g = 1; g < LM_TG; g++)
+        if (g < bt.n && bt.first[g] <= tb) {
+            c0.g = g;
+            tfirst = bt.first[g];
+        }
+    c0.d = bt.t[c0.g];
+    c0.tn = (tb - tfirst) / c0.d.ntk;
+    c0.tk = (tb - tfirst) % c0.d.ntk;
     c0.ok = true;
-    tc_load(c0);
     TC c1 = tc_next(c0, tb + 1);          // tile t + 1
-    TC c2 = tc_next(c1, tb + 2);          // tile t + 2
-    int sl = 0;                           // ring slot of tile t
-    issue_w(c0, 0);
+    u32x4_t WA[4], WB[4];
+    f32x4_t DA[2], DB[2];
     load_down(c0, DA);
-    issue_w(c1, 1);
+    load_w(c0, WA);
     load_down(c1, DB);
-    int staged = c0.g * nstrip + c0.tn;   // target and row strip of the staged up planes
-    stage_up(c0);          // vmcnt(0): down(tb) landed as well
+    load_w(c1, WB);
+    int up_g = c0.g, up_tn = c0.tn;       // the strip whose up rows are in registers
+    load_up(c0);
     put_down(DA, tb & 1);
-    // this wave's up fragments (B operands) stay in registers for the whole
-    // row strip: read from the staged planes after each staging barrier
-    bf16x8_t fb[4][3];
-    auto read_up = [&]() {
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++)
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-                fb[ks][p] = *(const bf16x8_t *)(upl[p] + (nblk * 32 + l32) * LT_LD + ks * 16 + lh * 8);
-    };
-    bool need_up = true;
-    // tile t splits down(t+1) (registers dsplit) for the next tile and loads
-    // down(t+2) into the registers down(t) used (dload); the loop runs two
-    // tiles per trip with the two register sets swapped, so no register
-    // holding a load in flight is ever copied
-    auto step = [&](int t, const f32x4_t (&dsplit)[2], f32x4_t (&dload)[2]) {
+    // tile t splits down(t+1) (dsplit) for the next tile and loads down(t+2)
+    // into the registers down(t) used (dload), and W(t+2) into those of W(t);
+    // the loop runs two tiles per trip with the register sets swapped, so no
+    // register holding a load in flight is ever copied
+    auto step = [&](int t, u32x4_t (&w)[4], const f32x4_t (&dsplit)[2], f32x4_t (&dload)[2]) {
         // the planes of tile t are written; every wave is past the previous
         // tile's MFMAs (the other plane buffer is free)
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (c0.g * nstrip + c0.tn != staged) {
-            stage_up(c0);
-            staged = c0.g * nstrip + c0.tn;
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            need_up = true;
+        if (c0.g != up_g || c0.tn != up_tn) {
+            load_up(c0);
+            up_g = c0.g;
+            up_tn = c0.tn;
         }
-        if (need_up) {
-            read_up();
-            need_up = false;
-        }
-        // the MFMAs of tile t; the next tile's down slice is split into the
-        // other plane buffer in between (independent VALU and LDS work)
-        const int b = t & 1;
-        // three accumulators by part-product order (2^-16: a2b0 a1b1 a0b2;
-        // 2^-8: a1b0 a0b1; leading: a0b0), summed smallest first at the end:
-        // three dependent MFMA chains of at most 12 instead of one of 24
-        f32x16_t acc_s, acc_m, acc_l;
-#pragma unroll
-        for (int e = 0; e < 16; e++) acc_s[e] = acc_m[e] = acc_l[e] = 0.f;
-        // every fragment of the tile is requested before the first MFMA
-        bf16x8_t fa[4][3];
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const int rc = ks * 16 + lh * 8;
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-                fa[ks][p] = *(const bf16x8_t *)(dpl[b][p] + (kblk * 32 + l32) * LT_LD + rc);
-        }
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            const bf16x8_t *a = fa[ks], *bb = fb[ks];
-            acc_s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], bb[0], acc_s, 0, 0, 0);
-            acc_m = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], bb[0], acc_m, 0, 0, 0);
-            acc_l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], bb[0], acc_l, 0, 0, 0);
-            acc_s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], bb[1], acc_s, 0, 0, 0);
-            acc_m = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], bb[1], acc_m, 0, 0, 0);
-            acc_s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], bb[2], acc_s, 0, 0, 0);
-        }
-        // the next tile's down slice into the other plane buffer (its reads
-        // above are issued; the MFMAs run meanwhile)
-        put_down(dsplit, b ^ 1);
-        f32x16_t acc;
-#pragma unroll
-        for (int e = 0; e < 16; e++) acc[e] = acc_l[e] + (acc_m[e] + acc_s[e]);
-        // loads for two tiles ahead, issued after down(t+1)'s registers are
-        // consumed so that waiting for those never waits for these
-        const int sl2 = sl == 0 ? 2 : sl - 1;   // tile t+2 takes the slot tile t-1 used
-        issue_w(c2, sl2);
+        const TC c2 = tc_next(c1, t + 2);
         load_down(c2, dload);
-        // W update in LDS, in this wave's own sub-tile: row l32, columns
-        // 8q + 4lh .. +3 (chunk q at position q ^ ((l32 >> 2) & 3)). W(t) of
-        // this wave landed: newer than it are the loads down(t), W(t+1),
-        // down(t+1), W(t+2) and down(t+2) (10) and the stores of t-2 and t-1
-        // (4). The count allows only the 10 newer loads in flight, so it
-        // holds even if the stores complete before older loads return (on
-        // the first tiles a full drain came since). The ring is touched
-        // through assembly only: the compiler would otherwise wait for every
-        // buffer->LDS load in flight (vmcnt(0)) before each access.
-        const uint16_t *sub = wring[sl] + wave * 1024;
-        {
-            uint32_t ad[4];
+        const int b = t & 1;
+        f32x4_t acc[4][2];   // [piece of W][half of its 8 columns]
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                ad[q] = (uint32_t)(size_t)(HD_LDS void *)(sub + (l32 * 4 + (q ^ ((l32 >> 2) & 3))) * 8 + lh * 4);
-            u32x2_t wv[4];
-            asm volatile(
-                "s_waitcnt vmcnt(10)\n\t"
-                "ds_read_b64 %0, %4\n\tds_read_b64 %1, %5\n\tds_read_b64 %2, %6\n\tds_read_b64 %3, %7\n\t"
-                "s_waitcnt lgkmcnt(0)"
-                : "=v"(wv[0]), "=v"(wv[1]), "=v"(wv[2]), "=v"(wv[3])
-                : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3])
-                : "memory");
-            u32x2_t o[4];
+        for (int kb = 0; kb < 4; kb++) {   // 32 (kb / 2) + 4 (kb % 2): the columns' kp and h
+            // three accumulators by part-product order (2^-16: a2b0 a1b1 a0b2;
+            // 2^-8: a1b0 a0b1; leading: a0b0), summed smallest first at the end
+            f32x4_t as[2], am[2], al[2];
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                o[q] = (u32x2_t){pack_bf2(fmaf(c0.scale, acc[4 * q], lo_bf(wv[q][0])),
-                                          fmaf(c0.scale, acc[4 * q + 1], hi_bf(wv[q][0]))),
-                                 pack_bf2(fmaf(c0.scale, acc[4 * q + 2], lo_bf(wv[q][1])),
-                                          fmaf(c0.scale, acc[4 * q + 3], hi_bf(wv[q][1])))};
-            asm volatile(
-                "ds_write_b64 %0, %1\n\tds_write_b64 %2, %3\n\tds_write_b64 %4, %5\n\tds_write_b64 %6, %7"
-                :
-                : "v"(ad[0]), "v"(o[0]), "v"(ad[1]), "v"(o[1]), "v"(ad[2]), "v"(o[2]), "v"(ad[3]), "v"(o[3])
-                : "memory");
+            for (int nb = 0; nb < 2; nb++) as[nb] = am[nb] = al[nb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            bf16x8_t fa[2][3];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+                    fa[ks][p] = *(const bf16x8_t *)(dpl[b][p] + (kb * 16 + l16) * LT_LD + ks * 32 + lg * 8);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                const bf16x8_t *a = fa[ks];
+#pragma unroll
+                for (int i = 0; i < 6; i++)
+#pragma unroll
+                    for (int nb = 0; nb < 2; nb++) {
+                        const bf16x8_t *bb = fb[nb][ks];
+                        if (i == 0) as[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], bb[0], as[nb], 0, 0, 0);
+                        if (i == 1) am[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bb[0], am[nb], 0, 0, 0);
+                        if (i == 2) al[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bb[0], al[nb], 0, 0, 0);
+                        if (i == 3) as[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bb[1], as[nb], 0, 0, 0);
+                        if (i == 4) am[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bb[1], am[nb], 0, 0, 0);
+                        if (i == 5) as[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bb[2], as[nb], 0, 0, 0);
+                    }
+            }
+            // the next tile's down slice into the other plane buffer, under the MFMAs
+            if (kb == 0) put_down(dsplit, b ^ 1);
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[nb * 2 + kb / 2][kb % 2][e] = al[nb][e] + (am[nb][e] + as[nb][e]);
         }
-        // the sub-tile leaves as it arrived (same lanes, same offsets)
-        const __amdgpu_buffer_rsrc_t rw = lt_rsrc(c0.w, w_bytes);
-        {
-            // LDS operations of one wave complete in order, so these reads
-            // see the update's writes above
-            const uint32_t sa0 = (uint32_t)(size_t)(HD_LDS void *)(sub + lane * 8);
-            const uint32_t sa1 = (uint32_t)(size_t)(HD_LDS void *)(sub + (64 + lane) * 8);
-            u32x4_t v0, v1;
-            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                         : "=v"(v0), "=v"(v1) : "v"(sa0), "v"(sa1) : "memory");
-            __builtin_amdgcn_raw_buffer_store_b128(v0, rw, w_off(c0, 0), 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(v1, rw, w_off(c0, 1), 0, 0);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const __amdgpu_buffer_rsrc_t rw = lt_rsrc(c0.d.w, (uint32_t)((size_t)c0.d.N * c0.d.K * 2));
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            u32x4_t o;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                o[e] = pack_bf2(fmaf(c0.d.scale, acc[p][e / 2][(e % 2) * 2], lo_bf(w[p][e])),
+                                fmaf(c0.d.scale, acc[p][e / 2][(e % 2) * 2 + 1], hi_bf(w[p][e])));
+            __builtin_amdgcn_raw_buffer_store_b128(o, rw, w_off(c0, p), 0, 0);
         }
+        load_w(c2, w);
         c0 = c1;
         c1 = c2;
-        c2 = tc_next(c2, t + 3);
-        sl = sl == 2 ? 0 : sl + 1;
     };
+    // waves 4..7 run half a tile behind: one group's loads, updates and stores
+    // run beside the other group's MFMAs
+    if (wave >= 4) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (int t = tb; t < te; t += 2) {
-        step(t, DB, DA);
-        if (t + 1 < te) step(t + 1, DA, DB);
+        step(t, WA, DB, DA);
+        if (t + 1 < te) step(t + 1, WB, DA, DB);
     }
-    // no LDS-bound load may land after the block ends
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (wave < 4) asm volatile("s_barrier" ::: "memory");
 #endif
 }
 
@@ -486,78 +419,70 @@ extern "C" hd_status hd_lora_merge_gpu(hd_lora_entry *entries, size_t count, voi
             return HD_ERR_UNSUPPORTED;
         }
     }
-    // Batches. An entry's level is one past the level of the last earlier
-    // entry on the same weight (two adapters on one target merge in entry
-    // order, as the reference's loop does); levels launch in order. Within a
-    // level, the entries the streaming kernel takes (R <= 64, R % 4 == 0,
-    // K % 8 == 0, W under 2 GiB) go into one launch per (N, K, R); the others
-    // run the fp32 matrix-core kernel, one launch each.
-    struct Key {
-        int level, N, K, R;
-        bool operator<(const Key &o) const {
-            return level != o.level ? level < o.level
-                                    : (N != o.N ? N < o.N : (K != o.K ? K < o.K : R < o.R));
-        }
+    // Batches. An entry's level is one past the highest level of the earlier
+    // entries whose weights overlap its own (two adapters on one target merge
+    // in entry order, as the reference's loop does); levels launch in order.
+    // Within a level, the entries the streaming kernel takes (R <= 64, R % 4
+    // == 0, K % 8 == 0, all operands under 2 GiB) go into one launch per LM_TG
+    // of them; the others run the fp32 matrix-core kernel, one launch each.
+    struct Range {
+        uintptr_t lo, hi;
+        bool operator<(const Range &o) const { return lo < o.lo; }
     };
-    std::map<const void *, int> last;
-    std::map<Key, std::vector<LmTarget>> stream_batches;
-    std::vector<std::pair<int, size_t>> mfma_entries;   // (level, entry)
+    std::vector<Range> range(count);
+    for (size_t i = 0; i < count; i++) {
+        range[i].lo = (uintptr_t)entries[i].base_dev;
+        range[i].hi = range[i].lo + (size_t)entries[i].out_dim * entries[i].in_dim * 2;
+    }
+    std::vector<Range> sorted = range;
+    std::sort(sorted.begin(), sorted.end());
+    bool overlap = false;   // sorted by start: two ranges overlap only if two neighbours do
+    for (size_t i = 1; i < count; i++) overlap = overlap || sorted[i].lo < sorted[i - 1].hi;
+    std::vector<int> levels(count, 0);
+    std::map<int, std::vector<LmTarget>> stream_batches;   // by level
+    std::vector<std::pair<int, size_t>> mfma_entries;      // (level, entry)
     int nlevels = 0;
     for (size_t i = 0; i < count; i++) {
         hd_lora_entry *e = &entries[i];
-        auto it = last.find(e->base_dev);
-        const int level = it == last.end() ? 0 : it->second + 1;
-        last[e->base_dev] = level;
+        int level = 0;
+        for (size_t j = 0; overlap && j < i; j++)
+            if (range[j].lo < range[i].hi && range[i].lo < range[j].hi && level <= levels[j]) level = levels[j] + 1;
+        levels[i] = level;
         nlevels = level + 1 > nlevels ? level + 1 : nlevels;
         const int N = (int)e->out_dim, K = (int)e->in_dim, R = (int)e->rank;
         const float scale = e->multiplier * e->alpha / (float)e->rank;   // lora_merge.cu:54
-        const bool stream_ok = R <= 64 && R % 4 == 0 && K % 8 == 0 && (size_t)N * K * 2 < ((size_t)1 << 31);
+        const bool stream_ok = R <= 64 && R % 4 == 0 && K % 8 == 0 &&
+                               (size_t)N * K * 2 < ((size_t)1 << 31) && (size_t)N * R * 4 < ((size_t)1 << 31) &&
+                               (size_t)K * R * 4 < ((size_t)1 << 31);
         if (stream_ok)
-            stream_batches[Key{level, N, K, R}].push_back(
-                LmTarget{(uint16_t *)e->base_dev, (const float *)e->up_dev, (const float *)e->down_dev, scale});
+            stream_batches[level].push_back(LmTarget{(uint16_t *)e->base_dev, (const float *)e->up_dev,
+                                                     (const float *)e->down_dev, scale, N, K, R,
+                                                     (int)hd_cdiv(K, LT_K), (int)hd_cdiv(N, LT_N)});
         else
             mfma_entries.push_back({level, i});
-    }
-    // the batches' target lists in one small device buffer (freed after the
-    // stream has run the launches, as the reference frees its delta scratch)
-    size_t ntg = 0;
-    for (auto &b : stream_batches) ntg += b.second.size();
-    std::vector<LmTarget> host_tg;
-    host_tg.reserve(ntg);
-    for (auto &b : stream_batches) host_tg.insert(host_tg.end(), b.second.begin(), b.second.end());
-    LmTarget *dev_tg = nullptr;
-    if (ntg) {
-        if (hipMalloc((void **)&dev_tg, ntg * sizeof(LmTarget)) != hipSuccess) {
-            hd_set_error("lora: target list allocation failed");
-            return HD_ERR_OOM;
-        }
-        if (hipMemcpyAsync(dev_tg, host_tg.data(), ntg * sizeof(LmTarget), hipMemcpyHostToDevice, st) !=
-            hipSuccess) {
-            (void)hipFree(dev_tg);
-            hd_set_error("lora: target list upload failed");
-            return HD_ERR_IO;
-        }
     }
     int cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     hd_status status = HD_OK;
-    size_t off = 0;
-    auto sb = stream_batches.begin();
     for (int level = 0; level < nlevels && status == HD_OK; level++) {
-        for (; sb != stream_batches.end() && sb->first.level == level; ++sb) {
-            const int N = sb->first.N, K = sb->first.K, R = sb->first.R;
-            const int ntk = hd_cdiv(K, LT_K), nstrip = hd_cdiv(N, LT_N);
-            const long tot = (long)nstrip * ntk * (long)sb->second.size();
-            if (tot >= ((long)1 << 31)) {
-                hd_set_error("lora: batch of %zu targets has too many tiles", sb->second.size());
-                status = HD_ERR_UNSUPPORTED;
-                break;
+        const std::vector<LmTarget> tg = stream_batches.count(level) ? stream_batches[level] : std::vector<LmTarget>();
+        for (size_t i0 = 0; i0 < tg.size(); i0 += LM_TG) {
+            // under 2 GiB of W a target has less than 2^20 tiles
+            LmBatch bt;
+            bt.n = (int)(tg.size() - i0 < LM_TG ? tg.size() - i0 : LM_TG);
+            bt.total = 0;
+            for (int g = 0; g < bt.n; g++) {
+                bt.t[g] = tg[i0 + g];
+                bt.first[g] = bt.total;
+                bt.total += bt.t[g].ntk * bt.t[g].nstrip;
             }
-            lora_merge_stream_kernel<<<tot < cus ? (unsigned)tot : (unsigned)cus, 512, 0, st>>>(
-                dev_tg + off, N, K, R, ntk, nstrip, (int)tot);
-            off += sb->second.size();
+            for (int g = bt.n; g < LM_TG; g++) {   // never read as targets
+                bt.t[g] = bt.t[0];
+                bt.first[g] = bt.total;
+            }
+            lora_merge_stream_kernel<<<(unsigned)(bt.total < cus ? bt.total : cus), 512, 0, st>>>(bt);
         }
         for (auto &m : mfma_entries) {
             if (m.first != level || status != HD_OK) continue;
@@ -574,9 +499,6 @@ extern "C" hd_status hd_lora_merge_gpu(hd_lora_entry *entries, size_t count, voi
             status = HD_ERR_RUNTIME;
         }
     }
-    if (dev_tg) {
-        (void)hipStreamSynchronize(st);
-        (void)hipFree(dev_tg);
-    }
+    if (!stream_batches.empty()) (void)hipStreamSynchronize(st);
     return status;
 }
