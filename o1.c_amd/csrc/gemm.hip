@@ -1310,7 +1310,8 @@ static void launch_kg(GemmArgs &g, int P, void *ws) {
 // 64-deep K tile of one block per CU (warm and cold operands of the block's and
 // the vision tower's shapes), and per round what it costs beside its
 // K tiles:
-//   256x256 1.50, 192x256 1.32, old 128x128 0.45 alone and 0.90 for two per CU;
+//   256x256 1.50, 192x256 1.32, old 128x128 0.58 alone (0.45 to 0.75 as the weight
+//   is warm or cold) and 0.90 for two per CU;
 //   K-group tiles 256x128 0.90, 192x128 0.66, 128x128 0.50, 64x128 0.345,
 //   64x64 0.21; the last two fit a CU twice, at 1.7-2 times the time.
 // The 128-wide families take 15 % longer on SwiGLU's two weights and, unsplit,
@@ -1362,7 +1363,7 @@ static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t 
         const long full = tiles / slots, rem = tiles % slots;
         if (occ == 2 && swiglu && tiles <= 256) return;   // one wave per SIMD: 0.83 on two cold weights
         const double usf = occ == 2 ? us2 : us1;
-        auto round = [&](long n) { return n <= 256 ? us1 : us1 * 1.6 + (us2 - us1 * 1.6) * (n - 256) / 256; };
+        auto round = [&](long n) { return n <= 256 ? us1 : us2 * (0.8 + 0.2 * (n - 256) / 256); };
         if (rem && P > 1)
             offer(fam, P, 4.0 + full * nk * usf + (nk + P - 1) / P * (full || occ == 1 ? usf : 1.3 * usf) +
                               merge_us(rem, P, bm, bna));
@@ -1376,7 +1377,7 @@ static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t 
     };
     if (K % 64 == 0) {
         const size_t s = qkv ? 2 : 0;
-        big(5, 128, 128, 2, swiglu ? 0.55 : 0.45, swiglu ? 1.10 : 0.90, s * 128 * 128);
+        big(5, 128, 128, 2, 0.58, swiglu ? 1.10 : 0.90, s * 128 * 128);
         big(6, 192, 256, 1, 1.32, 1.32, s * 192 * 256);
         big(7, 256, 256, 1, 1.50, 1.50, s * 256 * 256);
     }
