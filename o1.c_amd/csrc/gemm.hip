@@ -1310,8 +1310,9 @@ static void launch_kg(GemmArgs &g, int P, void *ws) {
 // 64-deep K tile of one block per CU (warm and cold operands of the block's and
 // the vision tower's shapes), and per round what it costs beside its
 // K tiles:
-//   256x256 1.50, 192x256 1.32, old 128x128 0.58 alone (0.45 to 0.75 as the weight
-//   is warm or cold) and 0.90 for two per CU;
+//   256x256 1.50, 192x256 1.32, old 128x128 0.90 for two per CU and 0.58 alone
+//   (0.45 warm to 0.75 cold; 0.45 where the operands are under 9 MB and can still
+//   be in the caches: there it also sums in the order of the SwiGLU kernel);
 //   K-group tiles 256x128 0.90, 192x128 0.66, 128x128 0.50, 64x128 0.345,
 //   64x64 0.21; the last two fit a CU twice, at 1.7-2 times the time.
 // The 128-wide families take 15 % longer on SwiGLU's two weights and, unsplit,
@@ -1377,7 +1378,7 @@ static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t 
     };
     if (K % 64 == 0) {
         const size_t s = qkv ? 2 : 0;
-        big(5, 128, 128, 2, 0.58, swiglu ? 1.10 : 0.90, s * 128 * 128);
+        big(5, 128, 128, 2, foot < 9e6 ? 0.45 : 0.58, swiglu ? 1.10 : 0.90, s * 128 * 128);
         big(6, 192, 256, 1, 1.32, 1.32, s * 192 * 256);
         big(7, 256, 256, 1, 1.50, 1.50, s * 256 * 256);
     }
