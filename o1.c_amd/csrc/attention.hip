@@ -528,9 +528,13 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         lin -= a.n_whole + a.n_chunks;
         causal_unit = true;
     } else if (lin >= a.n_whole) {
-        item = lin - a.n_whole;
-        chunk = item % a.split;
-        lin = a.n_whole + item / a.split;
+        // neighbouring units of one chunk on an XCD: they share its K / V^T in
+        // L2 (2371 tokens, all units split: 103.7 -> 100.2 us; others equal)
+        const int c = fa_xcd_remap(lin - a.n_whole, a.n_chunks), n_tail = a.n_chunks / a.split;
+        chunk = c / n_tail;
+        const int t = c - chunk * n_tail;
+        item = t * a.split + chunk;
+        lin = a.n_whole + t;
     } else {
         lin = fa_xcd_remap(lin, a.n_whole);
     }
