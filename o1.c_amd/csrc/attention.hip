@@ -932,7 +932,9 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
 // KS waves share each 32 queries, every KS-th key tile each, and merge at the
 // end: the tower's 576 rows are 80 blocks of 128 queries, so with KS = 2 its
 // 144 blocks of 64 take half the key tiles each on otherwise idle CUs.
-// @V72@
+// Bound by latency at 576 rows (9 key tiles): 14.8 us with heads padded to 128,
+// and 4.5 more to take the padding out again -> 10.9 us; three images, KS = 1:
+// 13.0 us.
 // ---------------------------------------------------------------------------
 struct FaV72Args {
     const uint16_t *q, *k, *vt;
@@ -1311,7 +1313,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     //    full ones in the same grid, so that no block mixes both kinds
     //    (S = 4239, 142 causal rows, one masked 4-wave launch: 314 -> 270 us;
     //    S = 16499: 4080 -> 3630; 2 x 1101 rows: equal), or
-    //  * there is a dense mask: its values are prefetched as 8-byte pieces
+    //  * there is a dense mask: its values are prefetched as 16-byte pieces
     //    under the MFMA phase, where a tile needs them (4-wave blocks
     //    with 2-byte loads, causal text rows above zeros: S = 300 26.6 ->
     //    25.6 us, 1209 199 -> 57, 4239 1937 -> 318; equal

@@ -38,7 +38,7 @@ __device__ __forceinline__ float wsum(float v) {
 // start off the 128-byte lines, so every 64-deep K tile of a row touches two
 // lines (17.0 -> 29 us at 576 rows); on rows of 4352 each touches one. As a
 // launch of its own the copy took 5.4 us; behind the LayerNorm that runs before
-// fc1 it costs @RP@ us and leaves the weight in the caches for fc2.
+// fc1 it costs 2.9 us and leaves the weight in the caches for fc2.
 struct Repitch {
     const uint16_t *src;
     uint16_t *dst;
@@ -223,7 +223,7 @@ __global__ void v_cos_sin_kernel(const uint16_t *__restrict__ rot, float *__rest
 // One block per (64-row tile, image and head) stages the tile's q, k and v
 // slices in LDS; 16-byte loads and stores. D = 72: rotary partners lie 36
 // columns away, so a lane works on groups of 4.
-// One launch's latency bounds it (144 blocks at 576 rows): 8.1 -> @ROPE@ us with
+// One launch's latency bounds it (144 blocks at 576 rows): 8.1 -> 7.2 us with
 // the tables read 16 bytes at a time and rows of 72 instead of 128.
 template <int DP>
 __global__ __launch_bounds__(256) void v_qkv_rope_kernel(

@@ -7,13 +7,15 @@ pytestmark = pytest.mark.gpu
 
 # few rows (1, 2, 16 | 17, 32: two row tiles; K below and off the 8 waves' 512),
 # 64x64 (ragged M and N, N % 64 = 8, odd tile counts, 8 chunks), 64x128 alone and
-# in 4 chunks, 128x128 in 8, 192x128, SwiGLU on 64x64, 128x128 and 192x128
+# in 4 chunks, 128x128 in 8, 192x128, SwiGLU on 64x64, 128x128 and 192x128, K
+# with a short last 64
 @pytest.mark.parametrize("M,N,K,epi", [
     (1, 4096, 256, "bias"), (2, 4096, 4096, "bias"), (16, 72, 64, "none"), (5, 1024, 3072, "res"), (16, 320, 576, "swiglu"),
     (17, 4096, 1088, "bias"), (32, 200, 4096, "res"), (70, 1000, 4032, "bias"), (64, 264, 4160, "res"),
     (129, 4104, 1088, "none"), (300, 4096, 4096, "bias"), (94, 4096, 4096, "res"), (94, 4096, 12288, "res"),
     (1100, 4096, 4096, "none"), (130, 6144, 4096, "res"), (70, 4096, 4096, "swiglu"), (40, 1024, 512, "swiglu"),
-    (94, 12288, 4096, "swiglu"), (150, 12288, 4096, "swiglu")])
+    (94, 12288, 4096, "swiglu"), (150, 12288, 4096, "swiglu"),
+    (3, 72, 72, "bias"), (33, 264, 200, "none"), (576, 1152, 4304, "bias"), (2371, 1024, 1096, "bias")])
 def test_small_gemms_vs_fp32(pkg, lib, dev, M, N, K, epi):
     """One rounding of the product, then the epilogue's own. Sums in another
     order move a product by ~1e-7 sqrt(K) relative, so a rounding flips for
