@@ -29,6 +29,7 @@
 #include <math.h>
 
 #include "hd_common.hpp"
+#include "flash_rows.hpp"
 #include "../../include/hd_hip.h"
 #include "../../include/hd_sdpa.h"
 
@@ -94,16 +95,6 @@ __global__ __launch_bounds__(64) void fa_mask_bits_kernel(const uint16_t *mask, 
         dead[at] = (uint8_t)d;
     }
 }
-
-// Row tiling of the ping-pong kernel's units: per (batch, kv head) the rows
-// [row0, row0 + 256 * ntile + left) are `ntile` whole 256-row tiles of every
-// query head of the group, then the `left` rows after them. The left-over
-// rows of up to `hp` = 256 / left heads share one unit (they read the same
-// keys), so 1024 + 1 rows cost 4 + 1/4 tiles per head and not 5. Units are
-// numbered whole tiles first.
-struct FaRows {
-    int row0, ntile, left, hp;
-};
 
 struct FaArgs {
     const uint16_t *q;     // [B,Hq,S,D]
@@ -462,42 +453,6 @@ __device__ __forceinline__ float xor16_32_sum(float v) {
     return xor32_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
-// Unit `lin` of a row tiling: batch, kv head, first row and first query head
-// of the group; left: rows per head of a left-over unit, 0 for a whole tile.
-struct FaUnit {
-    int b, hk, qbase, g0, left;
-};
-__device__ __forceinline__ FaUnit fa_unit(const FaArgs &a, const FaRows &r, int batch, int lin) {
-    const int group = a.Hq / a.Hkv, n_whole_tiles = batch * a.Hkv * r.ntile * group;
-    FaUnit u;
-    int bh;
-    if (lin < n_whole_tiles) {   // heads of a group are neighbours: they share K / V^T in L2
-        u.g0 = lin % group;
-        lin /= group;
-        u.qbase = r.row0 + (lin % r.ntile) * 256;
-        bh = lin / r.ntile;
-        u.left = 0;
-    } else {
-        lin -= n_whole_tiles;
-        const int per = (group + r.hp - 1) / r.hp;
-        u.g0 = (lin % per) * r.hp;
-        u.qbase = r.row0 + r.ntile * 256;
-        bh = lin / per;
-        u.left = r.left;
-    }
-    u.hk = bh % a.Hkv;
-    u.b = bh / a.Hkv;
-    return u;
-}
-// Query row and head of row i (0..255) of a unit; row = INT_MAX where it has none.
-__device__ __forceinline__ int2 fa_unit_row(const FaArgs &a, const FaUnit &u, int i) {
-    const int group = a.Hq / a.Hkv;
-    if (u.left == 0) return make_int2(u.qbase + i, u.hk * group + u.g0);
-    const int k = i / u.left, hp = 256 / u.left;
-    if (k >= hp || u.g0 + k >= group) return make_int2(0x7fffffff, u.hk * group + u.g0);
-    return make_int2(u.qbase + i % u.left, u.hk * group + u.g0 + k);
-}
-
 // MODE FA_PLAIN: S % 64 == 0, every row sees every key, tiles of every head by
 // themselves (the row bookkeeping of the other modes costs it 1-7 %, more than
 // sharing left-over rows gives). FA_CAUSAL: any S, and
@@ -556,21 +511,23 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         // vector loads and make everything below per-lane)
         FaRows rows = a.full;
         if (MODE == FA_CAUSAL && causal_unit) rows = a.causal;
-        FaUnit un = fa_unit(a, rows, a.batch, lin);
+        const int group = a.Hq / a.Hkv;
+        FaUnit un = fa_unit(rows, a.batch, a.Hkv, group, lin);
         un.b = __builtin_amdgcn_readfirstlane(un.b);
         un.hk = __builtin_amdgcn_readfirstlane(un.hk);
         un.qbase = __builtin_amdgcn_readfirstlane(un.qbase);
         un.g0 = __builtin_amdgcn_readfirstlane(un.g0);
         un.left = __builtin_amdgcn_readfirstlane(un.left);
+        un.hp = __builtin_amdgcn_readfirstlane(un.hp);
         b = un.b;
         hk = un.hk;
         qbase = un.qbase;
         q0 = qbase + (un.left ? 0 : wave * 32);   // lowest row of this wave
 #pragma unroll
         for (int qq = 0; qq < 2; qq++) {
-            const int2 rh = fa_unit_row(a, un, wave * 32 + qq * 16 + l16);
-            my_q[qq] = rh.x;
-            my_h[qq] = rh.y;
+            const FaRowHead rh = fa_unit_row(un, group, wave * 32 + qq * 16 + l16);
+            my_q[qq] = rh.row;
+            my_h[qq] = rh.head;
         }
         if (qbase < a.ar_len) {
             const int last_row = qbase + (un.left ? un.left : BQ) - 1;
@@ -1197,11 +1154,12 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaArgs a, int n_tail) {
     }
     int b, hq, my_q;
     if constexpr (SHARED) {
-        const FaUnit un = fa_unit(a, a.full, a.batch, a.n_whole + tu);
-        const int2 rh = fa_unit_row(a, un, row);
+        const int group = a.Hq / a.Hkv;
+        const FaUnit un = fa_unit(a.full, a.batch, a.Hkv, group, a.n_whole + tu);
+        const FaRowHead rh = fa_unit_row(un, group, row);
         b = un.b;
-        hq = rh.y;
-        my_q = rh.x;
+        hq = rh.head;
+        my_q = rh.row;
     } else {
         const int nqt = (a.q_row_end - a.q_row_begin + BQ - 1) / BQ, group = a.Hq / a.Hkv;
         int lin = a.n_whole + tu;
@@ -1327,19 +1285,11 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     a.full = a.causal = {};
     if (pp && !plain) {
         if (prefix) a.q_row_begin = ar_len;   // the causal rows are units of their own
-        auto rows_of = [&](int row0, int rows, bool share) {
-            FaRows r = {row0, rows / BQ, rows % BQ, 1};
-            if (r.left && share) r.hp = BQ / r.left < group ? BQ / r.left : group;
-            return r;
-        };
-        auto count = [&](const FaRows &r) {
-            return batch * hkv * (r.ntile * group + (r.left ? (group + r.hp - 1) / r.hp : 0));
-        };
-        a.full = rows_of(a.q_row_begin, q_row_end - a.q_row_begin, !mask);
-        units = count(a.full);
+        a.full = fa_rows_of(a.q_row_begin, q_row_end - a.q_row_begin, group, !mask);
+        units = fa_rows_units(a.full, batch, hkv, group);
         if (prefix) {
-            a.causal = rows_of(0, ar_len, false);
-            n_causal = count(a.causal);
+            a.causal = fa_rows_of(0, ar_len, group, false);
+            n_causal = fa_rows_units(a.causal, batch, hkv, group);
         }
     } else {
         units = batch * hq * ((q_row_end - a.q_row_begin + BQ - 1) / BQ);

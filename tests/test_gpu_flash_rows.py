@@ -71,3 +71,55 @@ def test_make_vt_bytes(pkg, lib, dev, S, off):
     want = torch.zeros(BH, D, sp, dtype=torch.bfloat16, device=dev)
     want[:, :, col[:S]] = v.view(BH, S, D).transpose(1, 2)
     assert torch.equal(vt, want)
+
+
+# S % 256 of 9, 44, 64 and 128 rows left over, one round of units and (32 heads of
+# 2348 keys) one and a part, split over the keys; mask values in every row
+@pytest.mark.parametrize("kind", ["random", "causal"])
+@pytest.mark.parametrize("Hq,Hkv,S", [(8, 2, 265), (8, 2, 300), (8, 2, 320), (8, 2, 364), (4, 1, 384), (8, 2, 1289),
+                                      (32, 8, 2348)])
+def test_dense_mask_on_left_over_rows(pkg, lib, dev, Hq, Hkv, S, kind):
+    """A dense mask with values in the last S % 256 rows too, workspace given (tile
+    bits and key split on). Bounds as above; every row of every head is compared."""
+    print(f"flash dense {kind} Hq={Hq} Hkv={Hkv} S={S}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn(1, h, S, D, generator=g, device=dev).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    if kind == "random":
+        mask = (torch.randn(S, S, generator=g, device=dev) * 3).to(torch.bfloat16)
+    else:
+        mask = torch.zeros(S, S, dtype=torch.bfloat16, device=dev).masked_fill_(
+            torch.ones(S, S, dtype=torch.bool, device=dev).triu(1), torch.finfo(torch.bfloat16).min)
+    vt = torch.empty(lib.hd_flash_vt_bytes(1, Hkv, S) // 2, dtype=torch.bfloat16, device=dev)
+    lib.hd_flash_make_vt(pkg.ptr(v), pkg.ptr(vt), Hkv, S)
+    out = torch.full((S, Hq, D), float("nan"), dtype=torch.bfloat16, device=dev)
+    w = torch.empty(lib.hd_flash_ws_bytes(), dtype=torch.uint8, device=dev)
+    assert lib.hd_flash_attention_ws(pkg.ptr(q), pkg.ptr(k), pkg.ptr(vt), pkg.ptr(mask), pkg.ptr(out), 1, Hq, Hkv, S, D,
+                                     0, D ** -0.5, 1, pkg.ptr(w), w.numel()) == 0
+    ref = attend(q[0], k[0], v[0], 0, mask)
+    got = out.transpose(0, 1).float()
+    per_row = (got - ref).norm(dim=-1) / ref.norm(dim=-1)
+    assert float((got - ref).norm() / ref.norm()) < 5e-3
+    assert float(per_row.max()) < 3e-2, divmod(int(per_row.argmax()), S)
+
+
+@pytest.mark.parametrize("B,S,ar", [(2, 1101, 76), (1, 2371, 114), (1, 1283, 1), (1, 1409, 300), (1, 2305, 0)])
+def test_causal_prefix_repeats_bit_for_bit(pkg, lib, dev, B, S, ar):
+    """One unit stores a row, so a call repeats itself exactly whatever order its
+    blocks run in; scores of 8 sigma move the running maximum in many tiles."""
+    print(f"flash repeat B={B} S={S} ar={ar}", flush=True)
+    Hq, Hkv = 32, 8
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn(B, h, S, D, generator=g, device=dev).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    q = (q * 8).to(torch.bfloat16)
+    vt = torch.empty(lib.hd_flash_vt_bytes(B, Hkv, S) // 2, dtype=torch.bfloat16, device=dev)
+    lib.hd_flash_make_vt(pkg.ptr(v), pkg.ptr(vt), B * Hkv, S)
+    w = torch.empty(lib.hd_flash_ws_bytes(), dtype=torch.uint8, device=dev)
+    outs = [torch.full((B, S, Hq * D), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(4)]
+    for o in outs:
+        assert lib.hd_flash_attention_ws(pkg.ptr(q), pkg.ptr(k), pkg.ptr(vt), None, pkg.ptr(o), B, Hq, Hkv, S, D, ar,
+                                         D ** -0.5, 1, pkg.ptr(w), w.numel()) == 0
+    for o in outs[1:]:
+        assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
+    ref = attend(q[0], k[0], v[0], ar, None)
+    got = outs[0][0].view(S, Hq, D).transpose(0, 1).float()
+    assert float((got - ref).norm() / ref.norm()) < 5e-3
