@@ -825,6 +825,14 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         wait_next(ld);
         fa_barrier();
     }
+    // The loop's speed depends on where it starts in the 32-byte instruction
+    // fetch windows: 12 or 16 bytes past one is 1-2 % faster than most other
+    // places (all 16 places of a word tried: 12 and 16 at 3490 us for 16640 keys,
+    // the rest 3520-3580; at 28, where it stood by chance, 3624 against 3588 in
+    // turn, 4352 keys x 2 520.2 against 515.6, 1152 keys 32.0 against 31.4). The
+    // code from here to the loop's first instruction ends 20 bytes past such a
+    // window, so 6 words more put it at 12 (a test reads it from the built code).
+    if constexpr (MODE == FA_PLAIN) asm volatile(".p2align 5\n\t.rept 6\n\ts_nop 0\n\t.endr");
     for (int t = t_begin + 1; t < t_end; t++) {
         softmax(t - 1);
         pin_softmax();
