@@ -1055,12 +1055,12 @@ template <int EPI> static void launch_skinny(GemmArgs &g) {
 // shapes the MFMA kernels do not take (K % 64, N % 8, misaligned).
 // ---------------------------------------------------------------------------
 __global__ void gemm_ref_kernel(const uint16_t *x, const uint16_t *w, const uint16_t *bias,
-                                uint16_t *y, int M, int N, int K) {
+                                uint16_t *y, int M, int N, int K, int lda, int ldb) {
     int n = blockIdx.x * 16 + (threadIdx.x & 15);
     int m = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (m >= M || n >= N) return;
     float acc = 0.f;
-    for (int k = 0; k < K; k++) acc += bf2f(x[(size_t)m * K + k]) * bf2f(w[(size_t)n * K + k]);
+    for (int k = 0; k < K; k++) acc += bf2f(x[(size_t)m * lda + k]) * bf2f(w[(size_t)n * ldb + k]);
     if (bias) acc += bf2f(bias[n]);
     y[(size_t)m * N + n] = f2bf(acc);
 }
@@ -1677,7 +1677,7 @@ extern "C" void hd_linear_reference(const void *x, const void *w, const void *bi
     }
     dim3 grid(hd_cdiv(N, 16), hd_cdiv(M, 16));
     gemm_ref_kernel<<<grid, 256, 0, hd_stream()>>>((const uint16_t *)x, (const uint16_t *)w,
-                                                   (const uint16_t *)bias, (uint16_t *)y, M, N, K);
+                                                   (const uint16_t *)bias, (uint16_t *)y, M, N, K, K, K);
     hd_check_launch("linear_reference");
 }
 
@@ -1737,23 +1737,43 @@ void hd_linear_gelu(const void *x, const void *w, const void *bias, void *y, int
     hd_check_launch("linear_gelu");
 }
 
-void hd_linear_strided(const void *x, int lda, const void *w, int ldb, const void *bias, void *y, int M, int N,
-                       int K, void *ws, int64_t ws_bytes) {
-    if (!x || !w || !bias || !y || M <= 0 || N <= 0 || K % 64 == 0 || lda < K || ldb < K || lda % 8 || ldb % 8 ||
-        !linear_ok(x, w, y, M, N, K) || ((uintptr_t)bias | (uintptr_t)ws) % 16 ||
-        ((size_t)M * lda | (size_t)N * ldb) >= ((size_t)1 << 30)) {
-        snprintf(hd_cuda_errbuf(), 512, "linear_strided: bad args");
-        return;
-    }
+// One piece of rows; the caller has checked the rows against 32-bit offsets.
+static void linear_strided_piece(const uint16_t *x, int lda, const uint16_t *w, int ldb, const uint16_t *bias,
+                                 uint16_t *y, int M, int N, int K, void *ws, int64_t ws_bytes) {
     GemmArgs g = {};
-    g.A = (const uint16_t *)x;
-    g.B[0] = g.B[1] = g.B[2] = (const uint16_t *)w;
+    g.A = x;
+    g.B[0] = g.B[1] = g.B[2] = w;
     g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
-    g.C = (uint16_t *)y;
-    g.bias = (const uint16_t *)bias;
+    g.C = y;
+    g.bias = bias;
     g.M = M; g.N = N; g.K = K; g.ldc = N;
     g.lda = lda; g.ldb = ldb;
     gemm_launch(EPI_BIAS, g, ws, ws ? ws_bytes : 0);
+}
+
+void hd_linear_strided(const void *x, int lda, const void *w, int ldb, const void *bias, void *y, int M, int N,
+                       int K, void *ws, int64_t ws_bytes) {
+    if (!x || !w || !bias || !y || M <= 0 || N <= 0 || K <= 0 || lda < K || ldb < K) {
+        snprintf(hd_cuda_errbuf(), 512, "linear_strided: bad args");
+        return;
+    }
+    const uint16_t *xp = (const uint16_t *)x, *wp = (const uint16_t *)w, *bp = (const uint16_t *)bias;
+    uint16_t *yp = (uint16_t *)y;
+    // rows whose operand stays under 2 GiB, in whole row tiles
+    const int rows = ((int)((((size_t)1 << 30) - 1) / lda) - 256) / 256 * 256;
+    if (!g_use_production || K % 64 == 0 || lda % 8 || ldb % 8 || rows <= 0 || (uintptr_t)bias % 16 ||
+        !linear_ok(x, w, y, M < rows ? M : rows, N, K) || (size_t)N * ldb >= ((size_t)1 << 30)) {
+        // as hd_linear: the reference kernel, the bias added to the rounded product
+        gemm_ref_kernel<<<dim3(hd_cdiv(N, 16), hd_cdiv(M, 16)), 256, 0, hd_stream()>>>(xp, wp, nullptr, yp, M, N, K,
+                                                                                    lda, ldb);
+        bias_add_kernel<<<hd_cdiv((size_t)M * N, 256), 256, 0, hd_stream()>>>(bp, yp, M, N);
+        hd_check_launch("linear_strided");
+        return;
+    }
+    if ((uintptr_t)ws % 16) ws = nullptr;
+    for (int m = 0; m < M; m += rows)
+        linear_strided_piece(xp + (size_t)m * lda, lda, wp, ldb, bp, yp + (size_t)m * N, M - m < rows ? M - m : rows, N,
+                             K, ws, ws_bytes);
     hd_check_launch("linear_strided");
 }
 

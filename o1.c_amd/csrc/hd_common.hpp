@@ -19,7 +19,8 @@ int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *
 // y = bf16(gelu(bf16(bf16(x . w^T) + bias))), tanh or erf form, rows of ldc (gemm.hip).
 void hd_linear_gelu(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, bool erf,
                     void *ws, int64_t ws_bytes, int ldc);
-// hd_linear_ws over operand rows of lda and ldb elements, K % 8 == 0 but not K % 64 (gemm.hip).
+// hd_linear_ws over operand rows of lda and ldb elements (gemm.hip): the K-group kernels where K % 8 == 0 but
+// not K % 64, in pieces of rows past 2 GiB of x; the reference kernel otherwise.
 void hd_linear_strided(const void *x, int lda, const void *w, int ldb, const void *bias, void *y, int M, int N,
                        int K, void *ws, int64_t ws_bytes);
 // Attention of the vision tower: q, k [batch * heads, seq, 72], vt [batch * heads, 72, round_up(seq, 64)]
