@@ -1271,31 +1271,6 @@ static void launch_ms(GemmArgs &g, void *ws = nullptr, int64_t ws_bytes = 0) {
     }
 }
 
-// Tile configuration per shape. The 8-wave 256-wide kernels are the main
-// path; a 192-row tile is taken when it quantises the grid onto the 256 CUs
-// better (M = 8704 without a workspace: 34 -> 46 row tiles), and 128x128
-// tiles for grids too small to fill the chip with 256x256 tiles.
-// Estimated time (s) of a tile family: rounds of resident blocks, each the
-// time of `occ` tiles on a CU (2*BM*BNA*K flops at ~half the per-CU peak x
-// the family's relative per-flop efficiency: 192-row tiles 8-18 % slower
-// per flop than 256-row ones, 128x128 tiles at two per CU ~20 %); with the
-// tail split the last round is one chunk plus the merge (the fp32 partials
-// written and read once at HBM rate, and a launch).
-static double tile_cost(long units, int occ, int BM, int BNA, int K, double eff, int P) {
-    const long slots = (long)(gemm_slots() > 0 ? gemm_slots() : 256) * occ;
-    const double rate = 2.5e15 / 256 * 0.5 * eff;
-    const double t_round = occ * 2.0 * BM * BNA * (double)K / rate;
-    const long full = units / slots, rem = units % slots;
-    double t = full * t_round;
-    if (rem) {
-        if (P > 1)
-            t += t_round / P + (double)rem * P * BM * BNA * 8.0 / 8e12 + 4e-6;
-        else
-            t += t_round;
-    }
-    return t;
-}
-
 template <int BM, int BN, int NS, int EPI, int OCC>
 static void launch_kg(GemmArgs &g, int P, void *ws) {
     constexpr int BN_OUT = EPI == EPI_SWIGLU ? BN / 2 : BN;
@@ -1316,23 +1291,27 @@ static void launch_kg(GemmArgs &g, int P, void *ws) {
                 <<<hd_cdiv((size_t)n_tail * BM * (BN_OUT / 4), 256), 256, 0, hd_stream()>>>(g, (int)n_tail);
     }
 }
-// Choice for grids of at most two rounds of 256 x 256 tiles. Measured us per
-// 64-deep K tile of one block per CU (warm and cold operands of the block's and
-// the vision tower's shapes), and per round what it costs beside its
-// K tiles:
-//   256x256 1.50, 192x256 1.32, old 128x128 0.90 for two per CU and 0.58 alone
-//   (0.45 warm to 0.75 cold; 0.45 where the operands are under 9 MB and can still
-//   be in the caches: there it also sums in the order of the SwiGLU kernel);
-//   K-group tiles 256x128 0.90, 192x128 0.66, 128x128 0.50, 64x128 0.345,
-//   64x64 0.21; the last two fit a CU twice, at 1.7-2 times the time.
-// The 128-wide families take 15 % longer on SwiGLU's two weights and, unsplit,
-// past K = 8192; the old 128 x 128 tiles 30 % longer when every tile is split.
-// A split adds the merge launch and its partials, written and read at 8 TB/s
-// (L2 and the cache behind it hold most). Tiles this small re-read the
-// operands: once these do not fit the L2s (32 MB in all) the re-reads are
-// served at 16-18 TB/s.
-struct SmallPick {
-    int fam, P;   // fam 0..4: kKg; 5 old 128x128, 6 192x256, 7 256x256
+// Tile choice: the family and K split with the lowest predicted time. Prices in
+// us per 64-deep K tile of a round of blocks (one block per CU), and what a
+// round costs beside its K tiles:
+//   ring 256x256 1.48, 192x256 1.26, 128x128 0.89 for two blocks per CU (SwiGLU
+//   0.95) and 0.56 for one;
+//   K groups 256x128 0.85, 192x128 0.64, 128x128 0.48, 64x128 0.365, 64x64 0.20;
+//   the last two fit a CU twice, at 1.7-2 times the time.
+// A split adds the merge launch (4.1 us, 6.1 for the QKV epilogue) and its
+// partials, written and read at 7.2 TB/s. Tiles of 128 columns and less re-read
+// the operands: once these do not fit the L2s (32 MB in all) the re-reads are
+// served at 14 (K groups) and 19 TB/s.
+// The numbers are a fit to every family and split forced at ~1400 shapes, M = 34 to
+// 33792, cold weights (the linears of block, tower, mergers and embedders): the
+// choice is 0.4 % off the fastest up to two rounds of 256 x 256 tiles and 0.6 %
+// above (two sets of prices, split at that size, were 1.5 and 1.0 % off, and more at
+// single shapes: 6978 x 3072 x 4096 164 -> 151 us, 310 x 4608 x 4608 37.8 -> 30,
+// 2567 x 4096 x 12288 262 -> 242, 20815 x 4096 x 4096 582 -> 562). With its
+// operands still in the caches the lone ring 128 x 128 block would be 7 % faster
+// than the K-group one; cold it is 13-20 % slower, and a model's weights are cold.
+struct TilePick {
+    int fam, P;   // fam 0..4: kKg; 5 ring 128x128, 6 ring 192x256, 7 ring 256x256
     double us;
 };
 struct KgFam {
@@ -1340,65 +1319,79 @@ struct KgFam {
     double us, fixed;
     bool twice;
 };
-constexpr KgFam kKg[5] = {{64, 64, 0.21, 1.5, true}, {64, 128, 0.345, 1.5, true}, {128, 128, 0.50, 1.5, false},
-                          {192, 128, 0.66, 3.0, false}, {256, 128, 0.90, 3.0, false}};
-static SmallPick pick_small(int M, int N, int K, bool swiglu, bool qkv, int64_t ws_bytes) {
-    SmallPick best = {7, 1, 1e30};
+constexpr KgFam kKg[5] = {{64, 64, 0.20, 1.2, true}, {64, 128, 0.365, 1.2, true}, {128, 128, 0.48, 1.2, false},
+                          {192, 128, 0.64, 3.3, false}, {256, 128, 0.85, 3.3, false}};
+// ring_only: the 256-wide ring families (operands of 2 GiB and more)
+static TilePick pick_tiles(int M, int N, int K, bool swiglu, bool qkv, int64_t ws_bytes, bool ring_only = false) {
+    TilePick best = {7, 1, 1e30};
     const int nk = (K + 63) / 64;
+    const long cus = gemm_slots() > 0 ? gemm_slots() : 256;
     const double foot = 2.0 * K * ((double)M + (swiglu ? 2.0 : 1.0) * N);
-    auto merge_us = [&](double tiles, int P, int bm, int bn) { return 5.0 + tiles * P * bm * bn * 8.0 / 8e6; };
+    auto merge_us = [&](double tiles, int P, int bm, int bn) { return (qkv ? 6.1 : 4.1) + tiles * P * bm * bn * 8.0 / 7.2e6; };
     auto offer = [&](int fam, int P, double us) {
-        if (fam < 6) us *= 1.03;   // near ties go to the large tiles
+        if (fam < 6) us *= 1.02;   // near ties go to the large tiles
         if (us < best.us) best = {fam, P, us};
     };
-    for (int f = qkv ? 1 : 0; f < 5; f++) {
+    auto tiles_of = [&](int bm, int bn) {
+        const int out = swiglu ? bn / 2 : bn;
+        return (long)((M + bm - 1) / bm) * ((N + out - 1) / out);
+    };
+    // the K groups were measured up to two rounds of 256 x 256 tiles, and K % 64
+    // runs on them only
+    const bool groups = !ring_only && (tiles_of(256, 256) <= 2 * cus || K % 64);
+    for (int f = qkv ? 1 : 0; groups && f < 5; f++) {
         const KgFam &k = kKg[f];
-        const long tiles = (long)((M + k.bm - 1) / k.bm) * ((N + (swiglu ? k.bn / 2 : k.bn) - 1) / (swiglu ? k.bn / 2 : k.bn));
+        const long tiles = tiles_of(k.bm, k.bn);
         for (int P = 1; P <= 8; P++) {
-            if (P > 1 && (nk / P < 4 || tiles * P > (k.twice ? 512 : 256) ||
+            if (P > 1 && (nk / P < 4 || tiles * P > (k.twice ? 2 * cus : cus) ||
                           (int64_t)tiles * P * k.bm * k.bn * 4 > ws_bytes))
                 break;
-            const double u = (double)tiles * P / 256;
-            const double rounds = u <= 1 ? 1.0 : !k.twice ? (double)((tiles * P + 255) / 256)
-                                                 : u <= 2 ? 1.4 + 0.3 * u : 1.1 * u;
-            double t = 3.0 + rounds * (k.fixed + ((nk + P - 1) / P) * k.us * (swiglu || K > 8192 ? 1.15 : 1.0));
+            const double u = (double)tiles * P / cus;
+            const double rounds = u <= 1 ? 1.0 : !k.twice ? (double)((tiles * P + cus - 1) / cus)
+                                                 : u <= 2 ? 1.35 + 0.32 * u : 1.25 * u;
+            double t = 3.3 + rounds * (k.fixed + ((nk + P - 1) / P) * k.us);
             const double reread = tiles * (double)(k.bm + k.bn) * K * 2;
-            if (foot > 32e6 && reread / 16e6 > t) t = reread / 16e6;
+            if (foot > 32e6 && reread / 14.3e6 > t) t = reread / 14.3e6;
             offer(f, P, t + (P > 1 ? merge_us(tiles, P, k.bm, k.bn) : 0.0));
         }
     }
-    auto big = [&](int fam, int bm, int bna, int occ, double us1, double us2, size_t stage) {
-        const int bn = swiglu ? bna / 2 : bna;
-        const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn), slots = 256L * occ;
+    // one: us per K tile of a round of one block per CU, two: of two per CU
+    auto ring = [&](int fam, int bm, int bna, int occ, double one, double two, size_t stage) {
+        const long tiles = tiles_of(bm, bna), slots = cus * occ;
         const int P = tail_split_of(tiles, nk, (size_t)bm * bna * 4, ws_bytes, stage, occ);
         const long full = tiles / slots, rem = tiles % slots;
-        if (occ == 2 && swiglu && tiles <= 256) return;   // one wave per SIMD: 0.83 on two cold weights
-        const double usf = occ == 2 ? us2 : us1;
-        auto round = [&](long n) { return n <= 256 ? us1 : us2 * (0.8 + 0.2 * (n - 256) / 256); };
+        if (occ == 2 && swiglu && tiles <= cus) return;   // one wave per SIMD: 0.83 on two weights
         if (rem && P > 1)
-            offer(fam, P, 4.0 + full * nk * usf + (nk + P - 1) / P * (full || occ == 1 ? usf : 1.3 * usf) +
+            offer(fam, P, 4.0 + full * nk * two + (nk + P - 1) / P * (full || occ == 1 ? two : 1.43 * two) +
                               merge_us(rem, P, bm, bna));
-        double t = 4.0 + nk * (full * usf + (rem ? (occ == 2 ? round(rem) : us1) : 0.0));
+        double t = 4.0 + nk * (full * two + (rem ? (rem <= cus ? one : two) : 0.0));
         if (occ == 2) {
-            if (K > 8192) t *= 1.15;
+            if (K > 8192) t *= 1.34;
             const double reread = tiles * (double)(bm + bna) * K * 2;
-            if (foot > 32e6 && reread / 18e6 > t) t = reread / 18e6;
+            if (foot > 32e6 && reread / 18.8e6 > t) t = reread / 18.8e6;
         }
         offer(fam, 1, t);
     };
     if (K % 64 == 0) {
         const size_t s = qkv ? 2 : 0;
-        big(5, 128, 128, 2, foot < 9e6 ? 0.45 : 0.58, swiglu ? 1.10 : 0.90, s * 128 * 128);
-        big(6, 192, 256, 1, 1.32, 1.32, s * 192 * 256);
-        big(7, 256, 256, 1, 1.50, 1.50, s * 256 * 256);
+        if (!ring_only) ring(5, 128, 128, 2, 0.56, swiglu ? 0.95 : 0.89, s * 128 * 128);
+        ring(6, 192, 256, 1, 1.26, 1.26, s * 192 * 256);
+        ring(7, 256, 256, 1, 1.48, 1.48, s * 256 * 256);
     }
     return best;
 }
-template <int EPI> static const char *launch_small(GemmArgs &g, const SmallPick &b, bool launch, void *ws, int64_t ws_bytes) {
+// The ring families are 8 waves (2 x 4) of 128x64 (96x64; 128x128: 2 x 2 of 64x64)
+// on v_mfma_f32_16x16x32_bf16 with one fragment ring across the K loop and buffer
+// loads straight to LDS, the A operand's LDS ring one stage deeper than B's, and
+// the next k-step's fragment reads and the refill loads placed between every
+// other MFMA; two waves per SIMD cover each other's barrier and load-issue
+// stalls. On N(0,1) data the matrix cores sustain ~14 % more FLOP/s with
+// 16x16x32 than with 32x32x16 instructions under the power limit.
+template <int EPI> static const char *launch_tiles(GemmArgs &g, const TilePick &b, bool launch, void *ws, int64_t ws_bytes) {
     static const char *name[8] = {"bf16_64x64x64_kg2", "bf16_64x128x64_kg2", "bf16_128x128x64_kg2", "bf16_192x128x64_kg2",
                                   "bf16_256x128x64_kg2", "bf16_128x128x64_w2x2_occ2_m16", "bf16_192x256x64_w2x4_m16_ring_buf",
                                   "bf16_256x256x64_w2x4_m16_ring_buf"};
-    if (b.P == 1) ws = nullptr;   // the tiled families split by themselves when they are given a workspace
+    if (b.P == 1) ws = nullptr;   // the ring families split by themselves when they are given a workspace
     if (launch) switch (b.fam) {
     case 0: if constexpr (EPI != EPI_QKV) launch_kg<64, 64, 5, EPI, 4>(g, b.P, ws); break;
     case 1: launch_kg<64, 128, 3, EPI, 4>(g, b.P, ws); break;
@@ -1422,55 +1415,23 @@ static const char *pick_and_launch(GemmArgs &g, bool launch, void *ws = nullptr,
         if (launch) launch_skinny<EPI>(g);
         return "bf16_skinny";
     }
-    const int bn_out = EPI == EPI_SWIGLU ? 128 : 256;
-    const long tn = (g.N + bn_out - 1) / bn_out;
-    const long t256 = (long)((g.M + 255) / 256) * tn;
-    const long t192 = (long)((g.M + 191) / 192) * tn;
-    const long t128 = (long)((g.M + 127) / 128) * ((g.N + bn_out / 2 - 1) / (bn_out / 2));
-    const int nk = g.K / 64;
-    // tail split plans (P = 1: none) of the three tile families
-    const int p256 = ws ? tail_split_of(t256, nk, (size_t)256 * 256 * 4, ws_bytes) : 1;
-    const int p192 = ws ? tail_split_of(t192, nk, (size_t)192 * 256 * 4, ws_bytes) : 1;
-    const int p128 = ws ? tail_split_of(t128, nk, (size_t)128 * 128 * 4, ws_bytes, 0, 2) : 1;
-    const double c256 = tile_cost(t256, 1, 256, 256, g.K, 1.0, p256);
-    const double c192 = tile_cost(t192, 1, 192, 256, g.K, 0.85, p192);
-    const double c128 = tile_cost(t128, 2, 128, 128, g.K, 0.8, p128);
+    if (!ws) ws_bytes = 0;
     // buffer loads address with 32-bit byte offsets: both operands under 2 GiB
     const bool fits = (size_t)(g.M + 256) * g.K * 2 < ((size_t)1 << 31) &&
                       (size_t)g.N * g.K * 2 < ((size_t)1 << 31);
-    const bool use192 = c192 < c256;
-    const bool split256 = p256 > 1;
+    const TilePick b = pick_tiles(g.M, g.N, g.K, EPI == EPI_SWIGLU, false, ws_bytes, !fits);
     if (!fits) {
         // operands of 2 GiB or more: equal-depth rings filled by
         // global_load_lds (64-bit addresses), the same MFMA tiles and K order
-        if (use192) {
+        if (b.P == 1) ws = nullptr;
+        if (b.fam == 6) {
             if (launch) launch_ms<192, 256, 64, 2, 2, 4, EPI, 3, 1, 0, 16>(g, ws, ws_bytes);
             return "bf16_192x256x64_w2x4_m16_ring";
         }
         if (launch) launch_ms<256, 256, 64, 2, 2, 4, EPI, 3, 1, 0, 16>(g, ws, ws_bytes);
-        return split256 ? "bf16_256x256x64_w2x4_m16_ring_tailsplit" : "bf16_256x256x64_w2x4_m16_ring";
+        return "bf16_256x256x64_w2x4_m16_ring";
     }
-    if (t256 <= 512 || g.K % 64)   // only the K-group kernels take K % 64 != 0
-        return launch_small<EPI>(g, pick_small(g.M, g.N, g.K, EPI == EPI_SWIGLU, false, ws ? ws_bytes : 0), launch, ws,
-                                 ws ? ws_bytes : 0);
-    if (c128 < c256 && c128 < c192) {
-        if (launch) launch_ms<128, 128, 64, 2, 2, 2, EPI, 8, 2, 5, 16>(g, ws, ws_bytes);
-        return p128 > 1 ? "bf16_128x128x64_w2x2_occ2_m16_split" : "bf16_128x128x64_w2x2_occ2_m16";
-    }
-    // 8 waves (2 x 4) of 128x64 (96x64) on v_mfma_f32_16x16x32_bf16 (8 x 4
-    // accumulator tiles per wave) with one fragment ring across the K loop
-    // and buffer loads straight to LDS, the A operand's LDS ring one stage
-    // deeper than B's, and the next k-step's fragment reads and the refill
-    // loads placed between every other MFMA; two waves per SIMD cover each
-    // other's barrier and load-issue stalls. On N(0,1) data the matrix cores
-    // sustain ~14 % more FLOP/s with 16x16x32 than with 32x32x16
-    // instructions under the power limit.
-    if (use192) {
-        if (launch) launch_ms<192, 256, 64, 2, 2, 4, EPI, 8, 1, 5, 16>(g, ws, ws_bytes);
-        return "bf16_192x256x64_w2x4_m16_ring_buf";
-    }
-    if (launch) launch_ms<256, 256, 64, 2, 2, 4, EPI, 8, 1, 5, 16>(g, ws, ws_bytes);
-    return split256 ? "bf16_256x256x64_w2x4_m16_ring_buf_tailsplit" : "bf16_256x256x64_w2x4_m16_ring_buf";
+    return launch_tiles<EPI>(g, b, launch, ws, ws_bytes);
 }
 
 static bool mfma_ok(const void *x, const void *y, int N, int K, int kmod = 64) {
@@ -1531,28 +1492,9 @@ int hd_qkv_rope_gemm(const void *x, const void *wq, const void *wk, const void *
     g.k_out = (uint16_t *)k;
     g.vt_out = (uint16_t *)vt;
     g.seq = seq; g.heads = heads; g.kv_heads = kv_heads; g.eps = eps;
-    // the cheapest tile family, as in pick_and_launch (8 waves: two 64-wide
-    // wave tiles per head, 16x16x32 MFMA tiles)
-    const long tn = N / 256;
-    const long t256 = (long)((M + 255) / 256) * tn, t192 = (long)((M + 191) / 192) * tn;
-    const long t128 = (long)((M + 127) / 128) * tn * 2;
     if (ws && (uintptr_t)ws % 16) ws = nullptr;
     if (!ws) ws_bytes = 0;
-    if (t256 <= 512) {
-        launch_small<EPI_QKV>(g, pick_small(M, N, hidden, false, true, ws_bytes), true, ws, ws_bytes);
-        hd_check_launch("linear_qkv_rope");
-        return 0;
-    }
-    const int nk = hidden / 64;
-    auto split = [&](long t, int bm, int bn, int occ) {
-        return tail_split_of(t, nk, (size_t)bm * bn * 4, ws_bytes, (size_t)bm * bn * 2, occ);
-    };
-    const double c256 = tile_cost(t256, 1, 256, 256, hidden, 1.0, split(t256, 256, 256, 1));
-    const double c192 = tile_cost(t192, 1, 192, 256, hidden, 0.85, split(t192, 192, 256, 1));
-    const double c128 = tile_cost(t128, 2, 128, 128, hidden, 0.8, split(t128, 128, 128, 2));
-    if (c128 < c256 && c128 < c192) launch_ms<128, 128, 64, 2, 2, 2, EPI_QKV, 8, 2, 5, 16>(g, ws, ws_bytes);
-    else if (c192 < c256) launch_ms<192, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws_bytes);
-    else launch_ms<256, 256, 64, 2, 2, 4, EPI_QKV, 8, 1, 5, 16>(g, ws, ws_bytes);
+    launch_tiles<EPI_QKV>(g, pick_tiles(M, N, hidden, false, true, ws_bytes), true, ws, ws_bytes);
     hd_check_launch("linear_qkv_rope");
     return 0;
 }

@@ -174,9 +174,9 @@ def test_gemm_epilogues_with_and_without_tail_split(pkg, lib, dev, M):
 
 def test_swiglu_epilogue_vs_exact_division(pkg, lib, dev):
     """The fused SwiGLU epilogue uses the hardware reciprocal for
-    1/(1 + e^-g); hd_linear twice + hd_swiglu compute the same bf16 gate and
-    up projections (same K order) and the sigmoid with an IEEE division
-    (act.cu:29-33). After the bf16 rounding of silu(g) the two agree except
+    1/(1 + e^-g); hd_linear over the gate and up rows together + hd_swiglu
+    compute the same bf16 projections (as many tiles as the fused call, so the
+    same kernel and K order) and the sigmoid with an IEEE division (act.cu:29-33). After the bf16 rounding of silu(g) the two agree except
     near rounding boundaries: >= 99.9 % identical, the rest one bf16 step."""
     M, F, K = 1024, 3072, 1024
     g = torch.Generator(device=dev).manual_seed(21)
@@ -184,12 +184,12 @@ def test_swiglu_epilogue_vs_exact_division(pkg, lib, dev):
     wg = (torch.randn(F, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
     wu = (torch.randn(F, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
     fused = torch.empty(M, F, dtype=torch.bfloat16, device=dev)
-    gt = torch.empty(M, F, dtype=torch.bfloat16, device=dev)
-    up = torch.empty(M, F, dtype=torch.bfloat16, device=dev)
     sep = torch.empty(M, F, dtype=torch.bfloat16, device=dev)
+    w2 = torch.cat([wg, wu])
+    both = torch.empty(M, 2 * F, dtype=torch.bfloat16, device=dev)
     lib.hd_linear_swiglu(pkg.ptr(x), pkg.ptr(wg), pkg.ptr(wu), pkg.ptr(fused), M, F, K)
-    lib.hd_linear(pkg.ptr(x), pkg.ptr(wg), None, pkg.ptr(gt), M, F, K, 1)
-    lib.hd_linear(pkg.ptr(x), pkg.ptr(wu), None, pkg.ptr(up), M, F, K, 1)
+    lib.hd_linear(pkg.ptr(x), pkg.ptr(w2), None, pkg.ptr(both), M, 2 * F, K, 1)
+    gt, up = both[:, :F].contiguous(), both[:, F:].contiguous()
     lib.hd_swiglu(pkg.ptr(gt), pkg.ptr(up), pkg.ptr(sep), M * F)
     pkg.check_prim("swiglu epilogue vs exact")
     torch.cuda.synchronize()
