@@ -114,8 +114,9 @@ void hd_linear_concat3(const void *x_dev, const void *w0, int N0,
  * of the launch (0 on bad arguments). */
 double hd_mfma_probe(const void *ops, int n_ops, int blocks, int iters, int shape, float *out);
 
-/* Name of the kernel configuration hd_linear* would launch for a shape
- * (diagnostics; static string). */
+/* Name of the kernel configuration hd_linear* would launch without a workspace
+ * for a shape with aligned operands (diagnostics; static string); "reference"
+ * also for a residual or SwiGLU epilogue with K off 64, which those refuse. */
 const char *hd_gemm_config_name(int M, int N, int K, int epilogue);
 
 /* Extension: the block's QKV projection with the per-head q/k RMSNorm and

@@ -1598,7 +1598,10 @@ extern "C" double hd_mfma_probe(const void *ops, int n_ops, int blocks, int iter
 extern "C" const char *hd_gemm_config_name(int M, int N, int K, int epi) {
     GemmArgs g = {};
     g.M = M; g.N = N; g.K = K;
-    if (K % 8 || N % 8) return "reference";
+    g.seg_end[0] = g.seg_end[1] = g.seg_end[2] = N;
+    // K off 64: hd_linear and hd_linear_ws only, as linear_ok has it for aligned operands
+    const bool fused = epi == EPI_RES || epi == EPI_SWIGLU;
+    if ((fused && K % 64) || !linear_ok(nullptr, nullptr, nullptr, M, N, K)) return "reference";
     switch (epi) {
     case EPI_BIAS: return pick_and_launch<EPI_BIAS>(g, false);
     case EPI_RES: return pick_and_launch<EPI_RES>(g, false);

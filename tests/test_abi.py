@@ -100,3 +100,17 @@ def test_forward_fails_closed(lib, pkg):
 def test_gemm_config_names(lib):
     assert lib.hd_gemm_config_name(16640, 6144, 4096, 0).startswith(b"bf16_")
     assert lib.hd_gemm_config_name(7, 5, 6, 0) == b"reference"
+
+
+# epilogues: 0 none, 1 bias, 2 residual, 3 SwiGLU
+@pytest.mark.parametrize("M,N,K,epi,name", [
+    (2, 4096, 4096, 1, b"bf16_skinny"), (16, 4096, 12288, 2, b"bf16_skinny"), (16, 12288, 4096, 3, b"bf16_skinny"),
+    (32, 4096, 4096, 0, b"bf16_skinny"), (33, 4096, 4096, 0, b"bf16_64x64x64_kg2"), (17, 12288, 4096, 3, None),
+    (64, 256, 200, 1, b"bf16_64x64x64_kg2"), (64, 256, 200, 2, b"reference"), (64, 256, 200, 3, b"reference"),
+    (1 << 20, 256, 1096, 1, b"reference")])
+def test_gemm_config_name_is_the_launched_kernel(lib, M, N, K, epi, name):
+    """Few rows run the skinny kernel for every epilogue up to 16 rows; K off 64
+    runs on the K-group kernels for the plain and bias forms under 2 GiB, and is
+    refused by the fused ones."""
+    got = lib.hd_gemm_config_name(M, N, K, epi)
+    assert got == name if name else got.startswith(b"bf16_") and got != b"bf16_skinny"
