@@ -469,7 +469,9 @@ extern "C" hd_status hd_lora_merge_gpu(hd_lora_entry *entries, size_t count, voi
     for (int level = 0; level < nlevels && status == HD_OK; level++) {
         const std::vector<LmTarget> tg = stream_batches.count(level) ? stream_batches[level] : std::vector<LmTarget>();
         for (size_t i0 = 0; i0 < tg.size(); i0 += LM_TG) {
-            // under 2 GiB of W a target has less than 2^20 tiles
+            // tiles of a target: N K < 2^30, and N, K < 2^27 (up and down under 2 GiB
+            // at R >= 4), so ceil(N / 256) ceil(K / 64) < 2^16 + 2^19 + 2^21 + 1;
+            // LM_TG of them stay under 2^27
             LmBatch bt;
             bt.n = (int)(tg.size() - i0 < LM_TG ? tg.size() - i0 : LM_TG);
             bt.total = 0;
