@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 
 
 # few rows (1, 2, 16 | 17, 32: two row tiles; K below and off the 8 waves' 512),
-# 64x64 (ragged M and N, N % 64 = 8, odd tile counts, 8 chunks), 64x128 alone and
-# in 4 chunks, 128x128 in 8, 192x128, SwiGLU on 64x64, 128x128 and 192x128, K
+# 64x64 alone, in 2 and in 8 chunks (ragged M and N, N % 64 = 8, odd tile counts),
+# 128x128 in 8, 192x128 alone and in 5, SwiGLU on 64x64, 128x128 and 192x128, K
 # with a short last 64
 @pytest.mark.parametrize("M,N,K,epi", [
     (1, 4096, 256, "bias"), (2, 4096, 4096, "bias"), (16, 72, 64, "none"), (5, 1024, 3072, "res"), (16, 320, 576, "swiglu"),
@@ -44,3 +44,20 @@ def test_small_gemms_vs_fp32(pkg, lib, dev, M, N, K, epi):
     assert float((got - want).norm() / want.norm()) < (3e-3 if epi == "swiglu" else 1e-3)   # 2 products, rcp / exp of SiLU
     assert bool(((got - want).abs() <= (want.abs() + prod.abs()) * 2.0 ** -6 + 1e-3 * float(want.square().mean().sqrt())).all())
     assert bool((y[M] == 7.0).all())
+
+
+# the other families and splits of the choice (name: the kernel, where the call
+# has no workspace and so no split)
+@pytest.mark.parametrize("M,N,K,epi,name", [
+    (273, 3456, 1152, "bias", "bf16_64x128x64_kg2"), (567, 4096, 1088, "none", "bf16_128x128x64_kg2"),
+    (1065, 4096, 1088, "bias", "bf16_192x128x64_kg2"), (1563, 4096, 1088, "none", "bf16_128x128x64_w2x2_occ2_m16"),
+    (2061, 4096, 1088, "bias", "bf16_192x256x64_w2x4_m16_ring_buf"),
+    (129, 2048, 4096, "res", "64x128 in 5"), (273, 4096, 4096, "res", "128x128 in 2"),
+    (1314, 1024, 4096, "res", "192x128 in 4"), (2061, 4096, 4096, "res", "ring 128x128, last round in 8"),
+    (129, 4096, 1024, "swiglu", "64x128"), (816, 4096, 2048, "swiglu", "256x128"),
+    (816, 4096, 1024, "swiglu", "ring 128x128"), (1065, 4096, 1024, "swiglu", "ring 192x256"),
+    (567, 12288, 4096, "swiglu", "ring 192x256 in 8"), (982, 12288, 4096, "swiglu", "ring 256x256, last round in 2")])
+def test_tile_families_vs_fp32(pkg, lib, dev, M, N, K, epi, name):
+    if name.startswith("bf16"):
+        assert lib.hd_gemm_config_name(M, N, K, 1 if epi == "bias" else 0).decode() == name
+    test_small_gemms_vs_fp32(pkg, lib, dev, M, N, K, epi)

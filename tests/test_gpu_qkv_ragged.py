@@ -10,13 +10,25 @@ pytestmark = pytest.mark.gpu
 
 
 # one sequence ending inside a 16-key group / a 64-key tile; batches whose
-# later sequences start on and off the 16-key groups; 128- and 256-row tiles,
-# with and without K chunks
+# later sequences start on and off the 16-key groups; 64- and 128-row tiles
 @pytest.mark.parametrize("B,S", [(1, 1), (1, 94), (1, 129), (1, 1209), (2, 80), (2, 77), (3, 205), (2, 1101)])
 def test_block_ragged_lengths(pkg, lib, dev, B, S):
     """hd_decoder_block_batched against a torch fp32 statement of the block
     (block.c:245-349); rel-L2 1e-2 is the bound of a block in bf16."""
-    H, KV, HID, FF, D = 8, 2, 1024, 1024, 128
+    check_block(pkg, lib, dev, B, S, 8, 2, 1024)
+
+
+# 64x128 in 4 K chunks, 128x128 in 5, 192x128 in 5 and alone, the ring's 128x128
+# alone and with its last round in 8, 192x256, 256x256
+@pytest.mark.parametrize("B,S,HID", [(1, 33, 2048), (1, 81, 4096), (2, 77, 4096), (1, 650, 2048), (1, 982, 2048),
+                                     (2, 657, 4096), (1, 1314, 2048), (3, 687, 2048)])
+def test_block_ragged_tile_families(pkg, lib, dev, B, S, HID):
+    """The same at 32 / 8 heads, where the QKV projection takes its other tiles."""
+    check_block(pkg, lib, dev, B, S, 32, 8, HID)
+
+
+def check_block(pkg, lib, dev, B, S, H, KV, HID):
+    FF, D = 1024, 128
     print(f"ragged block B={B} S={S}", flush=True)
     w = {k: to_dev(v, dev) for k, v in make_block_weights(HID, H, KV, FF, D, seed=S).items()}
     g = torch.Generator(device=dev).manual_seed(S)
