@@ -1315,7 +1315,7 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     const bool bits = bits_bytes > 0 && ws && bits_bytes <= ws_bytes;
     if (bits) ws_bytes -= bits_bytes;
     const int slots = ws ? fa_slots(nwv) : 0;
-    if (slots > 0 && (ar_len == 0 || prefix) && units >= slots) {
+    if (slots > 0 && (ar_len == 0 || (prefix && pp)) && units >= slots) {
         const int rem = units % slots, ntile = (seq + FA_BK - 1) / FA_BK;
         int P = rem ? (slots - n_causal) / rem : 1;
         if (P < 2 && rem) P = slots / rem;

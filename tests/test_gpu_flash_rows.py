@@ -57,6 +57,12 @@ def test_flash_rows_and_masks(pkg, lib, dev, B, Hq, Hkv, S, ar, dense, ws):
         assert float(per_row.max()) < 3e-2, int(per_row.max(0)[0].argmax())   # every row of every head is written
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,ar,ws", [(3, 32, 8, 1000, 300, True)])
+def test_causal_prefix_routes(pkg, lib, dev, B, Hq, Hkv, S, ar, ws):
+    """Bounds as above."""
+    test_flash_rows_and_masks(pkg, lib, dev, B, Hq, Hkv, S, ar, False, ws)
+
+
 @pytest.mark.parametrize("S,off", [(1, 0), (64, 0), (65, 1), (200, 0), (131, 1)])
 def test_make_vt_bytes(pkg, lib, dev, S, off):
     """V^T layout, 16-byte path and the element path of a misaligned V (off = 1):
