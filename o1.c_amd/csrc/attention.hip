@@ -510,8 +510,11 @@ __global__ __launch_bounds__(512, 1) void flash_pp16_kernel(FaArgs a) {
         // (by value: a selected pointer into the arguments would be read with
         // vector loads and make everything below per-lane)
         FaRows rows = a.full;
-        if (MODE == FA_CAUSAL && causal_unit) rows = a.causal;
         const int group = a.Hq / a.Hkv;
+        if (MODE == FA_CAUSAL && causal_unit) {
+            rows = a.causal;
+            lin = fa_longest_first(rows, a.batch, a.Hkv, group, lin);
+        }
         FaUnit un = fa_unit(rows, a.batch, a.Hkv, group, lin);
         un.b = __builtin_amdgcn_readfirstlane(un.b);
         un.hk = __builtin_amdgcn_readfirstlane(un.hk);
@@ -1236,23 +1239,112 @@ static int64_t fa_mask_bits_bytes(int seq) {
     return words <= 64 ? (seq + 31) / 32 * words * 8 : 0;
 }
 
+// Key tiles that the causal rows [0, ar_len) of one head read, in blocks of n rows.
+static int64_t fa_causal_tiles(int ar_len, int n) {
+    const int64_t full = ar_len / n;
+    return full * (full + 1) / 2 * (n / FA_BK) + (ar_len % n ? (ar_len + FA_BK - 1) / FA_BK : 0);
+}
+
+// Key chunks of the units in the last, partly filled round (rem of them, nt key
+// tiles each; 1: no split) beside n_causal causal units of w key tiles in all.
+static int fa_split(int rem, int nt, int n_causal, int64_t w, int slots) {
+    if (rem == 0) return 1;
+    int P = (slots - n_causal) / rem;
+    // causal units that need the free slots themselves: chunks short enough to
+    // end with them
+    if (P < 2) P = n_causal ? (int)hd_cdiv((int64_t)nt * slots, (int64_t)rem * nt + w) : slots / rem;
+    if (P > FA_MAX_SPLIT) P = FA_MAX_SPLIT;
+    return P < nt ? P : nt;
+}
+
+// Ways to run a causal text prefix (rows < ar_len see keys <= row, the others all):
+//  FA_ONE    one masked launch of 4-wave blocks. The block that holds row ar_len
+//            runs every key, masked ones too unless ar_len % 128 == 0
+//  FA_TWO    the prefix rows as FA_ONE, whose blocks all end at their diagonal,
+//            then the other rows as full attention (8-wave with a workspace)
+//  FA_UNITS  one launch of 8-wave blocks, causal rows as units of their own behind
+//            the full ones, longest first; FA_UNITS_WHOLE the same without key
+//            chunks
+// A call without a workspace takes the kernel for the causal rows that it would
+// take with one, so that these rows do not depend on it.
+// From FA_PP_MIN keys on the lowest predicted time is taken: us per 64-key tile of a
+// full round's and of a lone block, the launches' fixed costs, and the work of all
+// blocks over the CUs, fitted to all four at 1650 calls with a workspace (1-3 x 8-32
+// heads, S = 1024-8704, ar_len = 1 .. S - 1): the choice is 0.9 % off the fastest on
+// average. FA_UNITS in all cases would be 6 % off and up to 1.46 times as long where
+// causal rows are many or the grid is less than a round; us, fastest second:
+//   32 heads, S = 2371, ar_len 114: ONE 115, UNITS 103; 2370: UNITS 77, ONE 73
+//   32 heads, S = 4239, ar_len 142: ONE 318, UNITS 273
+//   32 heads, S = 4352, ar_len 256: UNITS 261, TWO 250; 2 x 1152, 142: 50.9, 46.5
+//   8 heads, S = 1101, ar_len 76: ONE 45, UNITS 34; 256: UNITS 34.4, ONE 25.5
+enum { FA_ONE, FA_TWO, FA_UNITS, FA_UNITS_WHOLE };
+static int fa_prefix_route(int batch, int hq, int hkv, int seq, int ar_len, int q_row_end, bool ws) {
+    const int slots = fa_slots(8), nt = (seq + FA_BK - 1) / FA_BK, group = hq / hkv, bh = batch * hq;
+    if (slots <= 0) return FA_ONE;
+    const double per_cu = 1.0 / slots;
+    double best = 1e30;
+    int route = FA_ONE;
+    auto offer = [&](int r, double us) {
+        if (us < best) {
+            best = us;
+            route = r;
+        }
+    };
+    // 4-wave blocks, two per CU: the longest one, or the work of all and the free
+    // slots of the last round (each hides most of the other)
+    auto blocks4_us = [&](int64_t blocks, double tiles, double longest) {
+        const int64_t last = blocks % (2 * slots);
+        double work = 0.96 * tiles * per_cu;
+        if (blocks > 2 * slots && last) work += 0.36 * nt * (1.0 - 0.5 * last * per_cu);
+        const double lo = fmin(longest, work), hi = fmax(longest, work);
+        return 7.4 + hi + 0.3 * lo * lo / hi;
+    };
+    const int mixed = ar_len % 128 ? nt - ar_len / FA_BK : 0;   // masked tiles of the block with row ar_len
+    const int64_t pre = ar_len / 128, per_head = (q_row_end + 127) / 128;
+    const double one = blocks4_us(bh * per_head, (double)bh * (pre * (pre + 1) + (per_head - pre) * nt + mixed),
+                                  1.02 * nt + 1.06 * mixed);
+    offer(FA_ONE, one);
+    // 8-wave blocks: whole rounds, then what is left over beside w causal tiles
+    auto units_us = [&](int units, int n_causal, int64_t w, double tile, bool split) {
+        const int rem = units % slots, P = split && units >= slots ? fa_split(rem, nt, n_causal, w, slots) : 1;
+        const double left = tile * ((double)rem * nt + w) * per_cu, us = 9.7 + tile * nt * (units / slots);
+        if (P > 1)
+            return us + 15.3 + 10.5 * fmax(0.0, (rem * P + n_causal) * per_cu - 1.0) +
+                   fmax(1.37 * ((nt + P - 1) / P) + 7.3, left);
+        return us + fmax(rem ? 1.37 * nt : 0.0, left) + (units + n_causal > slots ? 7.3 : 0.0);
+    };
+    const FaRows full = fa_rows_of(ar_len, q_row_end - ar_len, group, true), causal = fa_rows_of(0, ar_len, group, false);
+    const int units = fa_rows_units(full, batch, hkv, group), n_causal = fa_rows_units(causal, batch, hkv, group);
+    const int64_t w = bh * fa_causal_tiles(ar_len, FA_ROWS);
+    offer(FA_UNITS, units_us(units, n_causal, w, 1.80, true));
+    offer(FA_UNITS_WHOLE, 1.01 * units_us(units, n_causal, w, 1.80, false));
+    const double first = 3.4 + fmax(2.04 * ((ar_len + 127) / 128), 0.85 * bh * fa_causal_tiles(ar_len, 128) * per_cu);
+    if (seq % FA_BK == 0)
+        offer(FA_TWO, 1.02 * (first + units_us(bh * ((q_row_end - ar_len + FA_ROWS - 1) / FA_ROWS), 0, 0, 1.74, true)));
+    if (ws) return route;
+    if (route >= FA_UNITS) return FA_UNITS_WHOLE;
+    const int64_t rest = bh * ((q_row_end - ar_len + 127) / 128);   // 4-wave blocks here
+    return first + blocks4_us(rest, (double)rest * nt, 1.02 * nt) < one ? FA_TWO : FA_ONE;
+}
+
 static int fa_launch(const void *q, const void *k, const void *vt, const void *mask, void *out,
                      int batch, int hq, int hkv, int seq, int ar_len, int q_row_end, float scale,
                      int out_seq_major, hipStream_t st, void *ws = nullptr, int64_t ws_bytes = 0,
                      int out_rows = 0, int q_row_begin = 0) {
-    const bool prefix = ar_len > 0 && !mask && q_row_begin == 0 && ar_len < q_row_end;
-    // Short sequences (4-wave blocks) with a causal text prefix (rows < ar_len
-    // see keys <= row): the prefix rows run as a masked launch of their own,
-    // whose blocks all end at their diagonal, and rows ar_len.. are plain full
-    // attention. One masked launch over all rows costs 7-12 % more: its block
-    // holding row ar_len runs every key with most of its waves masked.
-    if (prefix && ws && seq < FA_PP_MIN && (seq % FA_BK) == 0) {
+    const bool with_prefix = ar_len > 0 && !mask && q_row_begin == 0 && ar_len < q_row_end;
+    int route = FA_ONE;
+    if (with_prefix) {
+        if (seq >= FA_PP_MIN) route = fa_prefix_route(batch, hq, hkv, seq, ar_len, q_row_end, ws != nullptr);
+        else if (ws && seq % FA_BK == 0) route = FA_TWO;
+    }
+    if (route == FA_TWO) {
         const int rc = fa_launch(q, k, vt, nullptr, out, batch, hq, hkv, seq, ar_len, ar_len, scale,
                                  out_seq_major, st, nullptr, 0, out_rows, 0);
         if (rc) return rc;
         return fa_launch(q, k, vt, nullptr, out, batch, hq, hkv, seq, 0, q_row_end, scale, out_seq_major, st,
                          ws, ws_bytes, out_rows, ar_len);
     }
+    const bool prefix = route >= FA_UNITS;   // causal rows on units of their own
     FaArgs a;
     a.q = (const uint16_t *)q;
     a.k = (const uint16_t *)k;
@@ -1275,10 +1367,8 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     // sequence is long enough to amortise the larger block and
     //  * the tail split can fill the last round (+3 % at S = 16640 / 16896,
     //    equal at 4352; without the split the finer grain of 4 waves wins), or
-    //  * there is a causal prefix: its rows are units of their own behind the
-    //    full ones in the same grid, so that no block mixes both kinds
-    //    (S = 4239, 142 causal rows, one masked 4-wave launch: 314 -> 270 us;
-    //    S = 16499: 4080 -> 3630; 2 x 1101 rows: equal), or
+    //  * there is a causal prefix that the route above gives to units of
+    //    their own, or
     //  * there is a dense mask: its values are prefetched as 16-byte pieces
     //    under the MFMA phase, where a tile needs them (4-wave blocks
     //    with 2-byte loads, causal text rows above zeros: S = 300 26.6 ->
@@ -1315,12 +1405,9 @@ static int fa_launch(const void *q, const void *k, const void *vt, const void *m
     const bool bits = bits_bytes > 0 && ws && bits_bytes <= ws_bytes;
     if (bits) ws_bytes -= bits_bytes;
     const int slots = ws ? fa_slots(nwv) : 0;
-    if (slots > 0 && (ar_len == 0 || (prefix && pp)) && units >= slots) {
+    if (slots > 0 && (ar_len == 0 || route == FA_UNITS) && units >= slots) {
         const int rem = units % slots, ntile = (seq + FA_BK - 1) / FA_BK;
-        int P = rem ? (slots - n_causal) / rem : 1;
-        if (P < 2 && rem) P = slots / rem;
-        if (P > FA_MAX_SPLIT) P = FA_MAX_SPLIT;
-        if (P > ntile) P = ntile;
+        int P = fa_split(rem, ntile, n_causal, n_causal ? batch * hq * fa_causal_tiles(ar_len, BQ) : 0, slots);
         const int64_t chunk_bytes = (int64_t)BQ * (FA_D + 2) * 4;
         if (bits && rem * P * chunk_bytes > ws_bytes) P = (int)(ws_bytes / (rem * chunk_bytes));
         if (rem && P >= 2 && rem * P * chunk_bytes <= ws_bytes) {

@@ -59,6 +59,17 @@ FA_HD FaUnit fa_unit(const FaRows &r, int batch, int kv_heads, int group, int li
     return u;
 }
 
+// The i-th causal unit to start, as a number of fa_unit: longest first (a unit of
+// causal rows reads the keys up to its last row), so the blocks that start last
+// end soonest. Left-over rows, then the whole tiles downwards, each of every head.
+FA_HD int fa_longest_first(const FaRows &r, int batch, int kv_heads, int group, int i) {
+    const int per_tile = batch * kv_heads * group, n_left = r.left ? batch * kv_heads * ((group + r.hp - 1) / r.hp) : 0;
+    if (i < n_left) return per_tile * r.ntile + i;
+    i -= n_left;
+    const int tile = r.ntile - 1 - i / per_tile, j = i % per_tile;
+    return (j / group * r.ntile + tile) * group + j % group;
+}
+
 // Query row and head of row i (0..255) of a unit; row = FA_NO_ROW where it has none.
 struct FaRowHead {
     int row, head;

@@ -25,6 +25,18 @@ extern "C" int fa_owners(int batch, int kv, int group, int row0, int rows, int s
     }
     return bad;
 }
+// keys that the causal unit in place i reads, or -1 if another place names it too
+extern "C" int fa_order(int batch, int kv, int group, int rows, int *keys) {
+    const FaRows r = fa_rows_of(0, rows, group, false);
+    const int n = fa_rows_units(r, batch, kv, group);
+    for (int i = 0; i < n; i++) {
+        const int lin = fa_longest_first(r, batch, kv, group, i);
+        const FaUnit u = fa_unit(r, batch, kv, group, lin);
+        keys[i] = lin < 0 || lin >= n ? -1 : u.qbase + (u.left ? u.left : FA_ROWS);
+        for (int j = 0; j < i; j++) if (fa_longest_first(r, batch, kv, group, j) == lin) keys[i] = -1;
+    }
+    return n;
+}
 """
 
 
@@ -35,12 +47,25 @@ def owners(tmp_path_factory):
     src.write_text(SHIM)
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "o1.c_amd", "csrc"),
                     "-o", str(so), str(src)], check=True)
-    fn = ctypes.CDLL(str(so)).fa_owners
+    shim = ctypes.CDLL(str(so))
+    fn = shim.fa_owners
 
     def run(batch, kv, group, row0, rows, share, S):
         n = np.zeros((batch, kv * group, S), np.int32)
         return n, fn(batch, kv, group, row0, rows, int(share), S, n.ctypes.data_as(ctypes.c_void_p))
+    run.order = shim.fa_order
     return run
+
+
+@pytest.mark.parametrize("batch,kv,group", [(1, 1, 1), (2, 2, 4), (1, 8, 3)])
+def test_causal_units_start_longest_first(owners, batch, kv, group):
+    """Every causal unit has one place in the order, and none reads more keys than
+    the one before it."""
+    for rows in (1, 114, 255, 256, 257, 512, 700, 1185):
+        keys = np.zeros(batch * kv * group * (rows // 256 + 1), np.int32)
+        n = owners.order(batch, kv, group, rows, keys.ctypes.data_as(ctypes.c_void_p))
+        assert n == batch * kv * group * -(-rows // 256)
+        assert (keys[:n] > 0).all() and (np.diff(keys[:n]) <= 0).all() and keys[0] == rows
 
 
 # every remainder of 256 rows, below and past whole tiles, with and without rows in front

@@ -57,7 +57,13 @@ def test_flash_rows_and_masks(pkg, lib, dev, B, Hq, Hkv, S, ar, dense, ws):
         assert float(per_row.max()) < 3e-2, int(per_row.max(0)[0].argmax())   # every row of every head is written
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,ar,ws", [(3, 32, 8, 1000, 300, True)])
+# causal prefixes on each route: one 4-wave launch (a grid below one round whose row
+# ar_len starts a block; nearly every row causal), two launches with and without a
+# workspace, units with whole tiles of causal rows beside key chunks, units unsplit
+@pytest.mark.parametrize("B,Hq,Hkv,S,ar,ws", [
+    (1, 8, 2, 1101, 256, True), (1, 8, 2, 1024, 1023, True), (1, 32, 8, 4352, 256, True), (1, 16, 4, 4160, 144, True),
+    (1, 16, 4, 4160, 144, False), (1, 32, 8, 4239, 2119, True), (1, 32, 8, 2371, 2370, True), (3, 32, 8, 1209, 255, True),
+    (1, 8, 2, 2371, 1185, True), (3, 32, 8, 1000, 300, True)])
 def test_causal_prefix_routes(pkg, lib, dev, B, Hq, Hkv, S, ar, ws):
     """Bounds as above."""
     test_flash_rows_and_masks(pkg, lib, dev, B, Hq, Hkv, S, ar, False, ws)
