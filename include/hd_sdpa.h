@@ -75,7 +75,8 @@ int hd_flash_attention(const void *q, const void *k, const void *vt,
  * (batch x heads x query tiles) units that see every key leave a last, partly
  * filled round of resident blocks, those units run as 2-16 key-range chunks
  * writing fp32 partials (running max, sum, unnormalised O) into ws, and a
- * merge kernel combines them (not for a mask together with ar_len > 0). With
+ * merge kernel combines them (not for a mask together with ar_len > 0, nor
+ * where a causal prefix runs faster without). With
  * a dense mask, ws also holds one bit per mask tile: tiles of zeros are not
  * read again for every head. A smaller ws leaves these out.
  * Results agree with the unsplit kernel to fp32 rounding of the merge. */

@@ -1098,7 +1098,7 @@ int hd_flash_v72(const void *q, const void *k, const void *vt, void *out, int ba
 // One block per 64-key tile: rows in through LDS (16-byte loads when V is
 // 16-byte aligned), 16-byte stores of 8 storage columns per dimension. HBM
 // bound in principle (4 B per element); at S = 2371, 8 heads it is one short
-// launch: 8.4 us with 2-byte accesses, 4.0 us in this form (S = 16640: 26.9 ->
+// launch: 8.4 us with 2-byte accesses, 4.0 us in this form, 5.2 in a trace (S = 16640: 26.9 ->
 // 11.5 us).
 template <bool V16>
 __global__ __launch_bounds__(256) void fa_vt_kernel(const uint16_t *v, uint16_t *vt, int S,
@@ -1273,10 +1273,9 @@ static int fa_split(int rem, int nt, int n_causal, int64_t w, int slots) {
 // heads, S = 1024-8704, ar_len = 1 .. S - 1): the choice is 0.9 % off the fastest on
 // average. FA_UNITS in all cases would be 6 % off and up to 1.46 times as long where
 // causal rows are many or the grid is less than a round; us, fastest second:
-//   32 heads, S = 2371, ar_len 114: ONE 115, UNITS 103; 2370: UNITS 77, ONE 73
-//   32 heads, S = 4239, ar_len 142: ONE 318, UNITS 273
-//   32 heads, S = 4352, ar_len 256: UNITS 261, TWO 250; 2 x 1152, 142: 50.9, 46.5
-//   8 heads, S = 1101, ar_len 76: ONE 45, UNITS 34; 256: UNITS 34.4, ONE 25.5
+//   32 heads, S = 2371, ar_len 114: ONE 114, UNITS 102; S = 4239, 142: ONE 311, UNITS 269
+//   32 heads, S = 1024, ar_len 1023: UNITS 36.4, ONE 25.5; 8 heads, 1101, 256: 34.4, 25.4
+//   32 heads, S = 4352, ar_len 256: UNITS 256, TWO 247; 2 x 1152, 142: 50.9, 46.5
 enum { FA_ONE, FA_TWO, FA_UNITS, FA_UNITS_WHOLE };
 static int fa_prefix_route(int batch, int hq, int hkv, int seq, int ar_len, int q_row_end, bool ws) {
     const int slots = fa_slots(8), nt = (seq + FA_BK - 1) / FA_BK, group = hq / hkv, bh = batch * hq;

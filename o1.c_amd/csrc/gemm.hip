@@ -722,9 +722,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, OCC) void gemm_ms_kernel(GemmArgs g
 // 128 B per cycle and issue 2 TM TN MFMAs of 16 cycles per SIMD: 640 against
 // 768 cycles for 192 x 128, 512 / 512 for 128 x 128, 384 / 256 for 128 x 64 and
 // 256 / 128 for 64 x 64, so the largest tile that still fills the CUs wins.
-// Measured (us, against the tiled kernels): o_proj of 94 rows 32.3 -> 17, of
-// 1152 rows 51.8 -> 45; SwiGLU of 94 rows 56 -> 46; 576 x 1152 x 1152 12.3 ->
-// 7.4; 576 x 1152 x 4352 25.3 -> 17.0; 432 x 4608 x 4608 40.9 -> 28.0.
+// Measured (us, cold weights, against the ring tiles at their best split): o_proj
+// of 94 rows 18.6 -> 16.7, of 1152 rows 56.4 -> 50.0; SwiGLU of 94 rows 56 -> 46;
+// 576 x 4304 x 1152 17.7 -> 15.2; 432 x 4096 x 4608 35.5 -> 31.0.
 // ---------------------------------------------------------------------------
 template <int BM, int BN, int NS, int EPI, int OCC>
 __global__ __launch_bounds__(512, OCC) void gemm_kg_kernel(GemmArgs g) {

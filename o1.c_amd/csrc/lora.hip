@@ -173,7 +173,7 @@ __device__ __forceinline__ void split3(float x, uint16_t &h0, uint16_t &h1, uint
 //  * waves 4 .. 7 run half a tile behind waves 0 .. 3, so that on each SIMD one
 //    wave updates and stores while the other multiplies (in step: 217 us).
 // One layer's seven targets at R = 64, 386 MB of W read and written: 241 us ->
-// 197 us per call, 189 us in the kernel = 4.1 TB/s (a copy here reaches 4.8).
+// 197 us per call, 177 us in the kernel = 4.4 TB/s (a copy here reaches 4.8).
 // Before, 128 x 64 tiles with W, up and down all staged in LDS took one launch
 // per shape, and five LDS passes over W. Without the MFMAs it would take 178 us.
 // Every load and store is unconditional: offsets past the data read as zero

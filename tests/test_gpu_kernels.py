@@ -741,11 +741,12 @@ def test_lora_merge_kernels_vs_oracle(pkg, lib, dev, N, K, R):
 @pytest.mark.parametrize("B,S,T", [(1, 1152, 128), (2, 640, 300), (1, 2176, 65), (1, 4352, 256)])
 def test_flash_causal_prefix_split_launch(pkg, lib, dev, B, S, T):
     """A causal text prefix (rows < ar_len = T - 1 see keys <= row) with the
-    tail-split workspace runs as two launches: the prefix rows masked, the
-    rows from ar_len on as full attention with a query-row offset and the
-    tail split (hd_cudnn_sdpa.cu:376-441 runs the same split as two cuDNN
-    passes). Checked against an fp32 torch statement of the attention with
-    that mask, and against the single masked launch (no workspace)."""
+    tail-split workspace runs on the route that its sizes favour: two launches
+    (the prefix rows masked, the rows from ar_len on as full attention with a
+    query-row offset and the tail split; hd_cudnn_sdpa.cu:376-441 runs the
+    same split as two cuDNN passes), or one. Checked against an fp32 torch
+    statement of the attention with that mask, and the prefix rows against the
+    call without a workspace, which takes the same kernel for them."""
     g = torch.Generator(device=dev).manual_seed(S + T)
     q = torch.randn(B, 32, S, 128, generator=g, device=dev).to(torch.bfloat16)
     k = torch.randn(B, 8, S, 128, generator=g, device=dev).to(torch.bfloat16)
